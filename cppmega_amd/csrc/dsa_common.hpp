@@ -302,6 +302,29 @@ __device__ __forceinline__ float buffer_load_f32(__amdgpu_buffer_rsrc_t r, int v
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voffset, soffset, 0));
 }
 
+// Buffer descriptor as a plain register quadruple (the operand of lds_dma_16).
+__device__ __forceinline__ i32x4 make_buffer_words(const void *base, uint32_t num_bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  return i32x4{(int)__builtin_amdgcn_readfirstlane((uint32_t)a), (int)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)),
+               (int)__builtin_amdgcn_readfirstlane(num_bytes), 0x00020000};
+}
+// Byte address of an LDS object, as M0 takes it.
+__device__ __forceinline__ uint32_t lds_address(const void *p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char *)p;
+}
+// LDS-DMA: lane l's 16 bytes at byte voffset of the resource (zeros past its
+// end) go to LDS bytes lds + 16 l .. + 15, lds wave-uniform.  Written in asm
+// because the builtin makes every later LDS read wait for all such loads; the
+// caller waits (vmcnt) before the barrier that publishes the data.  No register
+// is written, and the compiler's own vmcnt waits, which do not count this load,
+// only become stricter by it.
+__device__ __forceinline__ void lds_dma_16(uint32_t lds, uint32_t voffset, i32x4 rs) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :
+               : "s"(lds), "v"(voffset), "s"(rs)
+               : "memory", "m0");
+}
+
 // Remap a linear block id so that consecutive logical blocks land on the
 // same XCD (blocks are dispatched round-robin over the 8 XCDs of MI355X).
 __device__ __forceinline__ int64_t xcd_remap(int64_t bid, int64_t nblocks) {

@@ -711,11 +711,24 @@ static int64_t partial_elem_bytes(int flags, int64_t D_qk) {
   return (flags & DSA_BWD_FP32_PARTIALS) ? 4 : 2;
 }
 
+// Partial rows per entry: one per 32-head tile, or for the wide rows one per
+// 128-head group of the kv group.
+static int64_t row_tiles(int64_t H, int64_t G, int64_t D_qk) {
+  const int64_t ht = (H / (G > 0 ? G : 1) + 31) / 32;
+  return wide_row(D_qk) ? (ht + kWideRowTiles - 1) / kWideRowTiles : ht;
+}
+
+// Wide rows: bytes of the P and dS tiles of one (token, kv group).
+static uint64_t pd_token_bytes(int64_t H, int64_t G, int64_t D_qk, int64_t topk) {
+  if (!wide_row(D_qk)) return 0;
+  return (uint64_t)((topk + 31) / 32) * (uint64_t)((H / (G > 0 ? G : 1) + 31) / 32) * (uint64_t)kWidePdBytes;
+}
+
 static BwdPlan bwd_plan(int64_t B, int64_t S, int64_t H, int64_t G, int64_t D_qk, int64_t topk, int flags,
                         uint64_t cap) {
-  const int64_t hpg = H / (G > 0 ? G : 1);
-  const int64_t ntiles = (hpg + 31) / 32;
-  const uint64_t per_token = (uint64_t)(G * topk * ntiles) * (uint64_t)(D_qk * partial_elem_bytes(flags, D_qk) + 1);
+  const uint64_t per_token = (uint64_t)(G * topk * row_tiles(H, G, D_qk)) *
+                                 (uint64_t)(D_qk * partial_elem_bytes(flags, D_qk) + 1) +
+                             (uint64_t)G * pd_token_bytes(H, G, D_qk, topk);
   BwdPlan pl;
   if ((uint64_t)S * per_token <= cap) {
     pl.ct = S;
@@ -725,6 +738,9 @@ static BwdPlan bwd_plan(int64_t B, int64_t S, int64_t H, int64_t G, int64_t D_qk
   } else {
     int64_t ct = (int64_t)(cap / per_token) / kChunkTokens * kChunkTokens;
     pl.ct = ct < kChunkTokens ? kChunkTokens : ct;
+    pl.npb = (S + pl.ct - 1) / pl.ct;
+    // passes of equal length: a short last one would leave the GPU part idle
+    pl.ct = ((S + pl.npb - 1) / pl.npb + kChunkTokens - 1) / kChunkTokens * kChunkTokens;
     pl.npb = (S + pl.ct - 1) / pl.ct;
     pl.nb = 1;
   }
@@ -739,7 +755,7 @@ static BwdPlan bwd_plan(int64_t B, int64_t S, int64_t H, int64_t G, int64_t D_qk
 // dsa_sparse_mla_bwd_indexed takes the index section as a separate buffer that
 // dsa_sparse_mla_bwd_build_index filled ahead of the call.
 struct BwdWorkspace {
-  size_t partials, pexp, carry, rows_total;          // offsets in the rows section
+  size_t partials, pexp, carry, pd, rows_total;          // offsets in the rows section
   size_t mask, base, dup, dupc, tot, rowstart, pos_of, next, index_total;  // offsets in the index section
   size_t total;                                      // rows section + index section
   BwdPlan plan;
@@ -747,8 +763,7 @@ struct BwdWorkspace {
 
 static BwdWorkspace bwd_layout(int64_t B, int64_t S, int64_t S_kv, int64_t H, int64_t G, int64_t D_qk,
                                int64_t topk, int flags, uint64_t pass_bytes) {
-  const int64_t hpg = H / (G > 0 ? G : 1);
-  const int ntiles = (int)((hpg + 31) / 32);
+  const int ntiles = (int)row_tiles(H, G, D_qk);
   BwdWorkspace L;
   L.plan = bwd_plan(B, S, H, G, D_qk, topk, flags, pass_cap(pass_bytes));
   const BwdPlan &pl = L.plan;
@@ -762,6 +777,8 @@ static BwdWorkspace bwd_layout(int64_t B, int64_t S, int64_t S_kv, int64_t H, in
   off += align256(entries * ntiles + kTrashRows);
   L.carry = off;  // fp32 sums of one batch's kv rows, carried across its passes
   off += pl.npb > 1 ? align256((size_t)R * D_qk * 4) : 0;
+  L.pd = off;  // wide rows: P and dS tiles between the pass's two kernels
+  off += align256((size_t)(pl.nb * pl.ct * G) * pd_token_bytes(H, G, D_qk, topk));
   L.rows_total = off;
   off = 0;
   L.mask = off;
@@ -897,7 +914,7 @@ static int bwd_run(const void *q, const void *kv, const void *o, const void *dO,
                    int flags, const BwdWorkspace &L, hipStream_t st) {
   const int64_t R = S_kv * G;
   const int64_t hpg = H / G;
-  const int ntiles = (int)((hpg + 31) / 32);
+  const int ntiles = (int)row_tiles(H, G, D_qk);
   const bool f8 = dtype == DSA_DTYPE_E4M3;
   const bool wide = wide_shape(D_qk, D_v);
   const bool f32p = (flags & DSA_BWD_FP32_PARTIALS) != 0;
@@ -955,6 +972,8 @@ static int bwd_run(const void *q, const void *kv, const void *o, const void *dO,
     p.topk = topk;
     p.hpg = (int)hpg;
     p.ntiles = ntiles;
+    p.htiles = (int)((hpg + 31) / 32);
+    p.pd = ws + L.pd;
     p.sl2 = sm_scale * kLog2e;
     p.scale = sm_scale;
     if (wide) rc = launch_bwd_main_wide(p, D_qk, D_v, f8, f32p, st);

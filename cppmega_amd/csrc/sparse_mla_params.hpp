@@ -12,6 +12,11 @@ namespace dsa {
 // of all landing on one.
 constexpr int kTrashRows = 64;
 
+// Wide heads: heads whose dKV contributions are summed into one partial row,
+// and the bytes of one (block, 32-head tile)'s P and dS tiles.
+constexpr int kWideRowTiles = 4;
+constexpr int kWidePdBytes = 2 * 32 * 32 * 2;
+
 struct FwdParams {
   const unsigned char *q;
   const unsigned char *kv;
@@ -55,7 +60,10 @@ struct BwdParams {
   unsigned char *partials;
   int8_t *partial_exp;  // fp16 rows: power-of-two scale exponent per (position, tile)
   int64_t B, S, S_kv, H, G, topk;
-  int hpg, ntiles;
+  int hpg;
+  int ntiles;   // partial rows per entry: one per 32-head tile, or (wide heads) per 128-head group
+  int htiles;   // 32-head tiles per kv group
+  unsigned char *pd;  // wide heads: P and dS tiles [token, kv group][32-slot block][head tile][P, dS][32 heads][32 slots] bf16
   float sl2;    // sm_scale * log2(e)
   float scale;  // sm_scale
 };

@@ -1,11 +1,10 @@
-// SparseMLA forward and backward for wide heads on gfx950 (d_qk = 576 latent +
+// SparseMLA forward for wide heads on gfx950 (d_qk = 576 latent +
 // rope with d_v = 512: the DeepSeek-V3.2 MLA row and the reference's default
 // head dims; or d_v = 576, what a caller that passes no d_v gets).
 //
-// Reference semantics are those of the narrow kernels:
-// cppmega/megatron/sparse_mla_ops/tilelang_sparse_mla_fwd.py:137-290 (fwd),
-// tilelang_sparse_mla_fwd_fp8.py:187-393 (e4m3 fwd) and
-// tilelang_sparse_mla_bwd.py:123-419 (bwd).
+// Reference semantics are those of the narrow kernel:
+// cppmega/megatron/sparse_mla_ops/tilelang_sparse_mla_fwd.py:137-290 and
+// tilelang_sparse_mla_fwd_fp8.py:187-393 (e4m3).
 //
 // A wide row does not fit one wave's registers: Q over 576 dims is 144 VGPRs
 // per 32 heads and the O accumulator over 512 dims is 256.  So one workgroup of
@@ -21,134 +20,15 @@
 //   * O^T[d][head] += V^T P^T is split over d_v: wave w accumulates every
 //     fourth 32-column tile of d_v, t = w + 4q (V^T read with transposing LDS
 //     reads in accumulator order, P straight from registers).
-// The backward (bf16 and e4m3) splits S and dP the same way, then gives each wave every
-// fourth 32-column tile of d_qk for dQ^T = K^T dS^T and for the per-slot dKV
-// row c^T = Q^T dS^T + dO^T P^T, written at the entry's CSR position as fp16
-// scaled by a per-row power of two fixed from a bound before the products (as
-// in the narrow kernels), or as fp32 with DSA_BWD_FP32_PARTIALS; the kv-major
-// reduction sums those rows in a fixed order.
 #include <type_traits>
 
 #include "dsa_common.hpp"
 #include "sparse_mla_gather.hpp"
 #include "sparse_mla_params.hpp"
 #include "sparse_mla_wide.hpp"
+#include "sparse_mla_wide_tile.hpp"
 
 namespace dsa {
-
-template <int D_QK, int D_V, bool FP8, int NTHR_ = 256>
-struct WideCfg {
-  static constexpr int NTHR = NTHR_;               // threads that gather a block
-  static constexpr int ELT = FP8 ? 1 : 2;          // bytes per element in HBM
-  static constexpr int ROWB = D_QK * ELT;          // bytes per kv row
-  static constexpr int NCH = ROWB / 16;            // 16-byte chunks per row
-  static constexpr int NCH_V = D_V * ELT / 16;     // chunks of the V prefix
-  static constexpr int UNITS = 32 * NCH;           // (row, chunk) units per block
-  static constexpr int UPT = (UNITS + NTHR - 1) / NTHR;  // units per thread
-  static constexpr int KL_STRIDE = ROWB + 32;      // padded LDS row (conflict-free transposed reads)
-  static constexpr int KD_STRIDE = D_V * 2 + 32;   // e4m3: dequantised V rows (bf16)
-  static constexpr int KSTEPS = D_QK / 16;         // 32x32x16 k-steps over d_qk
-  static constexpr int KQ = KSTEPS / 4;            // S k-steps per wave
-  static constexpr int DT = D_V / 32;              // 32-column tiles of d_v
-  static constexpr int DTW = (DT + 3) / 4;         // O^T tiles per wave (tile t = w + 4 q, t < DT)
-  static_assert(ROWB % 16 == 0 && (D_V * ELT) % 16 == 0, "rows must be whole 16-byte chunks");
-  static_assert(KSTEPS % 4 == 0 && D_V % 32 == 0 && D_V <= D_QK, "head dims must split over four waves");
-  struct Regs {
-    i32x4 v[UPT];
-    float sc[UPT];
-    uint32_t valid;  // bit i: unit i is a real (unmasked) slot's chunk
-  };
-};
-
-// Issue the loads of one block's 32 rows: thread t takes units t + NTHR i,
-// unit u = chunk u % NCH of row u / NCH.  my_idx is the kv row of slot
-// (lane & 31) of this wave (-1: masked).
-// kv_scale_b holds one scale per row (sc_pitch 1) or, MX, one per 32-channel
-// block of every row (sc_pitch floats apart): a unit loads its own block's.
-// UNCOND (the backward): the loads are unconditional, a unit past the block
-// (or a masked slot) reading row 0, which wide_store drops, so that every wave
-// issues the same loads on every block.
-template <class C, bool FP8, bool MX = false, bool UNCOND = false>
-__device__ __forceinline__ void wide_issue(typename C::Regs &rg, const unsigned char *kv_b, const float *kv_scale_b,
-                                           int my_idx, uint32_t row_pitch, uint32_t sc_pitch = 1u) {
-  const int t = threadIdx.x;
-  uint32_t valid = 0;
-#pragma unroll
-  for (int i = 0; i < C::UPT; ++i) {
-    const int u = t + C::NTHR * i;
-    const int row = (u / C::NCH) & 31;
-    const int c = u % C::NCH;
-    const int ri = __shfl(my_idx, row, 64);
-    const bool exists = (i + 1 < C::UPT) || u < C::UNITS;
-    const bool ok = ri >= 0 && exists;
-    const uint32_t r = ok ? (uint32_t)ri : 0u;
-    if constexpr (UNCOND) {
-      rg.v[i] = ld_global_16(kv_b + r * row_pitch + c * 16);
-      if constexpr (FP8) rg.sc[i] = kv_scale_b[r * sc_pitch + (MX ? (uint32_t)(c >> 1) : 0u)];
-    } else {
-      rg.v[i] = i32x4{0, 0, 0, 0};
-      if (exists) rg.v[i] = ld_global_16(kv_b + r * row_pitch + c * 16);
-      if constexpr (FP8) rg.sc[i] = exists ? kv_scale_b[r * sc_pitch + (MX ? (uint32_t)(c >> 1) : 0u)] : 0.0f;
-    }
-    valid |= (ok ? 1u : 0u) << i;
-  }
-  rg.valid = valid;
-}
-
-// Store the staged rows: raw bytes row-major into Kl (masked slots zero); for
-// e4m3 also the first NCH_D chunks dequantised to bf16 (value * kv_scale, RNE)
-// into Kd (row stride KD_STRIDE) and the per-slot scales into Ksc (MX: the
-// per-(slot, block) scales, block-major Ksc[block * 32 + slot]).
-template <class C, bool FP8, int NCH_D = C::NCH_V, int KD_STRIDE = C::KD_STRIDE, bool MX = false>
-__device__ __forceinline__ void wide_store(const typename C::Regs &rg, unsigned char *Kl, unsigned char *Kd,
-                                           float *Ksc) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < C::UPT; ++i) {
-    const int u = t + C::NTHR * i;
-    if ((i + 1 < C::UPT) || u < C::UNITS) {
-      const int row = u / C::NCH, c = u % C::NCH;
-      const bool ok = (rg.valid >> i) & 1u;
-      const i32x4 v = ok ? rg.v[i] : i32x4{0, 0, 0, 0};
-      *reinterpret_cast<i32x4 *>(Kl + row * C::KL_STRIDE + c * 16) = v;
-      if constexpr (FP8) {
-        const float s = ok ? rg.sc[i] : 0.0f;
-        if (c < NCH_D) {
-          uint32_t wd[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const f32x2 v2 = e4m3x2_to_f32((uint32_t)v[e >> 1], (e & 1) != 0);
-            wd[e] = pack_bf16x2(v2[0] * s, v2[1] * s);
-          }
-          unsigned char *dst = Kd + row * KD_STRIDE + c * 32;
-          *reinterpret_cast<i32x4 *>(dst) = i32x4{(int)wd[0], (int)wd[1], (int)wd[2], (int)wd[3]};
-          *reinterpret_cast<i32x4 *>(dst + 16) = i32x4{(int)wd[4], (int)wd[5], (int)wd[6], (int)wd[7]};
-        }
-        if constexpr (MX) {
-          if ((c & 1) == 0) Ksc[(c >> 1) * 32 + row] = s;
-        } else if (c == 0) {
-          Ksc[row] = s;
-        }
-      }
-    }
-  }
-}
-
-// Sum of the four waves' partial 32x32 fp32 tiles (stored lane-linear per wave:
-// Sp[w][q4][lane][4]) in wave order: the same bits in every wave.
-__device__ __forceinline__ void sum_partials(const float *Sp, int stride_w, float (&s)[16]) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int q4 = 0; q4 < 4; ++q4) {
-    const f32x4 v0 = *reinterpret_cast<const f32x4 *>(Sp + 0 * stride_w + (q4 * 64 + lane) * 4);
-    const f32x4 v1 = *reinterpret_cast<const f32x4 *>(Sp + 1 * stride_w + (q4 * 64 + lane) * 4);
-    const f32x4 v2 = *reinterpret_cast<const f32x4 *>(Sp + 2 * stride_w + (q4 * 64 + lane) * 4);
-    const f32x4 v3 = *reinterpret_cast<const f32x4 *>(Sp + 3 * stride_w + (q4 * 64 + lane) * 4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) s[4 * q4 + j] = ((v0[j] + v1[j]) + v2[j]) + v3[j];
-    __builtin_amdgcn_sched_barrier(0);  // bound the loads in flight (register pressure)
-  }
-}
 
 // Split form of sum_partials for four waves: wave w sums quarter w (64 lanes x
 // 4 floats) of the four partial tiles in the same order and writes it to the
@@ -173,14 +53,6 @@ __device__ __forceinline__ void get_reduced(const float *Sr, float (&s)[16]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) s[4 * q4 + j] = v[j];
   }
-}
-
-__device__ __forceinline__ void put_partial(float *dst, const f32x16 &acc) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int q4 = 0; q4 < 4; ++q4)
-    *reinterpret_cast<f32x4 *>(dst + (q4 * 64 + lane) * 4) =
-        f32x4{acc[4 * q4], acc[4 * q4 + 1], acc[4 * q4 + 2], acc[4 * q4 + 3]};
 }
 
 // ---------------------------------------------------------------------------
@@ -490,414 +362,6 @@ int launch_fwd_wide(const FwdParams &p, int64_t d_qk, int64_t d_v, bool fp8, hip
   if (d_qk == 576 && d_v == 512) return fp8 ? launch_fwd_wide_t<576, 512, true>(p, st) : launch_fwd_wide_t<576, 512, false>(p, st);
   if (d_qk == 576 && d_v == 576) return fp8 ? launch_fwd_wide_t<576, 576, true>(p, st) : launch_fwd_wide_t<576, 576, false>(p, st);
   return set_error(DSA_ERR_UNSUPPORTED, "sparse_mla_fwd(wide): no kernel for d_qk=%lld d_v=%lld", (long long)d_qk,
-                   (long long)d_v);
-}
-
-// ---------------------------------------------------------------------------
-// Backward main pass (bf16 and e4m3)
-// ---------------------------------------------------------------------------
-// LDS of one workgroup: QL [head][d] and DOL [head][d] (bf16; e4m3 Q
-// dequantised, for the S / dP A operands and the transposed Q^T / dO^T
-// operands), LD = LSE (heads 0..31) and Delta * sm_scale (32..63), Kl [slot][d]
-// gathered rows (raw bytes), for e4m3 also Kd [slot][d] (rows dequantised to
-// bf16, the V and K operands of dP and dQ) and Ksc (row scales), the waves'
-// partial score tiles, and one dS[slot][head] tile per wave.  bf16 exchanges
-// the S and dP partials together (8 tiles); e4m3 has room for four and
-// exchanges them one after the other, as the reference's e4m3 kernel computes
-// QK^T on the codes and the other products on dequantised bf16.
-template <int D_QK, int D_V, bool FP8>
-struct WideBwdLds {
-  // (after DS) MX: per-wave max |Q| (0..3) and max |dO| (4..7) of the item
-  using C = WideCfg<D_QK, D_V, FP8>;
-  static constexpr int QL_STRIDE = D_QK * 2 + 32;
-  static constexpr int DOL_STRIDE = D_V * 2 + 32;
-  static constexpr int DS_STRIDE = 32 * 2 + 32;
-  static constexpr int KDB_STRIDE = D_QK * 2 + 32;  // e4m3: whole rows dequantised
-  static constexpr int OFF_QL = 0;
-  static constexpr int OFF_DOL = OFF_QL + 32 * QL_STRIDE;
-  static constexpr int OFF_LD = OFF_DOL + 32 * DOL_STRIDE;
-  static constexpr int OFF_KL = OFF_LD + 64 * 4;
-  static constexpr int OFF_KD = OFF_KL + 32 * C::KL_STRIDE;
-  static constexpr int OFF_SC = OFF_KD + (FP8 ? 32 * KDB_STRIDE : 0);
-  static constexpr int OFF_SP = OFF_SC + (FP8 ? 32 * 4 : 0);
-  static constexpr int SP_W = 16 * 64;  // floats per partial tile
-  static constexpr int SP_TILES = FP8 ? 4 : 8;
-  static constexpr int OFF_DS = OFF_SP + SP_TILES * SP_W * 4;
-  static constexpr int OFF_MX = OFF_DS + 4 * 32 * DS_STRIDE;
-  static constexpr int BYTES = OFF_MX + 8 * 4;
-  static_assert(BYTES <= 160 * 1024, "wide backward LDS");
-};
-
-template <int D_QK, int D_V, bool FP8, bool F32P>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1)))
-sparse_mla_bwd_wide_kernel(const BwdParams p) {
-  using C = WideCfg<D_QK, D_V, FP8>;
-  using L = WideBwdLds<D_QK, D_V, FP8>;
-  constexpr int DQT = D_QK / 32;          // 32-column tiles of d_qk
-  constexpr int DQW = (DQT + 3) / 4;      // tiles per wave (tile t = w + 4 q)
-  constexpr int DVT = D_V / 32;
-  constexpr int VQ = D_V / 16 / 4;        // dP k-steps per wave
-  static_assert((D_V / 16) % 4 == 0, "d_v k-steps split over four waves");
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-
-  const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
-  const int g32 = lane >> 5, l32 = lane & 31;
-  const int64_t item = xcd_remap(blockIdx.x, gridDim.x);
-  const int tile = (int)(item % p.ntiles);
-  const int64_t rest = item / p.ntiles;
-  const int64_t g = rest % p.G;
-  const int64_t tok = rest / p.G;
-  const int64_t b = tok / p.S;
-
-  unsigned char *QL = smem + L::OFF_QL;
-  unsigned char *DOL = smem + L::OFF_DOL;
-  float *LD = reinterpret_cast<float *>(smem + L::OFF_LD);
-  unsigned char *Kl = smem + L::OFF_KL;
-  unsigned char *Kd = smem + L::OFF_KD;
-  float *Ksc = reinterpret_cast<float *>(smem + L::OFF_SC);
-  float *Sp = reinterpret_cast<float *>(smem + L::OFF_SP);
-  const unsigned char *Ksrc = FP8 ? Kd : Kl;  // bf16 K / V rows for dP and dQ
-  constexpr int K_STRIDE = FP8 ? L::KDB_STRIDE : C::KL_STRIDE;
-  unsigned char *DS = smem + L::OFF_DS + w * 32 * L::DS_STRIDE;
-  float *MX = reinterpret_cast<float *>(smem + L::OFF_MX);
-
-  const int64_t head0 = tok * p.H + g * p.hpg + tile * 32;
-  const int nheads = p.hpg - tile * 32 < 32 ? p.hpg - tile * 32 : 32;
-  const int64_t entry0 = (tok * p.G + g) * p.topk;
-  const int64_t n_entries = p.B * p.S * p.G * p.topk;
-  const int32_t *idx_row = p.idx + entry0;
-  const unsigned char *kv_b = p.kv + ((b * p.S_kv) * p.G + g) * C::ROWB;
-  const float *kv_scale_b = FP8 ? p.kv_scale + b * p.S_kv : nullptr;
-  const uint32_t row_pitch = (uint32_t)(p.G * C::ROWB);
-
-  // Indices (two blocks ahead), rows and CSR positions (one block ahead) are
-  // loaded unconditionally through resources that end at the item's top-k, and
-  // every partial-row store is unconditional (masked slots write the trash row
-  // past the entries), so each wave issues the same memory operations on every
-  // block and the compiler's waits count exactly: waiting for a block's rows
-  // or positions leaves the previous block's stores in flight.
-  const auto idx_rs = slot_rsrc(idx_row, p.topk);
-  const auto pos_rs = slot_rsrc(p.pos_of + entry0, p.topk);
-  int idx_cur = slot_index(load_slot_raw(idx_rs, 0, l32), 0, l32, p.topk, p.S_kv);
-  int raw_nxt = load_slot_raw(idx_rs, 1, l32);
-  typename C::Regs rg;
-  wide_issue<C, FP8, false, true>(rg, kv_b, kv_scale_b, idx_cur, row_pitch);
-  int pos_cur = load_slot_raw(pos_rs, 0, l32);
-  // blocks up to the last valid slot: the same count in every wave (the loop has workgroup barriers)
-  const int nblk = valid_blocks(idx_rs, p.topk, p.S_kv);
-  // partial row no entry owns (this workgroup's trash row)
-  const uint64_t trash = (uint64_t)n_entries * (uint64_t)p.ntiles + (uint64_t)(item % kTrashRows);
-
-  float qsc = 1.0f;
-  if constexpr (FP8) qsc = p.q_scale[tok];
-  // ---------------- prologue: Q, dO tiles, LSE, Delta ----------------
-  {
-    const int t = threadIdx.x;
-    constexpr int QCH = D_QK / 8;
-    float mq = 0.0f, md = 0.0f;  // max |Q|, |dO| seen by this thread (fp16 rows only)
-    for (int u = t; u < 32 * QCH; u += 256) {
-      const int h = u / QCH, c = u % QCH;
-      i32x4 v = {0, 0, 0, 0};
-      if (h < nheads) {
-        if constexpr (FP8) {
-          const unsigned long raw = *reinterpret_cast<const unsigned long *>(p.q + (head0 + h) * D_QK + 8 * c);
-          uint32_t wq[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {  // codes 2e, 2e + 1 of the 8 in raw
-            const f32x2 v2 = e4m3x2_to_f32((uint32_t)(raw >> (32 * (e >> 1))), (e & 1) != 0);
-            wq[e] = pack_bf16x2(v2[0] * qsc, v2[1] * qsc);
-          }
-          v = i32x4{(int)wq[0], (int)wq[1], (int)wq[2], (int)wq[3]};
-        } else {
-          v = ld_global_16(p.q + ((head0 + h) * D_QK + 8 * c) * 2);
-        }
-      }
-      *reinterpret_cast<i32x4 *>(QL + h * L::QL_STRIDE + c * 16) = v;
-      if constexpr (!F32P) mq = fmaxf(mq, bf16x8_absmax(v));
-    }
-    // dO rows and Delta = sum_d O dO: one wave per head, lane = 8-element chunk
-    constexpr int VCH = D_V / 8;
-    for (int h = w; h < 32; h += 4) {
-      float part = 0.0f;
-      for (int c = lane; c < VCH; c += 64) {
-        i32x4 dv = {0, 0, 0, 0}, ov = {0, 0, 0, 0};
-        if (h < nheads) {
-          dv = ld_global_16(p.dO + (head0 + h) * D_V + 8 * c);
-          ov = ld_global_16(p.o + (head0 + h) * D_V + 8 * c);
-        }
-        *reinterpret_cast<i32x4 *>(DOL + h * L::DOL_STRIDE + c * 16) = dv;
-        if constexpr (!F32P) md = fmaxf(md, bf16x8_absmax(dv));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t du = (uint32_t)dv[e], ou = (uint32_t)ov[e];
-          part += bf16_bits_to_f32(ou & 0xffffu) * bf16_bits_to_f32(du & 0xffffu);
-          part += bf16_bits_to_f32(ou >> 16) * bf16_bits_to_f32(du >> 16);
-        }
-      }
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) part += __shfl_xor(part, off, 64);
-      if (lane == 0) {
-        float dl = part;
-        if (p.delta != nullptr && h < nheads) dl = p.delta[head0 + h];
-        LD[32 + h] = dl * p.scale;
-      }
-    }
-    if (t < 32) {
-      float lse_h = INFINITY;  // padded heads: P = exp2(x - inf) = 0
-      if (t < nheads) {
-        const float l = p.lse[head0 + t];
-        lse_h = (l == -INFINITY) ? INFINITY : l;  // all-masked row: zero gradient
-      }
-      LD[t] = lse_h;
-    }
-    if constexpr (!F32P) {
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) {
-        mq = fmaxf(mq, __shfl_xor(mq, off, 64));
-        md = fmaxf(md, __shfl_xor(md, off, 64));
-      }
-      if (lane == 0) {
-        MX[w] = mq;
-        MX[4 + w] = md;
-      }
-    }
-  }
-
-  // e4m3: this wave's quarter of the raw Q codes, the A operand of QK^T (head l32)
-  long qA8[FP8 ? C::KQ : 1];
-  if constexpr (FP8) {
-#pragma unroll
-    for (int k = 0; k < C::KQ; ++k)
-      qA8[k] = l32 < nheads ? *reinterpret_cast<const long *>(p.q + (head0 + l32) * D_QK + 16 * (w * C::KQ + k) + 8 * g32)
-                            : 0l;
-  }
-  f32x16 dqacc[DQW];
-#pragma unroll
-  for (int q = 0; q < DQW; ++q)
-#pragma unroll
-    for (int a = 0; a < 16; ++a) dqacc[q][a] = 0.0f;
-
-  const int k0 = w * C::KQ, v0 = w * VQ;
-  // the first block's rows and positions have landed: nothing is in flight on
-  // entry, so the loop's waits follow its own order (s_waitcnt vmcnt(0) with
-  // expcnt and lgkmcnt left open, gfx9 encoding)
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  for (int blk = 0; blk < nblk; ++blk) {
-    const int slot0 = blk * 32;
-    wide_store<C, FP8, C::NCH, L::KDB_STRIDE>(rg, Kl, Kd, Ksc);
-    const bool valid = idx_cur >= 0;  // slot slot0 + l32
-    const int32_t pos = pos_cur;
-    const bool wr = valid && pos >= 0 && pos < n_entries;  // (always true for a valid slot; a guard)
-    __syncthreads();  // rows (and, on the first block, the prologue tiles) are in LDS
-    const int raw_nn = load_slot_raw(idx_rs, blk + 2, l32);
-    const int idx_nxt = slot_index(raw_nxt, blk + 1, l32, p.topk, p.S_kv);
-    wide_issue<C, FP8, false, true>(rg, kv_b, kv_scale_b, idx_nxt, row_pitch);  // past the last block too
-    const int pos_nxt = load_slot_raw(pos_rs, blk + 1, l32);
-
-    // ---- partial S = Q K^T and dP = dO V^T (M = head, N = slot) over this wave's k-steps ----
-    f32x16 sacc, dpacc;
-#pragma unroll
-    for (int a = 0; a < 16; ++a) {
-      sacc[a] = 0.0f;
-      dpacc[a] = 0.0f;
-    }
-#pragma unroll
-    for (int k = 0; k < C::KQ; ++k) {
-      const int d0 = 16 * (k0 + k) + 8 * g32;
-      if constexpr (FP8) {
-        const long kb = *reinterpret_cast<const long *>(Kl + l32 * C::KL_STRIDE + d0);
-        sacc = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(qA8[k], kb, sacc, 0, 0, 0);
-      } else {
-        const i32x4 qa = *reinterpret_cast<const i32x4 *>(QL + l32 * L::QL_STRIDE + d0 * 2);
-        const i32x4 kb = *reinterpret_cast<const i32x4 *>(Kl + l32 * C::KL_STRIDE + d0 * 2);
-        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(qa), as_bf16x8(kb), sacc, 0, 0, 0);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < VQ; ++k) {
-      const int d0 = 16 * (v0 + k) + 8 * g32;
-      const i32x4 da = *reinterpret_cast<const i32x4 *>(DOL + l32 * L::DOL_STRIDE + d0 * 2);
-      const i32x4 vb = *reinterpret_cast<const i32x4 *>(Ksrc + l32 * K_STRIDE + d0 * 2);
-      dpacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(da), as_bf16x8(vb), dpacc, 0, 0, 0);
-    }
-    float s[16], dp[16];
-    if constexpr (FP8) {
-      put_partial(Sp + w * L::SP_W, sacc);
-      __syncthreads();  // S partial tiles written
-      sum_partials(Sp, L::SP_W, s);
-      __syncthreads();  // read before the dP partials reuse the tiles
-      put_partial(Sp + w * L::SP_W, dpacc);
-      __syncthreads();
-      sum_partials(Sp, L::SP_W, dp);
-    } else {
-      put_partial(Sp + (2 * w) * L::SP_W, sacc);
-      put_partial(Sp + (2 * w + 1) * L::SP_W, dpacc);
-      __syncthreads();  // all partial tiles written
-      sum_partials(Sp, 2 * L::SP_W, s);
-      sum_partials(Sp + L::SP_W, 2 * L::SP_W, dp);
-    }
-
-    // ---- P, dS (lane = slot slot0 + l32, heads 8i + 4*g32 + j; identical in every wave) ----
-    float xs = p.sl2;
-    if constexpr (FP8) xs *= qsc * Ksc[l32];
-    bf16x8 dsB[2], pB[2];
-    int pexp = 0;  // fp16 rows: the slot's partial-row scale exponent (identical in every wave)
-    {
-      uint32_t dsw[8], pw[8];
-      float P[16], dS[16];
-      float sabs = 0.0f, psum = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const f32x4 l4 = *reinterpret_cast<const f32x4 *>(LD + 8 * i + 4 * g32);
-        const f32x4 d4 = *reinterpret_cast<const f32x4 *>(LD + 32 + 8 * i + 4 * g32);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int a = 4 * i + j;
-          const float pv = valid ? exp2_fast(s[a] * xs - l4[j]) : 0.0f;
-          P[a] = pv;
-          dS[a] = pv * fmaf(dp[a], p.scale, -d4[j]);
-          sabs += fabsf(dS[a]);
-          psum += pv;
-        }
-        dsw[2 * i] = pack_bf16x2(dS[4 * i], dS[4 * i + 1]);
-        dsw[2 * i + 1] = pack_bf16x2(dS[4 * i + 2], dS[4 * i + 3]);
-        *reinterpret_cast<i32x2 *>(DS + l32 * L::DS_STRIDE + (8 * i + 4 * g32) * 2) =
-            i32x2{(int)dsw[2 * i], (int)dsw[2 * i + 1]};
-      }
-      float rs = 1.0f;
-      if constexpr (!F32P) {
-        // |c[d]| <= max|Q| sum_h |dS_h| + max|dO| sum_h P_h over the slot's 32
-        // heads; the margin 2^-6 covers the bf16 rounding of dS / P (2^-8) and
-        // the fp32 sums.  c is computed from dS 2^s and P 2^s (exact scalings).
-        const float maxq = fmaxf(fmaxf(MX[0], MX[1]), fmaxf(MX[2], MX[3]));
-        const float maxdo = fmaxf(fmaxf(MX[4], MX[5]), fmaxf(MX[6], MX[7]));
-        const float bnd = sum_halves(fmaf(maxq, sabs, maxdo * psum)) * 1.015625f;
-        pexp = partial_row_exponent_bound(bnd);
-        rs = exp2i(pexp);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          dsw[2 * i] = pack_bf16x2(dS[4 * i] * rs, dS[4 * i + 1] * rs);
-          dsw[2 * i + 1] = pack_bf16x2(dS[4 * i + 2] * rs, dS[4 * i + 3] * rs);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        pw[2 * i] = pack_bf16x2(P[4 * i] * rs, P[4 * i + 1] * rs);
-        pw[2 * i + 1] = pack_bf16x2(P[4 * i + 2] * rs, P[4 * i + 3] * rs);
-      }
-#pragma unroll
-      for (int kc = 0; kc < 2; ++kc) {
-        dsB[kc] = as_bf16x8(i32x4{(int)dsw[4 * kc], (int)dsw[4 * kc + 1], (int)dsw[4 * kc + 2], (int)dsw[4 * kc + 3]});
-        pB[kc] = as_bf16x8(i32x4{(int)pw[4 * kc], (int)pw[4 * kc + 1], (int)pw[4 * kc + 2], (int)pw[4 * kc + 3]});
-      }
-    }
-    wave_lds_sync();  // this wave's dS tile
-
-    // ---- dQ^T[d][head] += K^T[d][slot] dS^T[slot][head] on tiles t = w + 4q ----
-#pragma unroll
-    for (int kc = 0; kc < 2; ++kc) {
-      const i32x4 bv = tr_operand(DS, L::DS_STRIDE, 0, 16 * kc, 4, 8);
-#pragma unroll
-      for (int q = 0; q < DQW; ++q) {
-        const int t = w + 4 * q;
-        if (t < DQT) {
-          const i32x4 av = tr_operand(Ksrc, K_STRIDE, t * 32, 16 * kc, 4, 8);
-          dqacc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(av), as_bf16x8(bv), dqacc[q], 0, 0, 0);
-        }
-      }
-    }
-
-    // ---- c^T[d][slot] = Q^T dS^T + dO^T P^T on tiles t = w + 4q (fp16 rows: times 2^pexp) ----
-    const uint64_t prow = wr ? (uint64_t)(uint32_t)pos * (uint32_t)p.ntiles + tile : trash;
-    unsigned char *dst = p.partials + prow * (uint64_t)(D_QK * (F32P ? 4 : 2));
-    if constexpr (!F32P) p.partial_exp[prow] = (int8_t)pexp;  // every wave and lane half stores the same byte
-#pragma unroll
-    for (int q = 0; q < DQW; ++q) {
-      // a wave without a tile of its own on the last step redoes tile DQT - 1
-      // and stores the same bits again, so that every wave issues the same
-      // stores on every block
-      const int t = w + 4 * q < DQT ? w + 4 * q : DQT - 1;
-      {
-        f32x16 cacc;
-#pragma unroll
-        for (int a = 0; a < 16; ++a) cacc[a] = 0.0f;
-#pragma unroll
-        for (int kc = 0; kc < 2; ++kc) {
-          const i32x4 av = tr_operand(QL, L::QL_STRIDE, t * 32, 16 * kc, 8, 4);
-          cacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(av), dsB[kc], cacc, 0, 0, 0);
-        }
-        if (t < DVT) {
-#pragma unroll
-          for (int kc = 0; kc < 2; ++kc) {
-            const i32x4 av = tr_operand(DOL, L::DOL_STRIDE, t * 32, 16 * kc, 8, 4);
-            cacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(av), pB[kc], cacc, 0, 0, 0);
-          }
-        }
-        {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int d0 = t * 32 + 8 * i + 4 * g32;
-            // plain (write-back) stores: a row's pieces come from four waves and
-            // several instructions, and L2 merges them into whole lines
-            if constexpr (F32P) {
-              *reinterpret_cast<f32x4 *>(dst + d0 * 4) = f32x4{cacc[4 * i], cacc[4 * i + 1], cacc[4 * i + 2],
-                                                               cacc[4 * i + 3]};
-            } else {
-              *reinterpret_cast<i32x2 *>(dst + d0 * 2) =
-                  i32x2{(int)pack_f16x2(cacc[4 * i], cacc[4 * i + 1]), (int)pack_f16x2(cacc[4 * i + 2], cacc[4 * i + 3])};
-            }
-          }
-        }
-      }
-    }
-    __syncthreads();  // rows, partial tiles and dS tiles consumed before the next block
-    idx_cur = idx_nxt;
-    raw_nxt = raw_nn;
-    pos_cur = pos_nxt;
-  }
-
-  // ---- dQ: lane = head l32, d = t*32 + 8i + 4*g32 + j ----
-  if (l32 < nheads) {
-    uint16_t *drow = p.dq + (head0 + l32) * D_QK;
-#pragma unroll
-    for (int q = 0; q < DQW; ++q) {
-      const int t = w + 4 * q;
-      if (t < DQT) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const i32x2 pk = {(int)pack_bf16x2(dqacc[q][4 * i], dqacc[q][4 * i + 1]),
-                            (int)pack_bf16x2(dqacc[q][4 * i + 2], dqacc[q][4 * i + 3])};
-          *reinterpret_cast<i32x2 *>(drow + t * 32 + 8 * i + 4 * g32) = pk;
-        }
-      }
-    }
-  }
-}
-
-template <int D_QK, int D_V, bool FP8, bool F32P>
-static int launch_bwd_wide_t(const BwdParams &p, hipStream_t st) {
-  using L = WideBwdLds<D_QK, D_V, FP8>;
-  const size_t lds = L::BYTES;
-  hipError_t e = hipFuncSetAttribute((const void *)sparse_mla_bwd_wide_kernel<D_QK, D_V, FP8, F32P>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return set_error(DSA_ERR_HIP, "sparse_mla_bwd(wide): LDS attribute: %s", hipGetErrorString(e));
-  const int64_t nitems = p.B * p.S * p.G * p.ntiles;
-  if (nitems >= (1ll << 31)) return set_error(DSA_ERR_INVALID_ARG, "sparse_mla_bwd(wide): grid too large");
-  hipLaunchKernelGGL((sparse_mla_bwd_wide_kernel<D_QK, D_V, FP8, F32P>), dim3((unsigned)nitems), dim3(256), lds, st,
-                     p);
-  return check_launch("sparse_mla_bwd_main(wide)");
-}
-
-template <int D_QK, int D_V>
-static int launch_bwd_wide_f(const BwdParams &p, bool fp8, bool f32p, hipStream_t st) {
-  if (fp8) return f32p ? launch_bwd_wide_t<D_QK, D_V, true, true>(p, st) : launch_bwd_wide_t<D_QK, D_V, true, false>(p, st);
-  return f32p ? launch_bwd_wide_t<D_QK, D_V, false, true>(p, st) : launch_bwd_wide_t<D_QK, D_V, false, false>(p, st);
-}
-
-int launch_bwd_main_wide(const BwdParams &p, int64_t d_qk, int64_t d_v, bool fp8, bool f32p, hipStream_t st) {
-  if (d_qk == 576 && d_v == 512) return launch_bwd_wide_f<576, 512>(p, fp8, f32p, st);
-  if (d_qk == 576 && d_v == 576) return launch_bwd_wide_f<576, 576>(p, fp8, f32p, st);
-  return set_error(DSA_ERR_UNSUPPORTED, "sparse_mla_bwd(wide): no kernel for d_qk=%lld d_v=%lld", (long long)d_qk,
                    (long long)d_v);
 }
 

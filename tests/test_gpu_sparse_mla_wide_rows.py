@@ -1,0 +1,63 @@
+"""The wide backward's two kernels at the edges of their splits: head groups of
+one partial row (128 heads), 32-head tiles per workgroup (one, two, an odd
+count), kv groups, 32-slot blocks, and both partial-row formats, against the
+oracle at the usual bar (2e-2 relative / 1e-2 absolute)."""
+import pytest
+import torch
+
+from cppmega_amd import synthetic
+from cppmega_amd.sparse_mla_ops import sparse_mla_bwd, sparse_mla_bwd_fp8, sparse_mla_fwd_fp8_interface, \
+    sparse_mla_fwd_interface
+from oracle import fp8 as ofp8
+from oracle import sparse_mla as orc
+from tests._util import assert_close
+
+pytestmark = pytest.mark.gpu
+
+D = 576
+
+
+@pytest.mark.parametrize("S,S_kv,H,G,DV,topk,fp32_rows", [
+    (24, 24, 8, 1, 512, 32, False),      # one partial head tile
+    (20, 90, 160, 1, 512, 33, False),    # two rows per entry, the second of one tile; ragged last block
+    (20, 90, 288, 1, 512, 31, True),     # three rows per entry, fp32
+    (18, 70, 192, 2, 512, 65, False),    # two kv groups of three head tiles
+    (24, 40, 40, 1, 576, 96, False),     # V the whole row, a ragged second tile
+    (1, 300, 128, 1, 512, 257, False),   # one token
+])
+def test_wide_rows_splits(dev, S, S_kv, H, G, DV, topk, fp32_rows):
+    g = torch.Generator().manual_seed(H + topk)
+    q = (torch.randn((1, S, H, D), generator=g) * 0.5).to(torch.bfloat16)
+    kv = (torch.randn((1, S_kv, G, D), generator=g) * 0.5).to(torch.bfloat16)
+    do = torch.randn((1, S, H, DV), generator=g).to(torch.bfloat16)
+    idx = torch.rand((1, S, G, max(S_kv, topk)), generator=g).argsort(dim=-1)[..., :topk].to(torch.int32)
+    idx[idx >= S_kv] = -1
+    idx[0, 0, 0, ::3] = -1                                  # unsorted, masked slots throughout
+    idx = idx.contiguous()
+    scale = D ** -0.5
+    qd, kd, dod, idd = q.to(dev), kv.to(dev), do.to(dev), idx.to(dev)
+    out, lse = sparse_mla_fwd_interface(qd, kd, idd, sm_scale=scale, d_v=DV)
+    dq, dkv = sparse_mla_bwd(qd, kd, out, dod, idd, lse, sm_scale=scale, fp32_partials=fp32_rows)
+    rdq, rdkv = orc.sparse_mla_bwd(q, kv, out.cpu(), do, idx, lse.cpu(), scale, DV)
+    assert_close(dq, rdq, what="dq")
+    assert_close(dkv, rdkv, what="dkv")
+    dq2, dkv2 = sparse_mla_bwd(qd, kd, out, dod, idd, lse, sm_scale=scale, fp32_partials=fp32_rows)
+    assert torch.equal(dq, dq2) and torch.equal(dkv, dkv2)
+
+
+def test_wide_rows_e4m3_two_rows_per_entry(dev):
+    S, H, DV, topk = 40, 160, 512, 40
+    q = (torch.randn((1, S, H, D), generator=torch.Generator().manual_seed(1)) * 0.5).to(torch.bfloat16)
+    kv = (torch.randn((1, S, 1, D), generator=torch.Generator().manual_seed(2)) * 0.5).to(torch.bfloat16)
+    do = torch.randn((1, S, H, DV), generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
+    idx = synthetic.causal_indices(1, S, topk, seed=4)
+    q8, qs = ofp8.tensorwise_quantize(q)
+    k8, ks = ofp8.tensorwise_quantize(kv)
+    qsv, ksv = qs.expand(1, S).contiguous(), ks.expand(1, S).contiguous()
+    args = [t.to(dev) for t in (q8, k8, qsv, ksv)]
+    out, lse = sparse_mla_fwd_fp8_interface(args[0], args[1], idx.to(dev), q_scale=args[2], kv_scale=args[3],
+                                            sm_scale=D ** -0.5, d_v=DV)
+    dq, dkv = sparse_mla_bwd_fp8(*args, out, do.to(dev), idx.to(dev), lse, sm_scale=D ** -0.5)
+    rdq, rdkv = orc.sparse_mla_bwd(q8, k8, out.cpu(), do, idx, lse.cpu(), D ** -0.5, DV, q_scale=qsv, kv_scale=ksv)
+    assert_close(dq, rdq, what="dq")
+    assert_close(dkv, rdkv, what="dkv")
