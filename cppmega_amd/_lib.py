@@ -36,6 +36,7 @@ EXPORTED_SYMBOLS = (
     "dsa_device_check",
     "dsa_sparse_mla_fwd",
     "dsa_sparse_mla_fwd_workspace_size",
+    "dsa_sparse_mla_fwd_call_workspace_size",
     "dsa_sparse_mla_fwd_ws",
     "dsa_sparse_mla_bwd_workspace_size",
     "dsa_sparse_mla_bwd_index_size",
@@ -84,6 +85,7 @@ _SIGNATURES = {
                                   _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                   _f32, _i32, _c_void_p, _c_void_p, _c_void_p]),
     "dsa_sparse_mla_fwd_workspace_size": (_size_t, [_i64] * 5 + [_i32]),
+    "dsa_sparse_mla_fwd_call_workspace_size": (_size_t, [_i64] * 8 + [_i32]),
     "dsa_sparse_mla_fwd_ws": (_i32, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                      _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                      _f32, _i32, _c_void_p, _c_void_p, _c_void_p, _size_t, _c_void_p]),

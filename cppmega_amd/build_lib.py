@@ -45,6 +45,7 @@ FILE_FLAGS = {
     "sparse_mla_fwd.hip": _MFMA_VGPR + ["-fno-honor-nans", "-mno-amdgpu-ieee"],
     "sparse_mla_bwd.hip": _MFMA_VGPR,
     "sparse_mla_wide.hip": _MFMA_VGPR,
+    "sparse_mla_wide_bf16.hip": _MFMA_VGPR,
     "sparse_mla_wide_bwd.hip": _MFMA_VGPR,
     "indexer_kl_loss.hip": _MFMA_VGPR,
     "indexer_bwd.hip": _MFMA_VGPR,

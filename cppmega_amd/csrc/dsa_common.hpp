@@ -312,16 +312,17 @@ __device__ __forceinline__ i32x4 make_buffer_words(const void *base, uint32_t nu
 __device__ __forceinline__ uint32_t lds_address(const void *p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char *)p;
 }
-// LDS-DMA: lane l's 16 bytes at byte voffset of the resource (zeros past its
-// end) go to LDS bytes lds + 16 l .. + 15, lds wave-uniform.  Written in asm
+// LDS-DMA: lane l's 16 bytes at byte voffset + soffset of the resource (zeros
+// where voffset is past its end) go to LDS bytes lds + 16 l .. + 15; lds and
+// soffset are wave-uniform.  Written in asm
 // because the builtin makes every later LDS read wait for all such loads; the
 // caller waits (vmcnt) before the barrier that publishes the data.  No register
 // is written, and the compiler's own vmcnt waits, which do not count this load,
 // only become stricter by it.
-__device__ __forceinline__ void lds_dma_16(uint32_t lds, uint32_t voffset, i32x4 rs) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+__device__ __forceinline__ void lds_dma_16(uint32_t lds, uint32_t voffset, i32x4 rs, uint32_t soffset) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                :
-               : "s"(lds), "v"(voffset), "s"(rs)
+               : "s"(lds), "v"(voffset), "s"(rs), "s"(soffset)
                : "memory", "m0");
 }
 

@@ -422,6 +422,11 @@ static size_t v16_bytes(int64_t B, int64_t S_kv, int64_t G, int64_t D_v) {
   return ((size_t)B * S_kv * G * D_v * 2 + 255) & ~(size_t)255;
 }
 
+// Split slots: per (token, head, split) an fp32 O row, m and l.
+static size_t split_bytes(int64_t B, int64_t S, int64_t H, int64_t D_v, int nsplit) {
+  return nsplit > 1 ? (size_t)B * S * H * nsplit * (size_t)(D_v + 2) * 4 : 0;
+}
+
 // MX shapes with the exact-dequantisation path (a bf16 kernel for d_qk / d_v)
 static bool mx_exact_shape(int64_t D_qk, int64_t D_v) {
   return (D_qk == 128 && (D_v == 64 || D_v == 128)) || (D_qk == 192 && D_v == 128) || (D_qk == 576 && D_v == 512);
@@ -469,6 +474,8 @@ static int sparse_mla_fwd_impl(const void *q, const void *kv, const int32_t *ind
   p.hpg = (int)(H / G);
   p.ntiles = (p.hpg + 31) / 32;
   p.sl2 = sm_scale * kLog2e;
+  p.nsplit = 1;
+  p.part_o = p.part_ml = nullptr;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool f8 = dtype == DSA_DTYPE_E4M3;
   DSA_REQUIRE(S_kv * G * D_qk * 2 <= (int64_t)kMaskedOff, "dsa_sparse_mla_fwd: kv rows of one batch exceed 4 GiB - 64 KiB");
@@ -494,7 +501,11 @@ static int sparse_mla_fwd_impl(const void *q, const void *kv, const int32_t *ind
     pe.kv_scale = nullptr;
     pe.gate = gate;
     pe.gate_run = 0;
-    if (wide_shape(D_qk, D_v)) rc = launch_fwd_wide(pe, D_qk, D_v, false, st, false, true);
+    if (wide_shape(D_qk, D_v)) {
+      const WideFwdPlan pl = wide_fwd_plan(B * S * G, p.hpg, D_v, topk, false);
+      rc = pl.nt > 0 ? launch_fwd_wide_bf16(pe, D_qk, D_v, pl.nt, true, st)
+                     : launch_fwd_wide(pe, D_qk, D_v, false, st, false, true);
+    }
     else if (D_qk == 128 && D_v == 64) rc = launch_fwd_t<128, 64, false, false, false, true>(pe, st);
     else if (D_qk == 128) rc = launch_fwd_t<128, 128, false, false, false, true>(pe, st);
     else rc = launch_fwd_t<192, 128, false, false, false, true>(pe, st);
@@ -531,7 +542,19 @@ static int sparse_mla_fwd_impl(const void *q, const void *kv, const int32_t *ind
     return set_error(DSA_ERR_UNSUPPORTED, "dsa_sparse_mla_fwd: no MXFP8 kernel for d_qk=%lld d_v=%lld",
                      (long long)D_qk, (long long)D_v);
   }
-  if (wide_shape(D_qk, D_v)) return launch_fwd_wide(p, D_qk, D_v, f8, st);
+  if (wide_shape(D_qk, D_v)) {
+    WideFwdPlan pl = wide_fwd_plan(B * S * G, p.hpg, D_v, topk, !f8);
+    const size_t need = split_bytes(B, S, H, D_v, pl.nsplit);
+    if (need != 0 && workspace != nullptr && workspace_bytes >= need) {
+      p.nsplit = pl.nsplit;
+      p.part_o = static_cast<float *>(workspace);
+      p.part_ml = p.part_o + (size_t)B * S * H * pl.nsplit * D_v;
+    } else if (need != 0) {
+      pl = wide_fwd_plan(B * S * G, p.hpg, D_v, topk, false);
+    }
+    return f8 || pl.nt == 0 ? launch_fwd_wide(p, D_qk, D_v, f8, st)
+                            : launch_fwd_wide_bf16(p, D_qk, D_v, pl.nt, false, st);
+  }
   if (D_qk == 128 && D_v == 64) return f8 ? launch_fwd<128, 64, true>(p, st) : launch_fwd<128, 64, false>(p, st);
   if (D_qk == 128 && D_v == 128) return f8 ? launch_fwd<128, 128, true>(p, st) : launch_fwd<128, 128, false>(p, st);
   if (D_qk == 192 && D_v == 128) return f8 ? launch_fwd<192, 128, true>(p, st) : launch_fwd<192, 128, false>(p, st);
@@ -559,6 +582,13 @@ extern "C" size_t dsa_sparse_mla_fwd_workspace_size(int64_t B, int64_t S_kv, int
   return v16_bytes(B, S_kv, G, D_v);
 }
 
+extern "C" size_t dsa_sparse_mla_fwd_call_workspace_size(int64_t B, int64_t S, int64_t S_kv, int64_t H, int64_t G,
+                                                         int64_t D_qk, int64_t D_v, int64_t topk, int dtype) {
+  if (dtype != DSA_DTYPE_BF16) return dsa_sparse_mla_fwd_workspace_size(B, S_kv, G, D_qk, D_v, dtype);
+  if (B <= 0 || S <= 0 || H <= 0 || G <= 0 || H % G != 0 || topk <= 0 || !wide_shape(D_qk, D_v)) return 0;
+  return split_bytes(B, S, H, D_v, wide_fwd_plan(B * S * G, H / G, D_v, topk, true).nsplit);
+}
+
 extern "C" int dsa_sparse_mla_fwd_ws(const void *q, const void *kv, const int32_t *indices, void *out,
                                      float *lse2, int64_t B, int64_t S, int64_t S_kv, int64_t H, int64_t G,
                                      int64_t D_qk, int64_t D_v, int64_t topk, float sm_scale, int dtype,
@@ -567,5 +597,5 @@ extern "C" int dsa_sparse_mla_fwd_ws(const void *q, const void *kv, const int32_
   const size_t need = dsa_sparse_mla_fwd_workspace_size(B, S_kv, G, D_qk, D_v, dtype);
   DSA_REQUIRE(need == 0 || workspace, "dsa_sparse_mla_fwd_ws: null workspace (%zu bytes required)", need);
   return sparse_mla_fwd_impl(q, kv, indices, out, lse2, B, S, S_kv, H, G, D_qk, D_v, topk, sm_scale, dtype, q_scale,
-                             kv_scale, need ? workspace : nullptr, workspace_bytes, stream);
+                             kv_scale, need || dtype == DSA_DTYPE_BF16 ? workspace : nullptr, workspace_bytes, stream);
 }

@@ -63,17 +63,18 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t slot_rsrc(const int32_t *row, 
 // Number of 32-slot blocks of this row up to its last valid slot (an index in
 // [0, s_kv)), 0 when it has none: every later block is wholly masked and
 // contributes nothing, so the block loops stop there.  One pass of unconditional
-// bounded loads over the row's indices, then a wave maximum (the same value in
-// every wave of a workgroup).
+// bounded loads over the row's indices, U in flight per lane, then a wave maximum
+// (the same value in every wave of a workgroup).
+template <int U = 4>
 __device__ __forceinline__ int valid_blocks(__amdgpu_buffer_rsrc_t idx_rs, int64_t topk, int64_t s_kv) {
   const int lane = lane_id();
   int last = -1;
-  for (int64_t s0 = 0; s0 < topk; s0 += 256) {
-    int raw[4];
+  for (int64_t s0 = 0; s0 < topk; s0 += 64 * U) {
+    int raw[U];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) raw[u] = (int)__builtin_amdgcn_raw_buffer_load_b32(idx_rs, (int)((s0 + 64 * u + lane) * 4), 0, 0);
+    for (int u = 0; u < U; ++u) raw[u] = (int)__builtin_amdgcn_raw_buffer_load_b32(idx_rs, (int)((s0 + 64 * u + lane) * 4), 0, 0);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int64_t s = s0 + 64 * u + lane;
       last = (s < topk && raw[u] >= 0 && raw[u] < s_kv && (int)s > last) ? (int)s : last;
     }

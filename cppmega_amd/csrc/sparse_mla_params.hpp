@@ -35,6 +35,10 @@ struct FwdParams {
   int hpg;     // heads per kv group
   int ntiles;  // ceil(hpg / 32)
   float sl2;   // sm_scale * log2(e)
+  // splits of an item's slots over workgroups (bf16 wide kernel): the splits' unnormalised O
+  // [token, kv group][split][head][d_v] and (m, l) [...][2], or 1 and null
+  int nsplit;
+  float *part_o, *part_ml;
 };
 
 struct BwdParams {

@@ -1,6 +1,10 @@
-// SparseMLA forward for wide heads on gfx950 (d_qk = 576 latent +
-// rope with d_v = 512: the DeepSeek-V3.2 MLA row and the reference's default
-// head dims; or d_v = 576, what a caller that passes no d_v gets).
+// SparseMLA forward for wide heads on gfx950 (d_qk = 576 latent + rope with
+// d_v = 512: the DeepSeek-V3.2 MLA row and the reference's default head dims; or
+// d_v = 576, what a caller that passes no d_v gets): e4m3 and MXFP8 rows, and
+// bf16 rows of kv groups of at most 32 heads.  With one head tile there is
+// little to share a row tile with, and this kernel's 57 KiB of LDS lets two
+// workgroups hide each other's waits: 601 us at s = 4096, 32 heads, top-k 1024,
+// against 885 us for the pipelined kernel that larger groups take.
 //
 // Reference semantics are those of the narrow kernel:
 // cppmega/megatron/sparse_mla_ops/tilelang_sparse_mla_fwd.py:137-290 and
@@ -340,12 +344,15 @@ static int launch_fwd_wide_nt(const FwdParams &p, hipStream_t st) {
   return check_launch("sparse_mla_fwd(wide)");
 }
 
-// Two head tiles per workgroup when a kv group has at least 64 heads (the
-// gather and dequantisation of a block serve both), else one.
+// e4m3: two head tiles per workgroup when a kv group has at least 64 heads (the
+// gather and dequantisation of a block serve both), else one.  bf16: one (the
+// host sends larger groups to launch_fwd_wide_bf16).
 template <int D_QK, int D_V, bool FP8, bool MX = false, bool QMX = false>
 static int launch_fwd_wide_t(const FwdParams &p, hipStream_t st) {
-  return p.ntiles >= 2 ? launch_fwd_wide_nt<D_QK, D_V, FP8, MX, 2, QMX>(p, st)
-                       : launch_fwd_wide_nt<D_QK, D_V, FP8, MX, 1, QMX>(p, st);
+  if constexpr (FP8) {
+    if (p.ntiles >= 2) return launch_fwd_wide_nt<D_QK, D_V, FP8, MX, 2, QMX>(p, st);
+  }
+  return launch_fwd_wide_nt<D_QK, D_V, FP8, MX, 1, QMX>(p, st);
 }
 
 int launch_fwd_wide(const FwdParams &p, int64_t d_qk, int64_t d_v, bool fp8, hipStream_t st, bool mx, bool qmx) {

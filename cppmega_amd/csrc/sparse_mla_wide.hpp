@@ -16,9 +16,18 @@ inline bool wide_shape(int64_t d_qk, int64_t d_v) { return d_qk == 576 && (d_v =
 // passes depend on it).
 inline bool wide_row(int64_t d_qk) { return d_qk == 576; }
 
-// Forward over all (token, kv group, 32-head tile) items; bf16 or e4m3.
-// mx: block-scaled e4m3 kernel; qmx: bf16 kernel with Q converted from e4m3
-// codes and 32-channel block scales as it is loaded
+// Forward of bf16 rows, pipelined: head tiles per workgroup (0: the kernel of
+// launch_fwd_wide instead) and splits of the slots, and the launch (p.nsplit > 1:
+// p.part_o / p.part_ml hold the splits' results); qmx: Q converted from e4m3
+// codes and 32-channel block scales as it is loaded.
+struct WideFwdPlan {
+  int nt, nsplit;
+};
+WideFwdPlan wide_fwd_plan(int64_t tgs, int64_t hpg, int64_t d_v, int64_t topk, bool may_split);
+int launch_fwd_wide_bf16(const FwdParams &p, int64_t d_qk, int64_t d_v, int nt, bool qmx, hipStream_t st);
+
+// Forward over all (token, kv group, 32-head tile) items: e4m3 rows (mx: with one
+// scale per 32 channels), or bf16 rows (qmx: as above).
 int launch_fwd_wide(const FwdParams &p, int64_t d_qk, int64_t d_v, bool fp8, hipStream_t st, bool mx = false,
                     bool qmx = false);
 // Backward main pass (P, dS and dQ, then the partial dKV rows at CSR positions); bf16 or e4m3.

@@ -126,11 +126,9 @@ sparse_mla_bwd_wide_scores_kernel(const BwdParams p) {
   const uint32_t k_lds = lds_address(K);
 
   const int mat = w / (2 * NT), kh = (w / NT) & 1, ht = w % NT;  // (see below)
-  int rc[T::PW];
-  dma_lane_map<T>(rc, w);
   // this wave's share of the rows of a block whose slot indices it holds
   auto fetch = [&](int tile, int idx) {
-    dma_tile_issue<T>(rc, k_lds + (uint32_t)(tile * T::BYTES), kv_rs, idx >= 0 ? (uint32_t)idx * row_pitch : kMaskedOff, w);
+    dma_tile_issue<T>(k_lds + (uint32_t)(tile * T::BYTES), kv_rs, idx >= 0 ? (uint32_t)idx * row_pitch : kMaskedOff, w);
   };
   const int idx0 = slot_index(load_slot_raw(idx_rs, 0, l32), 0, l32, p.topk, p.S_kv);
   int idx_nxt = slot_index(load_slot_raw(idx_rs, 1, l32), 1, l32, p.topk, p.S_kv);
@@ -160,16 +158,16 @@ sparse_mla_bwd_wide_scores_kernel(const BwdParams p) {
   const int eh = w >> 2, eq = w & 3;
   const float delta_h = LD[2 * (32 * eh + l32)], lse_h = LD[2 * (32 * eh + l32) + 1];
 
-  // S / dP operand of k-step 2 i + kh: row l32, chunk 2 (2 i + kh) + g32; i and i + 2 are 128 bytes apart
+  // S / dP operand of k-step 2 i + kh: row l32, chunk 2 (2 i + kh) + g32; i and i + 2 are a panel apart
   int ka[2];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) ka[u] = l32 * T::ROWB + (((2 * (2 * u + kh) + g32) ^ row_swz(l32)) * 16);
+  for (int u = 0; u < 2; ++u) ka[u] = tile_byte(l32, 2 * (2 * u + kh) + g32);
   // K^T of d tile w + NW i: rows 8 g16 + (lane % 16) / 4 (+ 4), columns 4 (lane % 4) .. of the tile
   int kt[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int row = 8 * g16 + 4 * u + (l16 >> 2), q = l16 & 3;
-    kt[u] = row * T::ROWB + (((2 * (w & 3) + (q >> 1)) ^ row_swz(row)) * 16) + (q & 1) * 8 + (w >> 2) * 128;
+    kt[u] = tile_byte(row, 2 * (w & 3) + (q >> 1)) + (q & 1) * 8 + (w >> 2) * T::PANEL;
   }
   // dS[head][slot]: 64-byte rows, 16-byte chunk c of head h at c ^ ((h >> 2) & 3)
   const int ds_rd = 2048 + l16 * 64 + ((g16 ^ ((l16 >> 2) & 3)) * 16);
@@ -196,8 +194,8 @@ sparse_mla_bwd_wide_scores_kernel(const BwdParams p) {
 #pragma unroll
     for (int i = 0; i < C::DTW; ++i) {
       if (C::NDT % C::NW == 0 || i + 1 < C::DTW || w < C::NDT % C::NW) {
-        const i32x2 r0 = ds_read_tr16(Kb + kt[0] + i * (C::NW / 4) * 128);
-        const i32x2 r1 = ds_read_tr16(Kb + kt[1] + i * (C::NW / 4) * 128);
+        const i32x2 r0 = ds_read_tr16(Kb + kt[0] + i * (C::NW / 4) * T::PANEL);
+        const i32x2 r1 = ds_read_tr16(Kb + kt[1] + i * (C::NW / 4) * T::PANEL);
         const i32x4 a = {r0[0], r0[1], r1[0], r1[1]};
 #pragma unroll
         for (int h = 0; h < 2 * NT; ++h) dq[i][h] = mfma_16x16x32(a, bs[h], dq[i][h]);
@@ -230,13 +228,13 @@ sparse_mla_bwd_wide_scores_kernel(const BwdParams p) {
     for (int a = 0; a < 16; ++a) acc[a] = 0.0f;
 #pragma unroll
     for (int i = 0; i < C::KSV; ++i) {
-      const i32x4 a = *reinterpret_cast<const i32x4 *>(Kj + ka[i & 1] + (i >> 1) * 128);
+      const i32x4 a = *reinterpret_cast<const i32x4 *>(Kj + ka[i & 1] + (i >> 1) * T::PANEL);
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(op[i]), acc, 0, 0, 0);
     }
     if (C::KSQ > C::KSV && mat == 0) {
 #pragma unroll
       for (int i = C::KSV; i < C::KSQ; ++i) {
-        const i32x4 a = *reinterpret_cast<const i32x4 *>(Kj + ka[i & 1] + (i >> 1) * 128);
+        const i32x4 a = *reinterpret_cast<const i32x4 *>(Kj + ka[i & 1] + (i >> 1) * T::PANEL);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(op[i]), acc, 0, 0, 0);
       }
     }

@@ -134,57 +134,58 @@ __device__ __forceinline__ void put_partial(float *dst, const f32x16 &acc) {
 // ---------------------------------------------------------------------------
 // Row tiles filled by LDS-DMA loads (bf16 rows)
 // ---------------------------------------------------------------------------
-// 32 gathered rows of D_QK bf16, unpadded, written straight into LDS by
+// 32 gathered rows of D_QK bf16, written straight into LDS by
 // buffer_load_dwordx4 ... lds: no staging registers and no LDS write
 // instructions.  One such load fills 1 KiB of consecutive LDS from 64 lanes'
-// own addresses, so the layout's swizzle is made by choosing which 16-byte
-// chunk each lane fetches: chunk c of row r sits at chunk c ^ row_swz(r).
-// A row is NCH chunks with NCH * 16 bytes an odd multiple of 128, so
-// consecutive rows start 128 bytes apart on the 256 bytes of banks; the swizzle
-// permutes the eight chunks of each 128-byte span such that
+// own addresses: here 8 rows x 128 bytes.  The tile is stored by panels of 128
+// bytes of d (64 columns), 32 rows each: chunk c (16 bytes) of row r at byte
+//   (c >> 3) * 4096 + r * 128 + ((c & 7) ^ row_swz(r)) * 16,
+// so a wave that fetches an 8-row group needs one source address per lane for
+// all of its panels (the panel is a scalar offset), and neither the rows' order
+// nor a lane's chunk changes between panels.  Rows are 128 bytes apart on the
+// 256 bytes of banks; the swizzle permutes the eight chunks such that
 //   * 16 consecutive rows read at one chunk (MFMA operand, lane = row) and
 //   * rows {8g .. 8g + 3} (or + 4 .. + 7) of two neighbouring g, read at one
 //     chunk pair (a transposed read)
 // fall on distinct banks.
 template <int D_QK, int NW_>
 struct DmaTile {
-  static constexpr int NW = NW_;                       // waves that fill it
+  static constexpr int NW = NW_;                       // waves that fill it (w < NW)
   static constexpr int ROWB = D_QK * 2;
-  static constexpr int NCH = ROWB / 16;                // 16-byte chunks per row
   static constexpr int BYTES = 32 * ROWB;
-  static constexpr int NP = BYTES / 1024;              // 1 KiB pieces (one load instruction each)
-  static constexpr int PW = (NP + NW - 1) / NW;        // pieces per wave: w, w + NW, ...
-  static constexpr int REM = NP % NW;                  // waves below it take PW pieces, the others PW - 1 (0: all PW)
-  static_assert(BYTES % 1024 == 0 && NCH % 8 == 0 && NP >= NW, "row tile in whole pieces");
+  static constexpr int PANELS = ROWB / 128, PANEL = 4096;
+  static constexpr int RG = 4 / NW;                    // 8-row groups per wave: w, w + NW, ...
+  static_assert(ROWB % 128 == 0 && 4 % NW == 0, "whole panels, whole row groups");
 };
 
 __device__ __forceinline__ int row_swz(int row) {
   const int x = (row >> 1) & 7;
   return ((x & 1) << 1) | (x & 4) | ((x >> 1) & 1);
 }
+// Byte of chunk c of row r within a tile (c < 8: an offset that (c >> 3) panels are added to).
+__device__ __forceinline__ int tile_byte(int r, int c) { return r * 128 + ((c ^ row_swz(r)) * 16); }
 
-// The (row, source byte) that this lane fetches in each of its wave's pieces,
-// packed (row << 16 | byte): constant over the blocks.
-template <class T>
-__device__ __forceinline__ void dma_lane_map(int (&rc)[T::PW], int w) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int i = 0; i < T::PW; ++i) {
-    const int u = 64 * (w + T::NW * i) + lane, row = u / T::NCH;  // (the row is < 32 for every piece that exists)
-    rc[i] = ((row & 31) << 16) | (((u - row * T::NCH) ^ row_swz(row)) * 16);
-  }
+// The lane index as a value the compiler cannot trace: addresses derived from
+// it are formed where they are used (a few VALU operations) instead of being
+// kept in registers across the block loop, where accumulators and operands leave none to spare.
+__device__ __forceinline__ int lane_here() {
+  int l = lane_id();
+  asm volatile("" : "+v"(l));
+  return l;
 }
 
-// Fetch the 32 rows at byte offsets my_off (held by lane `row`; kMaskedOff: the
-// row reads as zeros) into the tile at LDS byte address lds.
+// Fetch 32 rows at byte offsets my_off (held by lane `row`; kMaskedOff: the row
+// reads as zeros) into the tile at LDS byte address lds.
 template <class T>
-__device__ __forceinline__ void dma_tile_issue(const int (&rc)[T::PW], uint32_t lds, i32x4 rs, uint32_t my_off, int w) {
-  uint32_t src[T::PW];
+__device__ __forceinline__ void dma_tile_issue(uint32_t lds, i32x4 rs, uint32_t my_off, int w) {
+  const int lane = lane_here();
 #pragma unroll
-  for (int i = 0; i < T::PW; ++i) src[i] = (uint32_t)__shfl((int)my_off, rc[i] >> 16, 64) + (uint32_t)(rc[i] & 0xffff);
+  for (int i = 0; i < T::RG; ++i) {
+    const int rg = w + T::NW * i, row = 8 * rg + (lane >> 3);
+    const uint32_t src = (uint32_t)__shfl((int)my_off, row, 64) + (uint32_t)(((lane & 7) ^ row_swz(row)) * 16);
 #pragma unroll
-  for (int i = 0; i < T::PW; ++i)
-    if (i + 1 < T::PW || T::REM == 0 || w < T::REM) lds_dma_16(lds + (uint32_t)((w + T::NW * i) * 1024), src[i], rs);
+    for (int pn = 0; pn < T::PANELS; ++pn) lds_dma_16(lds + (uint32_t)(pn * T::PANEL + rg * 1024), src, rs, (uint32_t)(pn * 128));
+  }
 }
 
 }  // namespace dsa

@@ -26,8 +26,8 @@ def _launch_fwd(q, kv, indices, sm_scale, d_v, dtype_code, q_scale=None, kv_scal
     lse = torch.empty((B, S, H), dtype=torch.float32, device=q.device)
     _, stream = stream_of(q)
     L = _lib.load()
-    # e4m3: the V rows are dequantised to bf16 once per call into a workspace
-    ws_bytes = int(L.dsa_sparse_mla_fwd_workspace_size(B, S_kv, G, D, d_v, dtype_code))
+    # e4m3: the V rows dequantised to bf16 once per call; bf16, few tokens: the results of splits of the slots
+    ws_bytes = int(L.dsa_sparse_mla_fwd_call_workspace_size(B, S, S_kv, H, G, D, d_v, topk, dtype_code))
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device) if ws_bytes else None
     rc = L.dsa_sparse_mla_fwd_ws(
         q.data_ptr(), kv.data_ptr(), indices.data_ptr(), out.data_ptr(), lse.data_ptr(),

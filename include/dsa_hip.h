@@ -102,9 +102,17 @@ int dsa_sparse_mla_fwd(const void *q, const void *kv, const int32_t *indices,
  * V in LDS; MXFP8: B * S_kv * G * D_qk bf16 plus 256; bf16 input: 0, and then
  * `workspace` may be NULL).  Replaces the same reference interfaces as
  * dsa_sparse_mla_fwd.
+ * dsa_sparse_mla_fwd_call_workspace_size returns the bytes the whole call can
+ * use: the same for e4m3 and MXFP8; for bf16 input with too few tokens to fill
+ * the GPU, room for the results of several workgroups per (token, head) that
+ * share its slots.  Given a smaller workspace (or none), a bf16 call runs
+ * unsplit.
  */
 size_t dsa_sparse_mla_fwd_workspace_size(int64_t B, int64_t S_kv, int64_t G,
                                          int64_t D_qk, int64_t D_v, int dtype);
+size_t dsa_sparse_mla_fwd_call_workspace_size(int64_t B, int64_t S, int64_t S_kv,
+                                              int64_t H, int64_t G, int64_t D_qk,
+                                              int64_t D_v, int64_t topk, int dtype);
 int dsa_sparse_mla_fwd_ws(const void *q, const void *kv, const int32_t *indices,
                           void *out, float *lse2, int64_t B, int64_t S,
                           int64_t S_kv, int64_t H, int64_t G, int64_t D_qk,

@@ -61,3 +61,51 @@ def test_wide_rows_e4m3_two_rows_per_entry(dev):
     rdq, rdkv = orc.sparse_mla_bwd(q8, k8, out.cpu(), do, idx, lse.cpu(), D ** -0.5, DV, q_scale=qsv, kv_scale=ksv)
     assert_close(dq, rdq, what="dq")
     assert_close(dkv, rdkv, what="dkv")
+
+
+@pytest.mark.parametrize("B,S,S_kv,H,G,DV,topk", [
+    (2, 1, 3000, 128, 1, 512, 2048),     # 16 splits of one head tile each
+    (20, 1, 600, 128, 1, 512, 513),      # two head tiles, splits of uneven blocks
+    (3, 7, 500, 96, 1, 512, 300),        # two head tiles of three (the last workgroup's second is empty)
+    (1, 40, 700, 128, 1, 512, 600),      # four head tiles
+    (1, 2, 600, 64, 2, 576, 290),        # kv groups, V the whole row
+    (1, 70, 300, 128, 1, 512, 200),      # four head tiles, no split
+    (1, 40, 300, 100, 1, 576, 100),      # two head tiles of four, no split
+])
+def test_wide_forward_splits(dev, B, S, S_kv, H, G, DV, topk):
+    """Few tokens against a long kv: the slots of a token split over workgroups.
+    One token's slots all masked, one's valid slots in its first block only."""
+    g = torch.Generator().manual_seed(S_kv + topk)
+    q = (torch.randn((B, S, H, D), generator=g) * 0.5).to(torch.bfloat16)
+    kv = (torch.randn((B, S_kv, G, D), generator=g) * 0.5).to(torch.bfloat16)
+    idx = torch.rand((B, S, G, max(S_kv, topk)), generator=g).argsort(dim=-1)[..., :topk].to(torch.int32)
+    idx[idx >= S_kv] = -1
+    idx[0, -1, 0] = -1
+    idx[0, 0, -1, 9:] = -1
+    if B > 1:
+        idx[1, -1, 0, ::2] = -1
+    idx = idx.contiguous()
+    scale = D ** -0.5
+    out, lse = sparse_mla_fwd_interface(q.to(dev), kv.to(dev), idx.to(dev), sm_scale=scale, d_v=DV)
+    ro, rl = orc.sparse_mla_fwd(q, kv, idx, scale, DV)
+    assert_close(out, ro, what="out")
+    assert_close(lse, rl, what="lse2")
+
+
+def test_wide_forward_split_matches_unsplit(dev):
+    """A call given no workspace runs unsplit: the same result within rounding (bf16 out: 2^-8 of an element)."""
+    from cppmega_amd import _lib
+    B, S, S_kv, H, topk, DV = 4, 1, 2000, 128, 1024, 512
+    g = torch.Generator().manual_seed(3)
+    q = (torch.randn((B, S, H, D), generator=g) * 0.5).to(torch.bfloat16).to(dev)
+    kv = (torch.randn((B, S_kv, 1, D), generator=g) * 0.5).to(torch.bfloat16).to(dev)
+    idx = torch.rand((B, S, 1, S_kv), generator=g).argsort(dim=-1)[..., :topk].to(torch.int32).contiguous().to(dev)
+    L = _lib.load()
+    assert int(L.dsa_sparse_mla_fwd_call_workspace_size(B, S, S_kv, H, 1, D, DV, topk, _lib.DTYPE_BF16)) > 0
+    out, lse = sparse_mla_fwd_interface(q, kv, idx, sm_scale=D ** -0.5, d_v=DV)
+    out1, lse1 = torch.empty_like(out), torch.empty_like(lse)
+    _lib.check(L.dsa_sparse_mla_fwd(q.data_ptr(), kv.data_ptr(), idx.data_ptr(), out1.data_ptr(), lse1.data_ptr(), B, S,
+                                    S_kv, H, 1, D, DV, topk, D ** -0.5, _lib.DTYPE_BF16, None, None,
+                                    torch.cuda.current_stream().cuda_stream), "dsa_sparse_mla_fwd")
+    torch.testing.assert_close(out.float(), out1.float(), rtol=2 ** -7, atol=2 ** -7)
+    torch.testing.assert_close(lse, lse1, rtol=1e-5, atol=1e-4)
