@@ -65,6 +65,10 @@ EXPORTED_SYMBOLS = (
     "dsa_indexer_kl_loss_workspace_size",
     "dsa_indexer_kl_loss",
     "dsa_indexer_kl_loss_backward",
+    "dsa_indexer_kl_loss_state_size",
+    "dsa_indexer_kl_loss_with_grad_workspace_size",
+    "dsa_indexer_kl_loss_with_grad",
+    "dsa_indexer_kl_loss_grad_apply",
     "dsa_topk_index_mask",
     "dsa_stage_timing",
     "dsa_stage_times",
@@ -136,6 +140,13 @@ _SIGNATURES = {
     "dsa_indexer_kl_loss_backward": (_i32, [_c_void_p, _c_void_p, _i32, _i64, _c_void_p, _c_void_p, _c_void_p,
                                             _c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _i32,
                                             _c_void_p, _size_t, _c_void_p]),
+    "dsa_indexer_kl_loss_state_size": (_size_t, [_i64] * 5 + [_i32]),
+    "dsa_indexer_kl_loss_with_grad_workspace_size": (_size_t, [_i64] * 6 + [_i32]),
+    "dsa_indexer_kl_loss_with_grad": (_i32, [_c_void_p, _c_void_p, _i32, _i64, _c_void_p, _c_void_p, _c_void_p,
+                                             _c_void_p, _size_t, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _i32,
+                                             _c_void_p, _size_t, _c_void_p]),
+    "dsa_indexer_kl_loss_grad_apply": (_i32, [_c_void_p, _size_t, _c_void_p, _c_void_p] + [_i64] * 5
+                                       + [_f32, _i32, _c_void_p]),
     "dsa_topk_index_mask": (_i32, [_c_void_p, _i32, _i64, _c_void_p, _i64, _i64, _i64, _i64, _i64,
                                    _f32, _f32, _i32, _c_void_p]),
     "dsa_stage_timing": (_i32, [_i32]),

@@ -47,6 +47,17 @@
 // R per key chunk instead of the KL terms; then
 //  6. kl_grad_kernel         one workgroup per row: R in chunk order, then the
 //     whole row of the gradient in place over P (16-byte loads and stores).
+//
+// Loss and gradient together (dsa_indexer_kl_loss_with_grad, what autograd
+// takes): the gradient is linear in g, so one run of kernels 1-3 leaves the
+// loss and a state from which dsa_indexer_kl_loss_grad_apply forms the gradient
+// for any g.  Recomputing in the backward ran both q.k kernels twice (index
+// stats, statistics and pass again: 565 of the 1510 us of a sparse training step
+// at b = 2, s = 4096, 32 heads of 128).  The state holds
+//   v_s = Q_s * R - P_s * Q_s / (Q_s + 1e-10):
+// dense, every column (the size of the scores, which then need not be kept);
+// sparse, the columns of the row's top-k set only, in column order (v is 0
+// elsewhere), with the set's bitmask: 12 MB instead of 128 MiB at top-256.
 #include "dsa_common.hpp"
 
 namespace dsa {
@@ -84,8 +95,14 @@ struct Params {
   float *loss;                    // [1]
   float *partial_r;               // [B, NC, Sq]  gradient: R partial sums per key chunk
   float *grad;                    // [B, Sq, Sk]  gradient: P (pass kernel), then dL/dz
-  const float *grad_loss;         // [1]          upstream gradient of the loss
+  const float *grad_loss;         // [1]          upstream gradient of the loss (null: the state's v)
+  // sparse state: rows of the top-k set in column order
+  int32_t *cpre;                  // [B, Sq, NC + 2] set columns before each key chunk, all, and those at or below the diagonal
+  float *pc;                      // [B, Sq, K]   P, then v
+  float *xc;                      // [B, Sq, K]   index score
+  float *flag;                    // [B, Sq]      NaN for a row whose loss is NaN, else 0
   int64_t B, Sq, Sk, H, G, K, W, NC;
+  int KC;                         // keys per chunk
   int64_t NI;                     // KL work items per batch (block, chunk pairs)
   int topk_i64;
   int sparse;
@@ -121,13 +138,64 @@ __global__ void __launch_bounds__(kNT) kl_index_stats_kernel(Params p) {
       if (s >= 0 && s < p.Sk) atomicOr(&bw[s >> 5], 1u << (s & 31));
     }
     wave_lds_sync();
-    for (int i = lane; i < p.W; i += 64) {
-      uint32_t word = bw[i];
-      p.mask[row * p.W + i] = word;
-      while (word) {  // each set column once (duplicates in the top-k list count once)
-        const int bpos = __builtin_ctz(word);
-        word &= word - 1u;
-        lse_merge(m, d, I[i * 32 + bpos] * kLog2e, 1.0f);
+    const int64_t t = row % p.Sq, last_k = t < p.Sk - 1 ? t : p.Sk - 1;
+    const int wpc = p.KC / 32;  // words per key chunk
+    int32_t *pre = p.cpre != nullptr ? p.cpre + row * (p.NC + 2) : nullptr;
+    int before = 0, adm = 0;  // set columns in the earlier rounds' words; those at or below the diagonal
+    for (int i0 = 0; i0 < p.W; i0 += 64) {
+      const int i = i0 + lane;
+      const bool in = i < p.W;
+      uint32_t word = in ? bw[i] : 0u;
+      if (in) p.mask[row * p.W + i] = word;
+      int at = 0;
+      if (pre != nullptr) {  // rank of the word's first column, by a prefix sum over the lanes
+        const int n = __popc(word);
+        int x = n;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const int y = __shfl_up(x, off, 64);
+          if (lane >= off) x += y;
+        }
+        at = before + x - n;
+        before += __shfl(x, 63, 64);
+        if (in && i % wpc == 0) pre[i / wpc] = at;
+        const int64_t lb = last_k - (int64_t)i * 32;  // last admissible bit of the word
+        adm += __popc(lb >= 31 ? word : (lb < 0 ? 0u : word & ((2u << lb) - 1u)));
+      }
+      // each set column once (duplicates in the top-k list count once), four loads in flight
+      while (word) {
+        int bp[4];
+        float x[4];
+        int n = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          bp[u] = word ? __builtin_ctz(word) : 0;
+          n += word ? 1 : 0;
+          word &= word - 1u;  // (0 stays 0)
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = u < n ? I[i * 32 + bp[u]] : -INFINITY;
+        if (pre != nullptr) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (u < n) p.xc[row * p.K + at + u] = x[u];
+          at += n;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] *= kLog2e;
+        float nm = fmaxf(m, fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
+        d = d * exp2_fast(m - nm) + exp2_fast(x[0] - nm);
+#pragma unroll
+        for (int u = 1; u < 4; ++u) d += u < n ? exp2_fast(x[u] - nm) : 0.0f;
+        m = nm;
+      }
+    }
+    if (pre != nullptr) {
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) adm += __shfl_xor(adm, off, 64);
+      if (lane == 0) {
+        pre[p.NC] = before;
+        pre[p.NC + 1] = adm;
       }
     }
   } else {
@@ -350,7 +418,9 @@ kl_attn_stats_kernel(Params p) {
 // ---------------------------------------------------------------------------
 // 3. KL partial sums per (token, key chunk)
 // ---------------------------------------------------------------------------
-template <int D, int NW, bool GRAD = false>
+// LOSS: the KL partial sums; GRAD: P (p.grad, or the sparse state's p.pc) and the
+// R partial sums.
+template <int D, int NW, bool LOSS, bool GRAD>
 __global__ void __launch_bounds__(64 * NW) kl_pass_kernel(Params p) {
   using C = Cfg<D, NW>;
   constexpr int kTB = C::TB;
@@ -445,12 +515,17 @@ __global__ void __launch_bounds__(64 * NW) kl_pass_kernel(Params p) {
   const float *irow = p.index_scores + b * p.Sq * p.Sk;
   const auto irs = make_buffer_rsrc(irow, (uint32_t)(p.Sq * p.Sk * 4));
   const bool vec = (p.Sk & 3) == 0;  // rows 16-byte aligned: one b128 load per 4 keys
-  float kl = 0.0f;
-  float *grow = GRAD ? p.grad + (b * p.Sq + (t < p.Sq ? t : 0)) * p.Sk : nullptr;
+  float kl = 0.0f, rsum = 0.0f;
+  const int64_t row = b * p.Sq + (t < p.Sq ? t : 0);
+  const bool compact = GRAD && p.pc != nullptr;
+  float *grow = GRAD && !compact ? p.grad + row * p.Sk : nullptr;
+  float *crow = compact ? p.pc + row * p.K : nullptr;
+  int at = compact ? p.cpre[row * (p.NC + 2) + ci] : 0;  // rank of the sub-tile's first set column
 #pragma unroll
   for (int sub = 0; sub < C::SUBS; ++sub) {
     if (!sub_on[sub]) continue;
     const int64_t key0 = k0 + 32 * sub;
+    const uint32_t word = compact ? mask_word(p, b, t, key0) : 0u;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       // keys key0 + 8i + 4g + (0..3) of this lane's row; reads past the row
@@ -468,44 +543,39 @@ __global__ void __launch_bounds__(64 * NW) kl_pass_kernel(Params p) {
           iv[j] = buffer_load_f32(irs, (int)off, 0);
         }
       }
-      if constexpr (GRAD) {
-        // P on this lane's four keys (0 off the admissible set), and R's terms
-        f32x4 pv;
+      f32x4 pv;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int a = 4 * i + j;
-          const bool on = (vb[sub] >> a) & 1u;
-          const float pr = on ? P[sub][a] * inv_h : 0.0f;
+      for (int j = 0; j < 4; ++j) {
+        const int a = 4 * i + j;
+        const bool on = (vb[sub] >> a) & 1u;
+        const float pr = on ? P[sub][a] * inv_h : 0.0f;
+        pv[j] = pr;
+        if (on) {
           const float q = exp2_fast(fmaf(iv[j], kLog2e, -gam));
-          pv[j] = pr;
-          if (on) kl += pr * (q / (q + kEps));
-        }
-        if (t < p.Sq && s0 < p.Sk) {
-          if (vec) {
-            *reinterpret_cast<f32x4 *>(grow + s0) = pv;
-          } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              if (s0 + j < p.Sk) grow[s0 + j] = pv[j];
-          }
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int a = 4 * i + j;
-          if ((vb[sub] >> a) & 1u) {
-            const float pr = P[sub][a] * inv_h;
-            const float q = exp2_fast(fmaf(iv[j], kLog2e, -gam));
-            kl += pr * (__builtin_amdgcn_logf(pr + kEps) - __builtin_amdgcn_logf(q + kEps));
+          if constexpr (LOSS) kl += pr * (__builtin_amdgcn_logf(pr + kEps) - __builtin_amdgcn_logf(q + kEps));
+          if constexpr (GRAD) {
+            rsum += pr * (q / (q + kEps));
+            if (compact) crow[at + __popc(word & ((1u << (8 * i + 4 * g + j)) - 1u))] = pr;
           }
         }
       }
+      if (GRAD && !compact && t < p.Sq && s0 < p.Sk) {  // 0 off the admissible set
+        if (vec) {
+          *reinterpret_cast<f32x4 *>(grow + s0) = pv;
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (s0 + j < p.Sk) grow[s0 + j] = pv[j];
+        }
+      }
     }
+    at += __popc(word);
   }
   if constexpr (GRAD) {
-    kl = sum_halves(kl);
-    if (g == 0 && t < p.Sq) p.partial_r[(b * p.NC + ci) * p.Sq + t] = kl;
-  } else {
+    rsum = sum_halves(rsum);
+    if (g == 0 && t < p.Sq) p.partial_r[(b * p.NC + ci) * p.Sq + t] = rsum;
+  }
+  if constexpr (LOSS) {
     kl = sum_halves(kl) * kLn2;
     if (g == 0 && t < p.Sq) p.partial[(b * p.NC + ci) * p.Sq + t] = kl;
   }
@@ -541,7 +611,8 @@ __global__ void __launch_bounds__(kNT) kl_grad_kernel(Params p) {
   const bool no_target = !(p.beta[b * p.H * p.Sq + t] > -INFINITY);
   const float gam = p.gamma[row];
   const bool nan_row = no_target || gam != gam;
-  const float gs = p.grad_loss[0] * p.coeff / (float)(p.B * p.Sq);
+  // (no upstream gradient: v itself, to be scaled by kl_scale_kernel)
+  const float gs = p.grad_loss != nullptr ? p.grad_loss[0] * p.coeff / (float)(p.B * p.Sq) : 1.0f;
   const float *zrow = p.index_scores + row * p.Sk;
   float *grow = p.grad + row * p.Sk;
   const uint32_t *mrow = p.sparse ? p.mask + row * p.W : nullptr;
@@ -563,7 +634,86 @@ __global__ void __launch_bounds__(kNT) kl_grad_kernel(Params p) {
     for (int j = 0; j < 4; ++j) {
       const float q = ((mw >> j) & 1u) ? exp2_fast(fmaf(z[j], kLog2e, -gam)) : 0.0f;
       const float pj = s0 + j <= last_k ? pr[j] : 0.0f;
-      out[j] = nan_row ? __builtin_nanf("") : gs * (q * R - pj * (q / (q + kEps)));
+      out[j] = nan_row ? __builtin_nanf("") : gs * fmaf(q, R, -(pj * (q / (q + kEps))));
+    }
+    if (vec) {
+      *reinterpret_cast<f32x4 *>(grow + s0) = out;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (s0 + j < p.Sk) grow[s0 + j] = out[j];
+    }
+  }
+}
+
+// Sparse state: v over P in place, one wave per row, and the row's loss.
+template <int D>
+__global__ void __launch_bounds__(kNT) kl_rows_state_kernel(Params p) {
+  const int lane = lane_id();
+  const int64_t row = (int64_t)blockIdx.x * 4 + wave_id();
+  if (row >= p.B * p.Sq) return;  // wave-uniform
+  const int64_t b = row / p.Sq, t = row % p.Sq;
+  const int64_t last_k = t < p.Sk - 1 ? t : p.Sk - 1;
+  const int64_t cmax = last_k / Cfg<D, 4>::KC;
+  float kl = 0.0f, R = 0.0f;
+#pragma unroll 8
+  for (int64_t c = 0; c <= cmax; ++c) {  // in chunk order, the same in every lane
+    kl += p.partial[(b * p.NC + c) * p.Sq + t];
+    R += p.partial_r[(b * p.NC + c) * p.Sq + t];
+  }
+  const bool no_target = !(p.beta[b * p.H * p.Sq + t] > -INFINITY);
+  const float gam = p.gamma[row];
+  const bool nan_row = no_target || gam != gam;
+  if (lane == 0) {
+    p.rows[row] = nan_row ? __builtin_nanf("") : kl;
+    p.flag[row] = nan_row ? __builtin_nanf("") : 0.0f;
+  }
+  const int32_t *pre = p.cpre + row * (p.NC + 2);
+  const int n = pre[p.NC], adm = pre[p.NC + 1];
+  float *v = p.pc + row * p.K;
+  const float *x = p.xc + row * p.K;
+  for (int e = lane; e < n; e += 64) {
+    const float q = exp2_fast(fmaf(x[e], kLog2e, -gam));
+    const float pe = e < adm ? v[e] : 0.0f;  // columns past the diagonal have no target
+    v[e] = fmaf(q, R, -(pe * (q / (q + kEps))));
+  }
+}
+
+// The gradient from the state: g * coeff / (B * Sq) * v.
+__global__ void __launch_bounds__(kNT) kl_scale_kernel(const float *v, const float *grad_loss, float *out, int64_t n,
+                                                       float coeff, float denom) {
+  const float gs = grad_loss[0] * coeff / denom;
+  const int64_t i0 = ((int64_t)blockIdx.x * kNT + threadIdx.x) * 4, stride = (int64_t)gridDim.x * kNT * 4;
+  for (int64_t i = i0; i < n; i += stride) {
+    if (i + 4 <= n) {
+      *reinterpret_cast<f32x4 *>(out + i) = gs * *reinterpret_cast<const f32x4 *>(v + i);
+    } else {
+      for (int64_t j = i; j < n; ++j) out[j] = gs * v[j];
+    }
+  }
+}
+// Sparse: one workgroup per row writes every column; a set column's rank is the
+// columns before its chunk plus those before it in the chunk's words.
+__global__ void __launch_bounds__(kNT) kl_expand_kernel(Params p) {
+  const int64_t row = blockIdx.x;
+  const float gs = p.grad_loss[0] * p.coeff / (float)(p.B * p.Sq);
+  const float off = p.flag[row];  // 0, or NaN over the whole row
+  const uint32_t *mrow = p.mask + row * p.W;
+  const int32_t *pre = p.cpre + row * (p.NC + 2);
+  const float *v = p.pc + row * p.K;
+  float *grow = p.grad + row * p.Sk;
+  const bool vec = (p.Sk & 3) == 0;
+  const int wpc = p.KC / 32;
+  for (int64_t s0 = 4 * (int64_t)threadIdx.x; s0 < p.Sk; s0 += 4 * kNT) {
+    const int wi = (int)(s0 >> 5), sh = (int)(s0 & 31);
+    const uint32_t word = mrow[wi];
+    f32x4 out = {gs * off, gs * off, gs * off, gs * off};
+    if ((word >> sh) & 0xfu) {
+      int at = pre[wi / wpc] + __popc(word & ((1u << sh) - 1u));
+      for (int k = wi / wpc * wpc; k < wi; ++k) at += __popc(mrow[k]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if ((word >> (sh + j)) & 1u) out[j] = gs * (v[at++] + off);
     }
     if (vec) {
       *reinterpret_cast<f32x4 *>(grow + s0) = out;
@@ -593,13 +743,35 @@ __global__ void __launch_bounds__(1024) kl_mean_kernel(Params p) {
 // host
 // ---------------------------------------------------------------------------
 struct Layout {
-  size_t mask, gamma, beta, partial, rows, partial_r, total;
+  size_t mask, gamma, beta, partial, rows, partial_r, xc, total;
+};
+
+// State of dsa_indexer_kl_loss_with_grad: dense v [B, Sq, Sk]; sparse the bitmask,
+// the ranks, the row flags and v [B, Sq, K].
+struct State {
+  size_t v, mask, cpre, flag, total;
 };
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-static Layout layout(int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t D, int sparse) {
-  const int64_t KC = D <= 128 ? 128 : 64;
+static int64_t chunk_keys(int64_t D) { return D <= 128 ? 128 : 64; }
+
+static State state_layout(int64_t B, int64_t Sq, int64_t Sk, int64_t D, int64_t topk, int sparse) {
+  State S{};
+  size_t o = 0;
+  S.v = o;     o += align256((size_t)(B * Sq * (sparse ? topk : Sk)) * 4);
+  if (sparse) {
+    S.mask = o;  o += align256((size_t)(B * Sq * ((Sk + 31) / 32)) * 4);
+    S.cpre = o;  o += align256((size_t)(B * Sq * ((Sk + chunk_keys(D) - 1) / chunk_keys(D) + 2)) * 4);
+    S.flag = o;  o += align256((size_t)(B * Sq) * 4);
+  }
+  S.total = o;
+  return S;
+}
+
+// topk > 0: with the sparse state's index scores (its mask lies in the state)
+static Layout layout(int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t D, int sparse, int64_t topk = 0) {
+  const int64_t KC = chunk_keys(D);
   const int64_t W = (Sk + 31) / 32, NC = (Sk + KC - 1) / KC;
   Layout L;
   size_t o = 0;
@@ -609,11 +781,12 @@ static Layout layout(int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t D, in
   L.partial = o; o += align256((size_t)(B * NC * Sq) * 4);
   L.rows = o;    o += align256((size_t)(B * Sq) * 4);
   L.partial_r = o; o += align256((size_t)(B * NC * Sq) * 4);
+  L.xc = o;      o += align256(sparse ? (size_t)(B * Sq * topk) * 4 : 0);
   L.total = o;
   return L;
 }
 
-template <int D, int NWS, int NWP, bool GRAD>
+template <int D, int NWS, int NWP, bool LOSS, bool GRAD>
 static int launch_mfma(const Params &p, hipStream_t st) {
   using CS = Cfg<D, NWS>;
   using CP = Cfg<D, NWP>;
@@ -629,12 +802,17 @@ static int launch_mfma(const Params &p, hipStream_t st) {
     q.NI += (lt < p.Sk - 1 ? lt : p.Sk - 1) / CP::KC + 1;
   }
   const int64_t items = (p.B * q.NI + 7) / 8 * 8;
-  hipLaunchKernelGGL((kl_pass_kernel<D, NWP, GRAD>), dim3((unsigned)items), dim3(CP::NT), 0, st, q);
+  hipLaunchKernelGGL((kl_pass_kernel<D, NWP, LOSS, GRAD>), dim3((unsigned)items), dim3(CP::NT), 0, st, q);
   rc = check_launch("kl_pass_kernel");
   if (rc) return rc;
+  if (p.pc != nullptr) {
+    hipLaunchKernelGGL(kl_rows_state_kernel<D>, dim3((unsigned)((p.B * p.Sq + 3) / 4)), dim3(kNT), 0, st, p);
+    return check_launch("kl_rows_state_kernel");
+  }
   if constexpr (GRAD) {
     hipLaunchKernelGGL(kl_grad_kernel<D>, dim3((unsigned)(p.B * p.Sq)), dim3(kNT), 0, st, p);
-    return check_launch("kl_grad_kernel");
+    rc = check_launch("kl_grad_kernel");
+    if (rc || !LOSS) return rc;
   }
   hipLaunchKernelGGL(kl_rows_kernel<D>, dim3((unsigned)((p.B * p.Sq + kNT - 1) / kNT)), dim3(kNT), 0, st, p);
   return check_launch("kl_rows_kernel");
@@ -644,7 +822,7 @@ static int launch_mfma(const Params &p, hipStream_t st) {
 static int kl_setup(const char *fn, const float *index_scores, const void *topk_indices, int topk_dtype,
                     int64_t topk, const void *query, const void *key, int64_t B, int64_t Sq, int64_t Sk,
                     int64_t H, int64_t G, int64_t D, float softmax_scale, float loss_coeff, int sparse,
-                    void *workspace, size_t workspace_bytes, Params &p) {
+                    void *workspace, size_t workspace_bytes, Params &p, bool state = false) {
   DSA_REQUIRE(index_scores && query && key, "%s: null pointer", fn);
   DSA_REQUIRE(B > 0 && Sq > 0 && Sk > 0 && H > 0 && G > 0, "%s: empty shape B=%lld Sq=%lld Sk=%lld H=%lld G=%lld",
               fn, (long long)B, (long long)Sq, (long long)Sk, (long long)H, (long long)G);
@@ -662,7 +840,7 @@ static int kl_setup(const char *fn, const float *index_scores, const void *topk_
                 fn, topk_dtype);
     DSA_REQUIRE(Sk <= 32 * kMaxW, "%s: sparse mode supports Sk <= %d (got %lld)", fn, 32 * kMaxW, (long long)Sk);
   }
-  const Layout L = layout(B, Sq, Sk, H, D, sparse);
+  const Layout L = layout(B, Sq, Sk, H, D, sparse, state ? topk : 0);
   if (!workspace || workspace_bytes < L.total)
     return set_error(DSA_ERR_WORKSPACE, "%s: workspace %zu bytes < %zu required", fn,
                      workspace ? workspace_bytes : (size_t)0, L.total);
@@ -680,7 +858,9 @@ static int kl_setup(const char *fn, const float *index_scores, const void *topk_
   p.partial_r = reinterpret_cast<float *>(ws + L.partial_r);
   p.B = B; p.Sq = Sq; p.Sk = Sk; p.H = H; p.G = G; p.K = sparse ? topk : 0;
   p.W = (Sk + 31) / 32;
-  p.NC = (Sk + (D <= 128 ? 128 : 64) - 1) / (D <= 128 ? 128 : 64);
+  p.KC = (int)chunk_keys(D);
+  p.NC = (Sk + p.KC - 1) / p.KC;
+  p.xc = reinterpret_cast<float *>(ws + L.xc);
   p.topk_i64 = topk_dtype == DSA_DTYPE_I64;
   p.sparse = sparse ? 1 : 0;
   p.c = softmax_scale * kLog2e;
@@ -688,16 +868,16 @@ static int kl_setup(const char *fn, const float *index_scores, const void *topk_
   return DSA_OK;
 }
 
-template <bool GRAD>
+template <bool LOSS, bool GRAD>
 static int kl_launch(const Params &p, int64_t D, hipStream_t st) {
   hipLaunchKernelGGL(kl_index_stats_kernel, dim3((unsigned)((p.B * p.Sq + 3) / 4)), dim3(kNT), 0, st, p);
   int rc = check_launch("kl_index_stats_kernel");
   if (rc) return rc;
   switch (D) {
-    case 64: return launch_mfma<64, 8, 4, GRAD>(p, st);
-    case 128: return launch_mfma<128, 8, 4, GRAD>(p, st);
-    case 192: return launch_mfma<192, 8, 4, GRAD>(p, st);
-    default: return launch_mfma<256, 8, 4, GRAD>(p, st);
+    case 64: return launch_mfma<64, 8, 4, LOSS, GRAD>(p, st);
+    case 128: return launch_mfma<128, 8, 4, LOSS, GRAD>(p, st);
+    case 192: return launch_mfma<192, 8, 4, LOSS, GRAD>(p, st);
+    default: return launch_mfma<256, 8, 4, LOSS, GRAD>(p, st);
   }
 }
 
@@ -725,7 +905,7 @@ extern "C" int dsa_indexer_kl_loss(const float *index_scores, const void *topk_i
   if (row_loss) p.rows = row_loss;
   p.loss = loss;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  rc = kl_launch<false>(p, D, st);
+  rc = kl_launch<true, false>(p, D, st);
   if (rc) return rc;
   hipLaunchKernelGGL(kl_mean_kernel, dim3(1), dim3(1024), 0, st, p);
   return check_launch("kl_mean_kernel");
@@ -747,5 +927,84 @@ extern "C" int dsa_indexer_kl_loss_backward(const float *index_scores, const voi
   if (rc) return rc;
   p.grad = grad_index_scores;
   p.grad_loss = grad_loss;
-  return kl_launch<true>(p, D, static_cast<hipStream_t>(stream));
+  return kl_launch<false, true>(p, D, static_cast<hipStream_t>(stream));
+}
+
+extern "C" size_t dsa_indexer_kl_loss_state_size(int64_t B, int64_t Sq, int64_t Sk, int64_t D, int64_t topk, int sparse) {
+  if (B <= 0 || Sq <= 0 || Sk <= 0 || D <= 0 || (sparse && topk <= 0)) return 0;
+  return dsa::kl::state_layout(B, Sq, Sk, D, topk, sparse).total;
+}
+
+extern "C" size_t dsa_indexer_kl_loss_with_grad_workspace_size(int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t D,
+                                                                int64_t topk, int sparse) {
+  if (B <= 0 || Sq <= 0 || Sk <= 0 || H <= 0 || D <= 0 || (sparse && topk <= 0)) return 0;
+  return dsa::kl::layout(B, Sq, Sk, H, D, sparse, sparse ? topk : 0).total;
+}
+
+static void kl_bind_state(dsa::kl::Params &p, void *state, const dsa::kl::State &S) {
+  unsigned char *s = static_cast<unsigned char *>(state);
+  if (!p.sparse) return;
+  p.pc = reinterpret_cast<float *>(s + S.v);
+  p.mask = reinterpret_cast<uint32_t *>(s + S.mask);
+  p.cpre = reinterpret_cast<int32_t *>(s + S.cpre);
+  p.flag = reinterpret_cast<float *>(s + S.flag);
+}
+
+extern "C" int dsa_indexer_kl_loss_with_grad(const float *index_scores, const void *topk_indices, int topk_dtype,
+                                             int64_t topk, const void *query, const void *key, float *loss, void *state,
+                                             size_t state_bytes, int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t G,
+                                             int64_t D, float softmax_scale, float loss_coeff, int sparse,
+                                             void *workspace, size_t workspace_bytes, void *stream) {
+  using namespace dsa;
+  using namespace dsa::kl;
+  DSA_REQUIRE(loss, "dsa_indexer_kl_loss_with_grad: null loss pointer");
+  Params p;
+  int rc = kl_setup("dsa_indexer_kl_loss_with_grad", index_scores, topk_indices, topk_dtype, topk, query, key, B, Sq, Sk,
+                    H, G, D, softmax_scale, loss_coeff, sparse, workspace, workspace_bytes, p, true);
+  if (rc) return rc;
+  const State S = state_layout(B, Sq, Sk, D, topk, sparse);
+  if (!state || state_bytes < S.total)
+    return set_error(DSA_ERR_WORKSPACE, "dsa_indexer_kl_loss_with_grad: state %zu bytes < %zu required",
+                     state ? state_bytes : (size_t)0, S.total);
+  kl_bind_state(p, state, S);
+  if (!p.sparse) p.grad = static_cast<float *>(state);
+  p.loss = loss;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  rc = kl_launch<true, true>(p, D, st);
+  if (rc) return rc;
+  hipLaunchKernelGGL(kl_mean_kernel, dim3(1), dim3(1024), 0, st, p);
+  return check_launch("kl_mean_kernel");
+}
+
+extern "C" int dsa_indexer_kl_loss_grad_apply(const void *state, size_t state_bytes, const float *grad_loss,
+                                              float *grad_index_scores, int64_t B, int64_t Sq, int64_t Sk, int64_t D,
+                                              int64_t topk, float loss_coeff, int sparse, void *stream) {
+  using namespace dsa;
+  using namespace dsa::kl;
+  const char *fn = "dsa_indexer_kl_loss_grad_apply";
+  DSA_REQUIRE(grad_loss && grad_index_scores, "%s: null gradient pointer", fn);
+  DSA_REQUIRE(B > 0 && Sq > 0 && Sk > 0 && D > 0 && (!sparse || topk > 0), "%s: empty shape", fn);
+  DSA_REQUIRE(B * Sq * Sk < ((int64_t)1 << 29), "%s: B*Sq*Sk=%lld index scores exceed 2 GiB", fn, (long long)(B * Sq * Sk));
+  const State S = state_layout(B, Sq, Sk, D, topk, sparse);
+  if (!state || state_bytes < S.total)
+    return set_error(DSA_ERR_WORKSPACE, "%s: state %zu bytes < %zu required", fn, state ? state_bytes : (size_t)0, S.total);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (!sparse) {
+    const int64_t n = B * Sq * Sk, blocks = (n / 4 + kNT) / kNT;
+    hipLaunchKernelGGL(kl_scale_kernel, dim3((unsigned)(blocks < 16384 ? blocks : 16384)), dim3(kNT), 0, st,
+                       static_cast<const float *>(state), grad_loss, grad_index_scores, n, loss_coeff, (float)(B * Sq));
+    return check_launch("kl_scale_kernel");
+  }
+  Params p{};
+  p.sparse = 1;
+  kl_bind_state(p, const_cast<void *>(state), S);
+  p.grad = grad_index_scores;
+  p.grad_loss = grad_loss;
+  p.coeff = loss_coeff;
+  p.B = B; p.Sq = Sq; p.Sk = Sk; p.K = topk;
+  p.W = (Sk + 31) / 32;
+  p.KC = (int)chunk_keys(D);
+  p.NC = (Sk + p.KC - 1) / p.KC;
+  hipLaunchKernelGGL(kl_expand_kernel, dim3((unsigned)(B * Sq)), dim3(kNT), 0, st, p);
+  return check_launch("kl_expand_kernel");
 }

@@ -14,10 +14,11 @@ Like the reference's Triton kernels, the [b, np, sq, sk] probabilities are
 never materialised.  The reference's scalar carries no autograd history; here,
 when ``index_scores`` requires grad, the loss is differentiable with respect to
 it as Megatron's ``compute_dsa_indexer_loss`` is (the indexer's only gradient):
-``indexer_kl_loss_backward`` recomputes P and writes
 dL/dz = g * coeff / (b * sq) * (Q * R - P * Q / (Q + 1e-10)),
 R = sum_j P_j Q_j / (Q_j + 1e-10), on the GPU (query and key get no gradient:
-P is the detached target, as in Megatron).
+P is the detached target, as in Megatron).  The forward forms it up to g beside
+the loss; ``indexer_kl_loss_backward`` recomputes P for a caller that kept
+only the scores.
 
 ``pg_collection`` is accepted for signature compatibility and, as in the
 reference, not used: with tensor-parallel heads the caller must combine the
@@ -108,22 +109,43 @@ def indexer_kl_loss_backward(grad_loss, index_scores, topk_indices, query, key, 
 
 
 class _IndexerKLLoss(torch.autograd.Function):
-    """Scalar KL loss, differentiable with respect to index_scores only."""
+    """Scalar KL loss, differentiable with respect to index_scores only.  The
+    forward leaves the gradient up to the upstream factor (dense: the size of
+    the scores; sparse: the top-k columns); the backward scales and expands it."""
 
     @staticmethod
     def forward(ctx, index_scores, topk_indices, query, key, softmax_scale, loss_coeff, sparse_loss):
-        loss, _ = _forward(index_scores, topk_indices, query, key, softmax_scale, loss_coeff, sparse_loss, False)
-        ctx.save_for_backward(index_scores, topk_indices if sparse_loss else None, query, key)
-        ctx.args = (softmax_scale, loss_coeff, sparse_loss)
+        scores, topk_indices, tdt, topk, query, key, sparse, (b, sq, sk, np_, g, hn) = _prepare(
+            index_scores, topk_indices, query, key, sparse_loss)
+        dev = _lib.ensure_device(query)
+        lib = _lib.load()
+        sp = 1 if sparse else 0
+        ws = torch.empty(max(int(lib.dsa_indexer_kl_loss_with_grad_workspace_size(b, sq, sk, np_, hn, topk, sp)), 1),
+                         dtype=torch.uint8, device=query.device)
+        state = torch.empty(max(int(lib.dsa_indexer_kl_loss_state_size(b, sq, sk, hn, topk, sp)), 1),
+                            dtype=torch.uint8, device=query.device)
+        loss = torch.empty((), dtype=torch.float32, device=query.device)
+        rc = lib.dsa_indexer_kl_loss_with_grad(
+            scores.data_ptr(), _lib.ptr(topk_indices), tdt, topk, query.data_ptr(), key.data_ptr(), loss.data_ptr(),
+            state.data_ptr(), state.numel(), b, sq, sk, np_, g, hn, float(softmax_scale), float(loss_coeff), sp,
+            ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
+        _lib.check(rc, "dsa_indexer_kl_loss_with_grad")
+        ctx.save_for_backward(state)
+        ctx.args = (b, sq, sk, hn, topk, float(loss_coeff), sp, index_scores.dtype)
         return loss
 
     @staticmethod
     def backward(ctx, grad_loss):
-        index_scores, topk_indices, query, key = ctx.saved_tensors
-        softmax_scale, loss_coeff, sparse_loss = ctx.args
-        grad = indexer_kl_loss_backward(grad_loss, index_scores, topk_indices, query, key, softmax_scale, loss_coeff,
-                                        sparse_loss)
-        return grad.to(index_scores.dtype), None, None, None, None, None, None
+        state, = ctx.saved_tensors
+        b, sq, sk, hn, topk, coeff, sp, dtype = ctx.args
+        dev = _lib.ensure_device(state)
+        gl = grad_loss.to(torch.float32).reshape(1).contiguous()
+        grad = torch.empty((b, sq, sk), dtype=torch.float32, device=state.device)
+        rc = _lib.load().dsa_indexer_kl_loss_grad_apply(
+            state.data_ptr(), state.numel(), gl.data_ptr(), grad.data_ptr(), b, sq, sk, hn, topk, coeff, sp,
+            _lib.stream_ptr(dev))
+        _lib.check(rc, "dsa_indexer_kl_loss_grad_apply")
+        return grad.to(dtype), None, None, None, None, None, None
 
 
 def indexer_kl_loss(index_scores, topk_indices, query, key, softmax_scale, loss_coeff=1.0, sparse_loss=False,

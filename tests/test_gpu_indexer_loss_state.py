@@ -1,0 +1,41 @@
+"""The KL loss's saved gradient state (autograd path) against the recomputing
+gradient call, bit for bit: top-k lists unsorted, padded, repeated, beyond the
+diagonal; chunk and word edges; rows without a target; several upstream factors."""
+import pytest
+import torch
+
+from cppmega_amd import indexer_kl_loss, indexer_kl_loss_backward
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sparse", [False, True], ids=["dense", "sparse"])
+@pytest.mark.parametrize("b,sq,sk,np_,hn,topk", [
+    (2, 130, 130, 4, 64, 40),     # a chunk edge at 128 keys
+    (1, 33, 2081, 2, 128, 70),    # more than 64 mask words, a ragged last word, keys beyond every diagonal
+    (1, 97, 63, 2, 192, 63),      # chunks of 64 keys, rows past the last key
+    (1, 20, 20, 1, 64, 1),
+])
+def test_state_gradient_matches_direct(dev, b, sq, sk, np_, hn, topk, sparse):
+    g = torch.Generator().manual_seed(sq * sk + topk)
+    z = torch.randn((b, sq, sk), generator=g)
+    idx = torch.rand((b, sq, max(sk, topk)), generator=g).argsort(dim=-1)[..., :topk]
+    idx = torch.where(torch.rand(idx.shape, generator=g) < 0.2, torch.full_like(idx, -1), idx)
+    if topk > 4:
+        idx[:, :, 3] = idx[:, :, 1]                       # repeats
+    idx[0, sq // 2] = -1                                  # no column: a NaN row (sparse)
+    z[0, 0, sk // 2] = -torch.inf
+    query = torch.randn((sq, b, np_, hn), generator=g).to(torch.bfloat16).to(dev)
+    key = torch.randn((sk, b, np_, hn), generator=g).to(torch.bfloat16).to(dev)
+    idx, scale = idx.to(dev), hn ** -0.5
+    zr = z.to(dev).requires_grad_()
+    loss = indexer_kl_loss(zr, idx, query, key, scale, 0.7, sparse)
+    with torch.no_grad():
+        plain, rows = indexer_kl_loss(zr.detach(), idx, query, key, scale, 0.7, sparse, return_rows=True)
+    assert torch.equal(loss.detach().isnan(), plain.isnan()) and (plain.isnan() or loss.detach() == plain)
+    assert bool(rows.isnan().any()) == sparse
+    for f in (1.0, -3.25):
+        got, = torch.autograd.grad(loss, zr, torch.tensor(f, device=dev), retain_graph=True)
+        want = indexer_kl_loss_backward(torch.tensor(f, device=dev), zr.detach(), idx, query, key, scale, 0.7, sparse)
+        assert torch.equal(got.isnan(), want.isnan())
+        assert torch.equal(got.nan_to_num(), want.nan_to_num())
