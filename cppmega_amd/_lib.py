@@ -143,7 +143,7 @@ _SIGNATURES = {
     "dsa_indexer_kl_loss_state_size": (_size_t, [_i64] * 5 + [_i32]),
     "dsa_indexer_kl_loss_with_grad_workspace_size": (_size_t, [_i64] * 6 + [_i32]),
     "dsa_indexer_kl_loss_with_grad": (_i32, [_c_void_p, _c_void_p, _i32, _i64, _c_void_p, _c_void_p, _c_void_p,
-                                             _c_void_p, _size_t, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _i32,
+                                             _c_void_p, _c_void_p, _size_t, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _i32,
                                              _c_void_p, _size_t, _c_void_p]),
     "dsa_indexer_kl_loss_grad_apply": (_i32, [_c_void_p, _size_t, _c_void_p, _c_void_p] + [_i64] * 5
                                        + [_f32, _i32, _c_void_p]),

@@ -25,7 +25,7 @@
 //     holds 16 keys of one token and row reductions stay in-lane); key chunks
 //     are double-buffered in LDS and shared by the 8 waves; a long and a short
 //     token block share one workgroup so every workgroup does equal work;
-//  3. kl_pass_kernel         per (b, 128-token block, key chunk): for every head
+//  3. kl_pass_kernel         per (b, 256-token block, key chunk): for every head
 //     recompute c * q.k, accumulate exp2(c * q.k - beta_h) in registers (the
 //     head sum of P), then form the KL terms of the chunk against
 //     Q = exp2(index * log2(e) - gamma) and write one partial sum per token;
@@ -88,6 +88,7 @@ struct Params {
   const unsigned char *query;     // [Sq, B, H, D] bf16
   const unsigned char *key;       // [Sk, B, G, D] bf16
   uint32_t *mask;                 // [B, Sq, W]   top-k bitmask (sparse only)
+  uint64_t *tiles;                // [B, ceil(Sq / 32), W, 16] lane masks of the admissible set (sparse only)
   float *gamma;                   // [B, Sq]      index normaliser (log2 units)
   float *beta;                    // [B, H, Sq]   attention normaliser (log2 units)
   float *partial;                 // [B, NC, Sq]  KL partial sums per key chunk
@@ -325,11 +326,50 @@ __device__ __forceinline__ float keep_or_neginf(float acc, uint32_t vb, int a) {
   return __uint_as_float((m & __float_as_uint(acc)) | (~m & 0xff800000u));
 }
 
+// One v_max3_f32 (a NaN operand is dropped, as fmaxf drops it; its exp2 term
+// still joins the sum).  Not for accumulators straight from an MFMA: the wait
+// that their first VALU read needs is inserted for instructions the compiler
+// knows, not for asm.
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
 // Chunks of KC keys that token block blk (TB tokens) needs: keys up to
 // min(last token of the block, Sk - 1).
 __device__ __forceinline__ int64_t block_chunks(const Params &p, int64_t blk, int64_t TB, int64_t KC) {
   const int64_t lt = (TB * (blk + 1) < p.Sq ? TB * (blk + 1) : p.Sq) - 1;
   return (lt < p.Sk - 1 ? lt : p.Sk - 1) / KC + 1;
+}
+
+// Lane masks of the admissible set (sparse): for 32 tokens and 32 keys, word
+// a = 4 i + j holds at bit (32 g + token) whether key 8 i + 4 g + j is in the
+// token's top-k set at or below its diagonal: the select operand, straight from
+// scalar registers, of accumulator register a in kl_attn_stats_kernel.  One
+// transposition serves every head; forming the selects per head from the row
+// bitmask took two VALU operations an element there (with it 229 -> 192 us at
+// b = 2, s = 4096, 32 heads of 128).  A workgroup takes a (b, 32-token block) and
+// every gridDim.y-th group of four words at or below the diagonal.
+__global__ void __launch_bounds__(kNT) kl_mask_tiles_kernel(Params p) {
+  const int lane = lane_id(), g = lane >> 5, l32 = lane & 31;
+  const int64_t NTB = (p.Sq + 31) / 32;
+  const int64_t tb = blockIdx.x % NTB, b = blockIdx.x / NTB, t = tb * 32 + l32;
+  const int64_t last_t = tb * 32 + 31 < p.Sk - 1 ? tb * 32 + 31 : p.Sk - 1;
+  uint64_t *tiles = p.tiles + (b * NTB + tb) * p.W * 16;
+  for (int64_t wi = blockIdx.y * (kNT / 64) + wave_id(); wi <= last_t / 32; wi += gridDim.y * (kNT / 64)) {
+    const int64_t last = (t < p.Sk - 1 ? t : p.Sk - 1) - wi * 32;
+    uint32_t word = t < p.Sq ? p.mask[(b * p.Sq + t) * p.W + wi] : 0u;
+    word = last < 0 ? 0u : (last >= 31 ? word : word & ((2u << last) - 1u));
+    word >>= 4 * g;
+    uint64_t mine = 0;
+#pragma unroll
+    for (int a = 0; a < 16; ++a) {
+      const uint64_t m = __ballot((word >> (8 * (a >> 2) + (a & 3))) & 1u);
+      if (lane == a) mine = m;
+    }
+    if (lane < 16) tiles[wi * 16 + lane] = mine;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -363,36 +403,43 @@ kl_attn_stats_kernel(Params p) {
     ld.load(p, b, grp, 0, kr);
     ChunkLoader<D, NW>::store(KS[0], kr);
     __syncthreads();
-    // sparse: the chunk's top-k mask words are loaded one chunk ahead
-    uint32_t mw[C::SUBS];
-#pragma unroll
-    for (int sub = 0; sub < C::SUBS; ++sub) mw[sub] = mask_word(p, b, t, 32 * sub);
+    // sparse: the wave's lane masks (scalar loads; the tile of 32 keys is 16 words)
+    typedef const __attribute__((address_space(4))) uint64_t *scalar_u64;
+    const scalar_u64 tiles =
+        p.sparse && wt0 < p.Sq ? (scalar_u64)(uintptr_t)(p.tiles + (b * ((p.Sq + 31) / 32) + wt0 / 32) * p.W * 16) : nullptr;
     for (int ci = 0; ci < nch; ++ci) {
       if (ci + 1 < nch) ld.load(p, b, grp, (int64_t)(ci + 1) * C::KC, kr);
-      uint32_t mwn[C::SUBS];
-#pragma unroll
-      for (int sub = 0; sub < C::SUBS; ++sub)
-        mwn[sub] = ci + 1 < nch ? mask_word(p, b, t, (int64_t)(ci + 1) * C::KC + 32 * sub) : 0u;
       const unsigned char *ks = KS[ci & 1];
 #pragma unroll
       for (int sub = 0; sub < C::SUBS; ++sub) {
         const int64_t key0 = (int64_t)ci * C::KC + 32 * sub;
-        if (key0 > wt_last || key0 >= p.Sk) continue;  // wave-uniform: wholly above the diagonal
+        if (key0 > wt_last || key0 >= p.Sk || wt0 >= p.Sq) continue;  // wave-uniform: wholly above the diagonal
         const f32x16 acc = qk_subtile<D>(ks, sub, Q);
-        const bool need_mask = p.sparse || key0 + 31 > wt0 || key0 + 31 >= p.Sk || wt_last >= p.Sq;
         // c > 0: max(c * acc) = c * max(acc), and exp2(c * acc - nm) is one fma
-        float x[16];
-        if (need_mask) {
-          const uint32_t vb = valid_bits(p, mw[sub], t, key0);
+        float x[16], lm;
+        if (p.sparse) {
+#pragma unroll
+          for (int a = 0; a < 16; ++a) {
+            const uint64_t m = tiles[(key0 >> 5) * 16 + a];
+            x[a] = __builtin_amdgcn_inverse_ballot_w64(m) ? acc[a] : -INFINITY;
+          }
+          lm = x[0];
+#pragma unroll
+          for (int a = 1; a < 15; a += 2) lm = max3(lm, x[a], x[a + 1]);
+          lm = max3(lm, x[15], x[15]);
+        } else if (key0 + 31 > wt0 || key0 + 31 >= p.Sk || wt_last >= p.Sq) {
+          const uint32_t vb = valid_bits(p, 0xffffffffu, t, key0);
 #pragma unroll
           for (int a = 0; a < 16; ++a) x[a] = keep_or_neginf(acc[a], vb, a);
         } else {
 #pragma unroll
           for (int a = 0; a < 16; ++a) x[a] = acc[a];
         }
-        float lm = x[0];
+        if (!p.sparse) {
+          lm = x[0];
 #pragma unroll
-        for (int a = 1; a < 16; ++a) lm = fmaxf(lm, x[a]);
+          for (int a = 1; a < 16; ++a) lm = fmaxf(lm, x[a]);
+        }
         const float nm = fmaxf(m, lm * p.c);
         float s = 0.0f;
 #pragma unroll
@@ -400,8 +447,6 @@ kl_attn_stats_kernel(Params p) {
         d = d * exp2_fast(m - nm) + s;
         m = nm;
       }
-#pragma unroll
-      for (int sub = 0; sub < C::SUBS; ++sub) mw[sub] = mwn[sub];
       if (ci + 1 < nch) {
         ChunkLoader<D, NW>::store(KS[(ci + 1) & 1], kr);
         __syncthreads();
@@ -418,13 +463,40 @@ kl_attn_stats_kernel(Params p) {
 // ---------------------------------------------------------------------------
 // 3. KL partial sums per (token, key chunk)
 // ---------------------------------------------------------------------------
+// The work per (head, token, key) is one fma, one exp2 (quarter rate) and one
+// add beside the products: 384 VALU cycles per 32x32 tile against 256 of MFMA at
+// D = 128, so the loop is built to keep the VALU fed: the head's q and k reach
+// LDS by coalesced LDS-DMA loads a head ahead (read as operands straight from
+// global, q's 32 rows of 16 bytes per instruction cost more address cycles than
+// the arithmetic), each wave owns its 32 tokens' q slice, and a wave whose four
+// key sub-tiles all count runs the next sub-tile's products under the current
+// one's exp2.  256 tokens share a key chunk.  At b = 2, s = 4096, 32 heads of 128:
+// 315 us before, 239 us now, of which the VALU's share is about 150 us (544
+// workgroups are a little over two rounds of 256 compute units).
+template <int D, int NW>
+struct PassCfg {
+  using C = Cfg<D, NW>;
+  static constexpr int QP = 32 * C::ROWB / 1024;            // 1 KiB pieces of a wave's q slice
+  static constexpr int KP = C::KC * C::ROWB / 1024 / NW;    // and of the key chunk, per wave
+  static constexpr int OFF_Q = 2 * C::KC * C::ROWB;
+  static constexpr int PT_STRIDE = C::KC + 4;               // sparse state: a token's P row in LDS (floats; rows on distinct banks)
+  static constexpr int PT_BYTES = 32 * PT_STRIDE * 4;
+  static constexpr int LOOP_BYTES = OFF_Q + NW * 32 * C::ROWB;
+  static constexpr int BYTES = LOOP_BYTES > NW * PT_BYTES ? LOOP_BYTES : NW * PT_BYTES;
+  static_assert(C::KC * C::ROWB % (1024 * NW) == 0 && BYTES <= 160 * 1024, "pass LDS");
+  // rows unpadded; 16-byte chunk c of row r at c ^ swz(r): 16 consecutive rows on distinct banks
+  __device__ static __forceinline__ int swz(int r) { return C::CPR % 16 == 0 ? (r & 15) : ((r >> 1) & 7); }
+  static_assert(C::CPR % 8 == 0, "swizzle within the row");
+};
+
 // LOSS: the KL partial sums; GRAD: P (p.grad, or the sparse state's p.pc) and the
 // R partial sums.
 template <int D, int NW, bool LOSS, bool GRAD>
-__global__ void __launch_bounds__(64 * NW) kl_pass_kernel(Params p) {
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4))) kl_pass_kernel(Params p) {
   using C = Cfg<D, NW>;
+  using PC = PassCfg<D, NW>;
   constexpr int kTB = C::TB;
-  __shared__ __attribute__((aligned(16))) unsigned char KS[2][C::KC * C::STRIDE];
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int w = wave_id(), lane = lane_id(), g = lane >> 5;
   // Work items are the (b, block, chunk) pairs at or below the diagonal:
   // first every block's full chunks, block-major, then the cheaper diagonal
@@ -432,39 +504,35 @@ __global__ void __launch_bounds__(64 * NW) kl_pass_kernel(Params p) {
   // work.  The grid is padded to a multiple of 8 so that each XCD takes one
   // contiguous, equal share (consecutive items share a token block's q rows
   // in that XCD's L2).
-  const int64_t NB = (p.Sq + kTB - 1) / kTB;
-  const int64_t bid = xcd_remap(blockIdx.x, gridDim.x);
-  if (bid >= p.B * p.NI) return;
-  const int64_t nfull = p.NI - NB;  // items per batch before the diagonal ones
-  int64_t b, blk = 0, ci;
-  if (bid < p.B * nfull) {
-    b = bid / nfull;
-    int64_t rem = bid % nfull;
-    for (;; ++blk) {  // scalar walk over the blocks' full-chunk counts (NB steps at most)
-      const int64_t n = block_chunks(p, blk, kTB, C::KC) - 1;
+  const uint32_t NB = (uint32_t)((p.Sq + kTB - 1) / kTB), NI = (uint32_t)p.NI, nb = (uint32_t)p.B;
+  const uint32_t bid = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);
+  if (bid >= nb * NI) return;
+  const uint32_t nfull = NI - NB;  // items per batch before the diagonal ones
+  uint32_t bb, bk = 0, cc;
+  if (bid < nb * nfull) {
+    bb = bid / nfull;
+    uint32_t rem = bid - bb * nfull;
+    for (;; ++bk) {  // scalar walk over the blocks' full-chunk counts (NB steps at most)
+      const uint32_t n = (uint32_t)block_chunks(p, bk, kTB, C::KC) - 1;
       if (rem < n) break;
       rem -= n;
     }
-    ci = rem;
+    cc = rem;
   } else {
-    const int64_t r = bid - p.B * nfull;
-    b = r / NB;
-    blk = r % NB;
-    ci = block_chunks(p, blk, kTB, C::KC) - 1;
+    const uint32_t r = bid - nb * nfull;
+    bb = r / NB;
+    bk = r - bb * NB;
+    cc = (uint32_t)block_chunks(p, bk, kTB, C::KC) - 1;
   }
+  const int64_t b = bb, blk = bk, ci = cc;
   const int64_t t0 = blk * kTB, k0 = ci * C::KC;
   const int64_t wt0 = t0 + 32 * w, t = wt0 + (lane & 31), wt_last = wt0 + 31;
-  const int64_t hpg = p.H / p.G;
-  ChunkLoader<D, NW> ld(p);
 
-  // admissible bits of this lane's 16 keys per sub-tile (same for every head)
-  uint32_t vb[C::SUBS];
   bool sub_on[C::SUBS];
 #pragma unroll
   for (int sub = 0; sub < C::SUBS; ++sub) {
     const int64_t key0 = k0 + 32 * sub;
     sub_on[sub] = key0 <= wt_last && key0 < p.Sk && wt0 < p.Sq;  // wave-uniform
-    vb[sub] = sub_on[sub] ? valid_bits(p, mask_word(p, b, t, key0), t, key0) : 0u;
   }
 
   float P[C::SUBS][16];
@@ -473,76 +541,211 @@ __global__ void __launch_bounds__(64 * NW) kl_pass_kernel(Params p) {
 #pragma unroll
     for (int a = 0; a < 16; ++a) P[sub][a] = 0.0f;
 
-  i32x4 kr[C::LOADS];
-  ld.load(p, b, 0, k0, kr);
-  ChunkLoader<D, NW>::store(KS[0], kr);
-  __syncthreads();
-  // the next head's q operand and normaliser are loaded one head ahead
+  // this lane's source bytes in its wave's pieces of the q slice and of the key chunk
+  const uint32_t qpitch = (uint32_t)(p.B * p.H * C::ROWB), kpitch = (uint32_t)(p.B * p.G * C::ROWB);
+  uint32_t qo[PC::QP], ko[PC::KP];
+#pragma unroll
+  for (int i = 0; i < PC::QP; ++i) {
+    const int u = 64 * i + lane, r = u / C::CPR;
+    qo[i] = (uint32_t)r * qpitch + (uint32_t)(((u - r * C::CPR) ^ PC::swz(r)) * 16);
+  }
+#pragma unroll
+  for (int i = 0; i < PC::KP; ++i) {
+    const int u = 64 * (w * PC::KP + i) + lane, r = u / C::CPR;
+    ko[i] = (uint32_t)r * kpitch + (uint32_t)(((u - r * C::CPR) ^ PC::swz(r)) * 16);
+  }
+  const int64_t nq = p.Sq - wt0 < 32 ? p.Sq - wt0 : 32;  // (rows past Sq and Sk read zeros)
+  const uint32_t qbytes = nq > 0 ? (uint32_t)((nq - 1) * qpitch + C::ROWB) : 0u;
+  const int64_t nk = p.Sk - k0 < C::KC ? p.Sk - k0 : C::KC;
+  const uint32_t kbytes = (uint32_t)((nk - 1) * kpitch + C::ROWB);
+  const unsigned char *qb = p.query + (((nq > 0 ? wt0 : 0) * p.B + b) * p.H) * (int64_t)C::ROWB;
+  const unsigned char *kbase = p.key + ((k0 * p.B + b) * p.G) * (int64_t)C::ROWB;
+  const uint32_t lds = lds_address(smem);
+  const uint32_t q_lds = lds + (uint32_t)(PC::OFF_Q + w * 32 * C::ROWB);
+  // piece i of this wave's loads for a head: its share of the key chunk (into
+  // buffer kbuf; a head of the same key group fetches it again), then its q slice
+  const int hpg = (int)(p.H / p.G), H = (int)p.H;
+  auto fetch = [&](i32x4 krs, i32x4 qrs, int kbuf, int i) {
+    if (i < PC::KP)
+      lds_dma_16(lds + (uint32_t)(kbuf * C::KC * C::ROWB + (w * PC::KP + i) * 1024), ko[i < PC::KP ? i : 0], krs, 0u);
+    else
+      lds_dma_16(q_lds + (uint32_t)((i - PC::KP) * 1024), qo[i < PC::KP ? 0 : i - PC::KP], qrs, 0u);
+  };
+  auto key_rs = [&](int h) { return make_buffer_words(kbase + h / hpg * C::ROWB, kbytes); };
+  auto query_rs = [&](int h) { return make_buffer_words(qb + h * C::ROWB, qbytes); };
+  constexpr int NF = PC::KP + PC::QP;  // loads per head
+  bool all_on = true, any_on = false;  // wave-uniform
+#pragma unroll
+  for (int sub = 0; sub < C::SUBS; ++sub) {
+    all_on = all_on && sub_on[sub];
+    any_on = any_on || sub_on[sub];
+  }
+  // operand of k-step k: row (lane & 31), chunk 2 k + g
+  const int l32 = lane & 31;
+  auto operand = [&](const unsigned char *tile, int r0, int k) {
+    return as_bf16x8(*reinterpret_cast<const i32x4 *>(tile + (r0 + l32) * C::ROWB + (((2 * k + g) ^ PC::swz(l32)) * 16)));
+  };
   const float *beta_bt = p.beta + b * p.H * p.Sq + (t < p.Sq ? t : 0);
-  bf16x8 Qn[C::KSTEPS];
-  load_q_operand<D>(p, b, 0, t, Qn);
-  float bn = beta_bt[0];
-  for (int64_t h = 0; h < p.H; ++h) {
-    const int64_t grp = h / hpg;
-    const bool last_of_grp = h % hpg == hpg - 1;
-    if (h % hpg == 0 && grp + 1 < p.G) ld.load(p, b, grp + 1, k0, kr);
+  i32x4 krs = key_rs(0), qrs = query_rs(0);
+#pragma unroll
+  for (int i = 0; i < NF; ++i) fetch(krs, qrs, 0, i);
+  // The previous head's last sub-tile and its normaliser: its exp2 work runs
+  // under the next head's first products (before head 0: exp2(-inf) = 0).
+  f32x16 cur;
+#pragma unroll
+  for (int a = 0; a < 16; ++a) cur[a] = 0.0f;
+  float bprev = INFINITY, bn = beta_bt[0];
+  for (int h = 0; h < H; ++h) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this head's q and k, fetched a head ago
+    __syncthreads();                     // every wave's share of k; the other k buffer is consumed
+    const unsigned char *ks = smem + (h & 1) * C::KC * C::ROWB;
     bf16x8 Q[C::KSTEPS];
 #pragma unroll
-    for (int k = 0; k < C::KSTEPS; ++k) Q[k] = Qn[k];
+    for (int k = 0; k < C::KSTEPS; ++k) Q[k] = operand(smem + PC::OFF_Q + w * 32 * C::ROWB, 0, k);
     const float bh = bn;
-    if (h + 1 < p.H) {
-      load_q_operand<D>(p, b, h + 1, t, Qn);
-      bn = beta_bt[(h + 1) * p.Sq];
-    }
-    const unsigned char *ks = KS[grp & 1];
+    const int hn = h + 1 < H ? h + 1 : h;  // (past the last head: its own again, unused)
+    bn = beta_bt[(int64_t)hn * p.Sq];
+    krs = key_rs(hn);
+    qrs = query_rs(hn);
+    const int kb = (h + 1) & 1;
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the q slice is in registers, its LDS free
+    if (all_on) {
+      // key operands are read two products ahead
+      constexpr int kSteps = C::SUBS * C::KSTEPS;
+      auto key_operand = [&](int i) { return operand(ks, 32 * (i / C::KSTEPS), i % C::KSTEPS); };
+      bf16x8 ring[3];
+      ring[0] = key_operand(0);
+      ring[1] = key_operand(1);
 #pragma unroll
-    for (int sub = 0; sub < C::SUBS; ++sub) {
-      if (!sub_on[sub]) continue;
-      const f32x16 acc = qk_subtile<D>(ks, sub, Q);
+      for (int sub = 0; sub < C::SUBS; ++sub) {
+        // sub-tile sub's products, each followed by its share of the exp2 work of the sub-tile before it
+        constexpr int kE = 16 / C::KSTEPS > 0 ? (16 + C::KSTEPS - 1) / C::KSTEPS : 1;
+        const int ps = sub == 0 ? C::SUBS - 1 : sub - 1;
+        const float pb = sub == 0 ? bprev : bh;
+        f32x16 nxt;
 #pragma unroll
-      for (int a = 0; a < 16; ++a) P[sub][a] += exp2_fast(fmaf(acc[a], p.c, -bh));
-    }
-    if (last_of_grp && grp + 1 < p.G) {
-      // the other buffer was last read for group grp - 1, before the previous barrier
-      ChunkLoader<D, NW>::store(KS[(grp + 1) & 1], kr);
-      __syncthreads();
+        for (int a = 0; a < 16; ++a) nxt[a] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < C::KSTEPS; ++k) {
+          const int i = sub * C::KSTEPS + k;
+          if (i + 2 < kSteps) ring[(i + 2) % 3] = key_operand(i + 2);
+          nxt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[i % 3], Q[k], nxt, 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < kE; ++e)
+            if (k * kE + e < 16) P[ps][k * kE + e] += exp2_fast(fmaf(cur[k * kE + e], p.c, -pb));
+          // the next head's loads, spread over the first sub-tiles
+          constexpr int kPer = (NF + C::KSTEPS * (C::SUBS - 1) - 1) / (C::KSTEPS * (C::SUBS - 1));
+#pragma unroll
+          for (int u = 0; u < kPer; ++u) {
+            const int f = i * kPer + u;
+            if (f < NF) fetch(krs, qrs, kb, f);
+          }
+          __builtin_amdgcn_sched_barrier(0);  // keep this order
+        }
+        cur = nxt;
+      }
+      bprev = bh;
+    } else {
+#pragma unroll
+      for (int i = 0; i < NF; ++i) fetch(krs, qrs, kb, i);
+      if (any_on) {
+#pragma unroll
+        for (int sub = 0; sub < C::SUBS; ++sub) {
+          if (!sub_on[sub]) continue;
+          f32x16 acc;
+#pragma unroll
+          for (int a = 0; a < 16; ++a) acc[a] = 0.0f;
+#pragma unroll
+          for (int k = 0; k < C::KSTEPS; ++k)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(ks, 32 * sub, k), Q[k], acc, 0, 0, 0);
+#pragma unroll
+          for (int a = 0; a < 16; ++a) P[sub][a] += exp2_fast(fmaf(acc[a], p.c, -bh));
+        }
+      }
     }
   }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // the last loads have landed before the LDS is given up
+  if (all_on) {
+#pragma unroll
+    for (int a = 0; a < 16; ++a) P[C::SUBS - 1][a] += exp2_fast(fmaf(cur[a], p.c, -bprev));
+  }
 
-  // KL terms of the chunk: P = (head sum) / H on admissible columns, 0 elsewhere
-  const float inv_h = 1.0f / (float)p.H;
+  const float inv_h = 1.0f / (float)p.H;  // P = (head sum) / H on admissible columns, 0 elsewhere
+  const int64_t row = b * p.Sq + (t < p.Sq ? t : 0);
+  if (GRAD && p.pc != nullptr) {
+    // sparse state: the set columns' P at their rank (kl_rows_state_kernel forms
+    // the rest).  P goes through LDS, so that each lane walks the set bits of half
+    // its token's words instead of testing every accumulator
+    __syncthreads();  // every wave is done with the key chunks
+    float *tile = reinterpret_cast<float *>(smem + w * PC::PT_BYTES);
+    if (any_on) {
+#pragma unroll
+      for (int sub = 0; sub < C::SUBS; ++sub)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *reinterpret_cast<f32x4 *>(tile + l32 * PC::PT_STRIDE + 32 * sub + 8 * i + 4 * g) =
+              f32x4{P[sub][4 * i], P[sub][4 * i + 1], P[sub][4 * i + 2], P[sub][4 * i + 3]};
+      wave_lds_sync();
+      float *crow = p.pc + row * p.K;
+      int at = p.cpre[row * (p.NC + 2) + ci];  // rank of the chunk's first set column
+      uint32_t words[C::SUBS];
+#pragma unroll
+      for (int sub = 0; sub < C::SUBS; ++sub) words[sub] = mask_word(p, b, t, k0 + 32 * sub);
+#pragma unroll
+      for (int sub = 0; sub < C::SUBS; ++sub) {
+        if (sub >= C::SUBS / 2 == (g != 0)) {  // lane half 0: the first words, half 1: the last
+          const int64_t last = (t < p.Sk - 1 ? t : p.Sk - 1) - (k0 + 32 * sub);  // last admissible bit
+          uint32_t word = t >= p.Sq || last < 0 ? 0u : words[sub] & (last >= 31 ? 0xffffffffu : (2u << last) - 1u);
+          int r = at;
+          while (word) {
+            const int bit = __builtin_ctz(word);
+            word &= word - 1u;
+            crow[r++] = tile[l32 * PC::PT_STRIDE + 32 * sub + bit] * inv_h;
+          }
+        }
+        at += __popc(words[sub]);
+      }
+    }
+    return;
+  }
+  // admissible bits of this lane's 16 keys per sub-tile
+  uint32_t vb[C::SUBS];
+#pragma unroll
+  for (int sub = 0; sub < C::SUBS; ++sub)
+    vb[sub] = sub_on[sub] ? valid_bits(p, mask_word(p, b, t, k0 + 32 * sub), t, k0 + 32 * sub) : 0u;
+
+  // KL terms of the chunk against Q; the index scores of every sub-tile are loaded before any is used
   const float gam = t < p.Sq ? p.gamma[b * p.Sq + t] : 0.0f;
   const float *irow = p.index_scores + b * p.Sq * p.Sk;
   const auto irs = make_buffer_rsrc(irow, (uint32_t)(p.Sq * p.Sk * 4));
   const bool vec = (p.Sk & 3) == 0;  // rows 16-byte aligned: one b128 load per 4 keys
-  float kl = 0.0f, rsum = 0.0f;
-  const int64_t row = b * p.Sq + (t < p.Sq ? t : 0);
-  const bool compact = GRAD && p.pc != nullptr;
-  float *grow = GRAD && !compact ? p.grad + row * p.Sk : nullptr;
-  float *crow = compact ? p.pc + row * p.K : nullptr;
-  int at = compact ? p.cpre[row * (p.NC + 2) + ci] : 0;  // rank of the sub-tile's first set column
+  f32x4 iv[C::SUBS][4];
 #pragma unroll
-  for (int sub = 0; sub < C::SUBS; ++sub) {
-    if (!sub_on[sub]) continue;
-    const int64_t key0 = k0 + 32 * sub;
-    const uint32_t word = compact ? mask_word(p, b, t, key0) : 0u;
+  for (int sub = 0; sub < C::SUBS; ++sub)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      // keys key0 + 8i + 4g + (0..3) of this lane's row; reads past the row
-      // (or past Sq) only feed inadmissible columns
-      const int64_t s0 = key0 + 8 * i + 4 * g;
-      f32x4 iv;
+      // keys s0 .. s0 + 3 of this lane's row; reads past the row (or past Sq) only feed inadmissible columns
+      const int64_t s0 = k0 + 32 * sub + 8 * i + 4 * g;
       if (vec) {
-        const uint32_t off = t < p.Sq ? (uint32_t)((t * p.Sk + s0) * 4) : 0xfffffff0u;
-        iv = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(irs, (int)off, 0, 0));
+        const uint32_t off = t < p.Sq && s0 < p.Sk ? (uint32_t)((t * p.Sk + s0) * 4) : 0xfffffff0u;
+        iv[sub][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(irs, (int)off, 0, 0));
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int64_t s = s0 + j;
           const uint32_t off = (t < p.Sq && s < p.Sk) ? (uint32_t)((t * p.Sk + s) * 4) : 0xfffffff0u;
-          iv[j] = buffer_load_f32(irs, (int)off, 0);
+          iv[sub][i][j] = buffer_load_f32(irs, (int)off, 0);
         }
       }
+    }
+  float kl = 0.0f, rsum = 0.0f;
+  float *grow = GRAD ? p.grad + row * p.Sk : nullptr;
+#pragma unroll
+  for (int sub = 0; sub < C::SUBS; ++sub) {
+    if (!sub_on[sub]) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t s0 = k0 + 32 * sub + 8 * i + 4 * g;
       f32x4 pv;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -551,15 +754,12 @@ __global__ void __launch_bounds__(64 * NW) kl_pass_kernel(Params p) {
         const float pr = on ? P[sub][a] * inv_h : 0.0f;
         pv[j] = pr;
         if (on) {
-          const float q = exp2_fast(fmaf(iv[j], kLog2e, -gam));
+          const float q = exp2_fast(fmaf(iv[sub][i][j], kLog2e, -gam));
           if constexpr (LOSS) kl += pr * (__builtin_amdgcn_logf(pr + kEps) - __builtin_amdgcn_logf(q + kEps));
-          if constexpr (GRAD) {
-            rsum += pr * (q / (q + kEps));
-            if (compact) crow[at + __popc(word & ((1u << (8 * i + 4 * g + j)) - 1u))] = pr;
-          }
+          if constexpr (GRAD) rsum += pr * (q / (q + kEps));
         }
       }
-      if (GRAD && !compact && t < p.Sq && s0 < p.Sk) {  // 0 off the admissible set
+      if (GRAD && t < p.Sq && s0 < p.Sk) {  // 0 off the admissible set
         if (vec) {
           *reinterpret_cast<f32x4 *>(grow + s0) = pv;
         } else {
@@ -569,7 +769,6 @@ __global__ void __launch_bounds__(64 * NW) kl_pass_kernel(Params p) {
         }
       }
     }
-    at += __popc(word);
   }
   if constexpr (GRAD) {
     rsum = sum_halves(rsum);
@@ -646,35 +845,41 @@ __global__ void __launch_bounds__(kNT) kl_grad_kernel(Params p) {
   }
 }
 
-// Sparse state: v over P in place, one wave per row, and the row's loss.
+// Sparse state, one wave per row: the row's loss and R over its set columns (a
+// fixed order: lane strides, then a tree), then v over P in place.  A twentieth
+// of the columns a dense chunk would visit, all lanes busy: the logarithms and
+// the division cost 35 K cycles per 256 x 128 chunk in the pass kernel.
 template <int D>
 __global__ void __launch_bounds__(kNT) kl_rows_state_kernel(Params p) {
   const int lane = lane_id();
   const int64_t row = (int64_t)blockIdx.x * 4 + wave_id();
   if (row >= p.B * p.Sq) return;  // wave-uniform
   const int64_t b = row / p.Sq, t = row % p.Sq;
-  const int64_t last_k = t < p.Sk - 1 ? t : p.Sk - 1;
-  const int64_t cmax = last_k / Cfg<D, 4>::KC;
-  float kl = 0.0f, R = 0.0f;
-#pragma unroll 8
-  for (int64_t c = 0; c <= cmax; ++c) {  // in chunk order, the same in every lane
-    kl += p.partial[(b * p.NC + c) * p.Sq + t];
-    R += p.partial_r[(b * p.NC + c) * p.Sq + t];
-  }
   const bool no_target = !(p.beta[b * p.H * p.Sq + t] > -INFINITY);
   const float gam = p.gamma[row];
   const bool nan_row = no_target || gam != gam;
-  if (lane == 0) {
-    p.rows[row] = nan_row ? __builtin_nanf("") : kl;
-    p.flag[row] = nan_row ? __builtin_nanf("") : 0.0f;
-  }
   const int32_t *pre = p.cpre + row * (p.NC + 2);
   const int n = pre[p.NC], adm = pre[p.NC + 1];
   float *v = p.pc + row * p.K;
   const float *x = p.xc + row * p.K;
+  float kl = 0.0f, R = 0.0f;
+  for (int e = lane; e < adm; e += 64) {  // (columns past the diagonal have no target)
+    const float q = exp2_fast(fmaf(x[e], kLog2e, -gam)), pe = v[e];
+    kl += pe * (__builtin_amdgcn_logf(pe + kEps) - __builtin_amdgcn_logf(q + kEps));
+    R += pe * (q / (q + kEps));
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    kl += __shfl_xor(kl, off, 64);
+    R += __shfl_xor(R, off, 64);
+  }
+  if (lane == 0) {
+    p.rows[row] = nan_row ? __builtin_nanf("") : kl * kLn2;
+    p.flag[row] = nan_row ? __builtin_nanf("") : 0.0f;
+  }
   for (int e = lane; e < n; e += 64) {
     const float q = exp2_fast(fmaf(x[e], kLog2e, -gam));
-    const float pe = e < adm ? v[e] : 0.0f;  // columns past the diagonal have no target
+    const float pe = e < adm ? v[e] : 0.0f;
     v[e] = fmaf(q, R, -(pe * (q / (q + kEps))));
   }
 }
@@ -743,7 +948,7 @@ __global__ void __launch_bounds__(1024) kl_mean_kernel(Params p) {
 // host
 // ---------------------------------------------------------------------------
 struct Layout {
-  size_t mask, gamma, beta, partial, rows, partial_r, xc, total;
+  size_t mask, tiles, gamma, beta, partial, rows, partial_r, xc, total;
 };
 
 // State of dsa_indexer_kl_loss_with_grad: dense v [B, Sq, Sk]; sparse the bitmask,
@@ -776,6 +981,7 @@ static Layout layout(int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t D, in
   Layout L;
   size_t o = 0;
   L.mask = o;    o += align256(sparse ? (size_t)(B * Sq * W) * 4 : 0);
+  L.tiles = o;   o += align256(sparse ? (size_t)(B * ((Sq + 31) / 32) * W) * 128 : 0);
   L.gamma = o;   o += align256((size_t)(B * Sq) * 4);
   L.beta = o;    o += align256((size_t)(B * H * Sq) * 4);
   L.partial = o; o += align256((size_t)(B * NC * Sq) * 4);
@@ -802,7 +1008,11 @@ static int launch_mfma(const Params &p, hipStream_t st) {
     q.NI += (lt < p.Sk - 1 ? lt : p.Sk - 1) / CP::KC + 1;
   }
   const int64_t items = (p.B * q.NI + 7) / 8 * 8;
-  hipLaunchKernelGGL((kl_pass_kernel<D, NWP, LOSS, GRAD>), dim3((unsigned)items), dim3(CP::NT), 0, st, q);
+  const auto pass = kl_pass_kernel<D, NWP, LOSS, GRAD>;
+  constexpr int lds = PassCfg<D, NWP>::BYTES;
+  const hipError_t e = hipFuncSetAttribute((const void *)pass, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return set_error(DSA_ERR_HIP, "kl_pass_kernel: LDS attribute: %s", hipGetErrorString(e));
+  hipLaunchKernelGGL(pass, dim3((unsigned)items), dim3(CP::NT), lds, st, q);
   rc = check_launch("kl_pass_kernel");
   if (rc) return rc;
   if (p.pc != nullptr) {
@@ -851,6 +1061,7 @@ static int kl_setup(const char *fn, const float *index_scores, const void *topk_
   p.query = static_cast<const unsigned char *>(query);
   p.key = static_cast<const unsigned char *>(key);
   p.mask = reinterpret_cast<uint32_t *>(ws + L.mask);
+  p.tiles = reinterpret_cast<uint64_t *>(ws + L.tiles);
   p.gamma = reinterpret_cast<float *>(ws + L.gamma);
   p.beta = reinterpret_cast<float *>(ws + L.beta);
   p.partial = reinterpret_cast<float *>(ws + L.partial);
@@ -873,11 +1084,18 @@ static int kl_launch(const Params &p, int64_t D, hipStream_t st) {
   hipLaunchKernelGGL(kl_index_stats_kernel, dim3((unsigned)((p.B * p.Sq + 3) / 4)), dim3(kNT), 0, st, p);
   int rc = check_launch("kl_index_stats_kernel");
   if (rc) return rc;
+  if (p.sparse) {
+    hipLaunchKernelGGL(kl_mask_tiles_kernel, dim3((unsigned)(p.B * ((p.Sq + 31) / 32)), (unsigned)(p.W < 64 ? (p.W + 7) / 8 : 8)),
+                       dim3(kNT), 0, st, p);
+    rc = check_launch("kl_mask_tiles_kernel");
+    if (rc) return rc;
+  }
   switch (D) {
-    case 64: return launch_mfma<64, 8, 4, LOSS, GRAD>(p, st);
-    case 128: return launch_mfma<128, 8, 4, LOSS, GRAD>(p, st);
-    case 192: return launch_mfma<192, 8, 4, LOSS, GRAD>(p, st);
-    default: return launch_mfma<256, 8, 4, LOSS, GRAD>(p, st);
+    case 64: return launch_mfma<64, 8, 8, LOSS, GRAD>(p, st);
+    case 128: return launch_mfma<128, 8, 8, LOSS, GRAD>(p, st);
+    case 192: return launch_mfma<192, 8, 8, LOSS, GRAD>(p, st);
+    default:  // (eight q slices and two key chunks would pass 160 KiB)
+      return launch_mfma<256, 8, 4, LOSS, GRAD>(p, st);
   }
 }
 
@@ -951,8 +1169,8 @@ static void kl_bind_state(dsa::kl::Params &p, void *state, const dsa::kl::State 
 }
 
 extern "C" int dsa_indexer_kl_loss_with_grad(const float *index_scores, const void *topk_indices, int topk_dtype,
-                                             int64_t topk, const void *query, const void *key, float *loss, void *state,
-                                             size_t state_bytes, int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t G,
+                                             int64_t topk, const void *query, const void *key, float *loss,
+                                             float *row_loss, void *state, size_t state_bytes, int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t G,
                                              int64_t D, float softmax_scale, float loss_coeff, int sparse,
                                              void *workspace, size_t workspace_bytes, void *stream) {
   using namespace dsa;
@@ -968,6 +1186,7 @@ extern "C" int dsa_indexer_kl_loss_with_grad(const float *index_scores, const vo
                      state ? state_bytes : (size_t)0, S.total);
   kl_bind_state(p, state, S);
   if (!p.sparse) p.grad = static_cast<float *>(state);
+  if (row_loss) p.rows = row_loss;
   p.loss = loss;
   hipStream_t st = static_cast<hipStream_t>(stream);
   rc = kl_launch<true, true>(p, D, st);

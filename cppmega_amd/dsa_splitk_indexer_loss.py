@@ -70,6 +70,10 @@ def _prepare(index_scores, topk_indices, query, key, sparse_loss):
 
 
 def _forward(index_scores, topk_indices, query, key, softmax_scale, loss_coeff, sparse_loss, return_rows):
+    if sparse_loss:  # the rows' terms over their top-k columns alone
+        loss, _, _, rows = _forward_state(index_scores, topk_indices, query, key, softmax_scale, loss_coeff, True,
+                                          return_rows)
+        return loss, rows
     index_scores, topk_indices, tdt, topk, query, key, sparse, (b, sq, sk, np_, g, hn) = _prepare(
         index_scores, topk_indices, query, key, sparse_loss)
     dev = _lib.ensure_device(query)
@@ -87,16 +91,53 @@ def _forward(index_scores, topk_indices, query, key, softmax_scale, loss_coeff, 
     return loss, rows
 
 
+def _forward_state(index_scores, topk_indices, query, key, softmax_scale, loss_coeff, sparse_loss, return_rows=False):
+    """(loss, state, args of _apply_state, per-row losses or None): the loss and its gradient up to the upstream
+    factor."""
+    index_scores, topk_indices, tdt, topk, query, key, sparse, (b, sq, sk, np_, g, hn) = _prepare(
+        index_scores, topk_indices, query, key, sparse_loss)
+    dev = _lib.ensure_device(query)
+    lib = _lib.load()
+    sp = 1 if sparse else 0
+    ws = torch.empty(max(int(lib.dsa_indexer_kl_loss_with_grad_workspace_size(b, sq, sk, np_, hn, topk, sp)), 1),
+                     dtype=torch.uint8, device=query.device)
+    state = torch.empty(max(int(lib.dsa_indexer_kl_loss_state_size(b, sq, sk, hn, topk, sp)), 1),
+                        dtype=torch.uint8, device=query.device)
+    loss = torch.empty((), dtype=torch.float32, device=query.device)
+    rows = torch.empty((b, sq), dtype=torch.float32, device=query.device) if return_rows else None
+    rc = lib.dsa_indexer_kl_loss_with_grad(
+        index_scores.data_ptr(), _lib.ptr(topk_indices), tdt, topk, query.data_ptr(), key.data_ptr(), loss.data_ptr(),
+        _lib.ptr(rows), state.data_ptr(), state.numel(), b, sq, sk, np_, g, hn, float(softmax_scale), float(loss_coeff), sp,
+        ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
+    _lib.check(rc, "dsa_indexer_kl_loss_with_grad")
+    return loss, state, (b, sq, sk, hn, topk, float(loss_coeff), sp), rows
+
+
+def _apply_state(state, grad_loss, args):
+    """dL/d index_scores [b, sq, sk] f32 from a state and the upstream factor (1-element f32)."""
+    b, sq, sk, hn, topk, coeff, sp = args
+    dev = _lib.ensure_device(state)
+    grad = torch.empty((b, sq, sk), dtype=torch.float32, device=state.device)
+    rc = _lib.load().dsa_indexer_kl_loss_grad_apply(
+        state.data_ptr(), state.numel(), grad_loss.data_ptr(), grad.data_ptr(), b, sq, sk, hn, topk, coeff, sp,
+        _lib.stream_ptr(dev))
+    _lib.check(rc, "dsa_indexer_kl_loss_grad_apply")
+    return grad
+
+
 def indexer_kl_loss_backward(grad_loss, index_scores, topk_indices, query, key, softmax_scale, loss_coeff=1.0,
                              sparse_loss=False):
     """dL/d index_scores [b, sq, sk] f32 for the upstream gradient ``grad_loss``
     (a scalar tensor or number) of ``indexer_kl_loss``'s scalar; the target P is
     recomputed on the GPU.  NaN over a row whose loss is NaN."""
+    gl = torch.as_tensor(grad_loss, dtype=torch.float32, device=query.device).reshape(1).contiguous()
+    if sparse_loss:  # the top-k columns' state, expanded
+        _, state, args, _ = _forward_state(index_scores, topk_indices, query, key, softmax_scale, loss_coeff, True)
+        return _apply_state(state, gl, args)
     index_scores, topk_indices, tdt, topk, query, key, sparse, (b, sq, sk, np_, g, hn) = _prepare(
         index_scores, topk_indices, query, key, sparse_loss)
     dev = _lib.ensure_device(query)
     lib = _lib.load()
-    gl = torch.as_tensor(grad_loss, dtype=torch.float32, device=query.device).reshape(1).contiguous()
     ws_bytes = lib.dsa_indexer_kl_loss_workspace_size(b, sq, sk, np_, hn, 1 if sparse else 0)
     ws = torch.empty(max(int(ws_bytes), 1), dtype=torch.uint8, device=query.device)
     grad = torch.empty((b, sq, sk), dtype=torch.float32, device=query.device)
@@ -115,37 +156,18 @@ class _IndexerKLLoss(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, index_scores, topk_indices, query, key, softmax_scale, loss_coeff, sparse_loss):
-        scores, topk_indices, tdt, topk, query, key, sparse, (b, sq, sk, np_, g, hn) = _prepare(
-            index_scores, topk_indices, query, key, sparse_loss)
-        dev = _lib.ensure_device(query)
-        lib = _lib.load()
-        sp = 1 if sparse else 0
-        ws = torch.empty(max(int(lib.dsa_indexer_kl_loss_with_grad_workspace_size(b, sq, sk, np_, hn, topk, sp)), 1),
-                         dtype=torch.uint8, device=query.device)
-        state = torch.empty(max(int(lib.dsa_indexer_kl_loss_state_size(b, sq, sk, hn, topk, sp)), 1),
-                            dtype=torch.uint8, device=query.device)
-        loss = torch.empty((), dtype=torch.float32, device=query.device)
-        rc = lib.dsa_indexer_kl_loss_with_grad(
-            scores.data_ptr(), _lib.ptr(topk_indices), tdt, topk, query.data_ptr(), key.data_ptr(), loss.data_ptr(),
-            state.data_ptr(), state.numel(), b, sq, sk, np_, g, hn, float(softmax_scale), float(loss_coeff), sp,
-            ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
-        _lib.check(rc, "dsa_indexer_kl_loss_with_grad")
+        loss, state, args, _ = _forward_state(index_scores, topk_indices, query, key, softmax_scale, loss_coeff,
+                                           sparse_loss)
         ctx.save_for_backward(state)
-        ctx.args = (b, sq, sk, hn, topk, float(loss_coeff), sp, index_scores.dtype)
+        ctx.args = args
+        ctx.dtype = index_scores.dtype
         return loss
 
     @staticmethod
     def backward(ctx, grad_loss):
         state, = ctx.saved_tensors
-        b, sq, sk, hn, topk, coeff, sp, dtype = ctx.args
-        dev = _lib.ensure_device(state)
-        gl = grad_loss.to(torch.float32).reshape(1).contiguous()
-        grad = torch.empty((b, sq, sk), dtype=torch.float32, device=state.device)
-        rc = _lib.load().dsa_indexer_kl_loss_grad_apply(
-            state.data_ptr(), state.numel(), gl.data_ptr(), grad.data_ptr(), b, sq, sk, hn, topk, coeff, sp,
-            _lib.stream_ptr(dev))
-        _lib.check(rc, "dsa_indexer_kl_loss_grad_apply")
-        return grad.to(dtype), None, None, None, None, None, None
+        grad = _apply_state(state, grad_loss.to(torch.float32).reshape(1).contiguous(), ctx.args)
+        return grad.to(ctx.dtype), None, None, None, None, None, None
 
 
 def indexer_kl_loss(index_scores, topk_indices, query, key, softmax_scale, loss_coeff=1.0, sparse_loss=False,

@@ -531,10 +531,11 @@ int dsa_indexer_kl_loss_backward(const float *index_scores,
 
 /*
  * The loss and the gradient together, for a caller that will ask for both: one
- * run leaves the loss (as dsa_indexer_kl_loss) and a state of
+ * run leaves the loss (and row_loss, or NULL, as dsa_indexer_kl_loss; sparse: the
+ * row sums in another order) and a state of
  * dsa_indexer_kl_loss_state_size bytes, from which
  * dsa_indexer_kl_loss_grad_apply forms grad_index_scores (as
- * dsa_indexer_kl_loss_backward, bit for bit) for any upstream gradient, any
+ * dsa_indexer_kl_loss_backward up to that order) for any upstream gradient, any
  * number of times, without the scores, query or key.  The state is the size of
  * the scores, or (sparse) 4 bytes per top-k entry and about Sk / 8 + Sk / 32
  * bytes per row.  loss_coeff is read by the second call.  The workspace
@@ -547,9 +548,9 @@ size_t dsa_indexer_kl_loss_with_grad_workspace_size(int64_t B, int64_t Sq, int64
                                                     int sparse);
 int dsa_indexer_kl_loss_with_grad(const float *index_scores, const void *topk_indices,
                                   int topk_dtype, int64_t topk, const void *query,
-                                  const void *key, float *loss, void *state,
-                                  size_t state_bytes, int64_t B, int64_t Sq,
-                                  int64_t Sk, int64_t H, int64_t G, int64_t D,
+                                  const void *key, float *loss, float *row_loss,
+                                  void *state, size_t state_bytes, int64_t B,
+                                  int64_t Sq, int64_t Sk, int64_t H, int64_t G, int64_t D,
                                   float softmax_scale, float loss_coeff, int sparse,
                                   void *workspace, size_t workspace_bytes,
                                   void *stream);

@@ -1,10 +1,11 @@
-"""The KL loss's saved gradient state (autograd path) against the recomputing
-gradient call, bit for bit: top-k lists unsorted, padded, repeated, beyond the
-diagonal; chunk and word edges; rows without a target; several upstream factors."""
+"""The KL loss's saved gradient state (autograd path) against the gradient call,
+bit for bit, and against the loss and gradient kernels that keep no state: top-k
+lists unsorted, padded, repeated, beyond the diagonal; chunk and word edges; rows
+without a target; several upstream factors."""
 import pytest
 import torch
 
-from cppmega_amd import indexer_kl_loss, indexer_kl_loss_backward
+from cppmega_amd import _lib, indexer_kl_loss, indexer_kl_loss_backward
 
 pytestmark = pytest.mark.gpu
 
@@ -27,15 +28,30 @@ def test_state_gradient_matches_direct(dev, b, sq, sk, np_, hn, topk, sparse):
     z[0, 0, sk // 2] = -torch.inf
     query = torch.randn((sq, b, np_, hn), generator=g).to(torch.bfloat16).to(dev)
     key = torch.randn((sk, b, np_, hn), generator=g).to(torch.bfloat16).to(dev)
-    idx, scale = idx.to(dev), hn ** -0.5
+    idx, scale = idx.contiguous().to(dev), hn ** -0.5
     zr = z.to(dev).requires_grad_()
     loss = indexer_kl_loss(zr, idx, query, key, scale, 0.7, sparse)
     with torch.no_grad():
         plain, rows = indexer_kl_loss(zr.detach(), idx, query, key, scale, 0.7, sparse, return_rows=True)
-    assert torch.equal(loss.detach().isnan(), plain.isnan()) and (plain.isnan() or loss.detach() == plain)
+    assert torch.equal(loss.detach().isnan(), plain.isnan()) and (bool(plain.isnan()) or loss.detach() == plain)
     assert bool(rows.isnan().any()) == sparse
+    lib = _lib.load()
     for f in (1.0, -3.25):
-        got, = torch.autograd.grad(loss, zr, torch.tensor(f, device=dev), retain_graph=True)
-        want = indexer_kl_loss_backward(torch.tensor(f, device=dev), zr.detach(), idx, query, key, scale, 0.7, sparse)
+        gl = torch.tensor([f], device=dev)
+        got, = torch.autograd.grad(loss, zr, gl[0], retain_graph=True)
+        want = indexer_kl_loss_backward(gl[0], zr.detach(), idx, query, key, scale, 0.7, sparse)
         assert torch.equal(got.isnan(), want.isnan())
         assert torch.equal(got.nan_to_num(), want.nan_to_num())
+        direct = torch.empty_like(got)
+        ws = torch.empty(int(lib.dsa_indexer_kl_loss_workspace_size(b, sq, sk, np_, hn, int(sparse))), dtype=torch.uint8,
+                         device=dev)
+        zd = zr.detach().contiguous()
+        _lib.check(lib.dsa_indexer_kl_loss_backward(
+            zd.data_ptr(), idx.data_ptr() if sparse else None, _lib.DTYPE_I64, topk if sparse else 0, query.data_ptr(),
+            key.data_ptr(), gl.data_ptr(), direct.data_ptr(), b, sq, sk, np_, np_, hn, scale, 0.7, int(sparse),
+            ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream), "dsa_indexer_kl_loss_backward")
+        assert torch.equal(got.isnan(), direct.isnan())
+        got, direct = got.nan_to_num(), direct.nan_to_num()
+        # the same terms summed in another order: at most sk + sq of them, 2^-24 each
+        bound = (sk + sq) * 2.0 ** -24
+        assert float((got - direct).abs().max()) <= 2 * bound * float(direct.abs().max())
