@@ -47,6 +47,8 @@ struct IdxParams {
   int64_t mask_bstride;
   const int32_t *row_plain;
   int64_t B, Sq, Sk;
+  int64_t chunk; // causal modes 0 / 1: keys per workgroup, a multiple of the key tile
+  int split;     // causal modes 0 / 1: every wave scores the workgroup's one token group, each a share of the keys
   int64_t coff;  // causal modes 1 / 2: row t keeps keys s <= t + coff (q starts coff tokens into the sequence)
   int w_f32;
   int causal;
@@ -65,8 +67,7 @@ struct IdxCfg {
   static constexpr int ROWB = D * ELT;          // bytes per key row
   static constexpr int KT = 16384 / ROWB;       // keys per LDS tile (16 KiB of key rows)
   static constexpr int SUBS = KT / 32;          // 32-key sub-tiles per tile
-  static constexpr int CHUNK = 2048;            // keys per workgroup
-  static constexpr int NKT = CHUNK / KT;        // tiles per workgroup chunk
+  static constexpr int CHUNK = 2048;            // modes 0 and 1: most keys per workgroup
   static constexpr int KS_STRIDE = ROWB + 16;
   static constexpr int KSTEPS = FP8 ? D / 64 : D / 16;  // MFMA k-steps: 32x32x64 f8f6f4 or 32x32x16 bf16
   static constexpr int CPR = ROWB / 16;         // 16-byte chunks per key row
@@ -140,7 +141,7 @@ __device__ __forceinline__ void idx_segment(const IdxParams &p, unsigned char (&
   // holding channels [16 g32, +16) and [32 + 16 g32, +16) of each 64-channel chunk
   typedef typename std::conditional<FP8, i32x8, bf16x8>::type aop_t;
   aop_t A[C::MT][C::KSTEPS];
-  const int64_t wave_tok0 = t0 + w * C::TPW;
+  const int64_t wave_tok0 = t0 + (p.split ? 0 : w * C::TPW);
 #pragma unroll
   for (int m = 0; m < C::MT; ++m) {
     const int r = m * 32 + l32;
@@ -229,7 +230,7 @@ __device__ __forceinline__ void idx_segment(const IdxParams &p, unsigned char (&
     const int tl = C::TPW >= 2 ? 2 * j + g32 : 0;
     soff_lane[j] = (uint32_t)(((wave_tok0 + tl - t0) * p.Sk + k0 + l32) * 4);
   }
-  const bool wave_in_sq = wave_tok0 + C::TPW - 1 < p.Sq;
+  const bool wave_in_sq = wave_tok0 + C::TPW - 1 < p.Sq && !p.split;  // split: sub-tiles are picked below
 
   // window mode: this wave's token windows (wave-uniform scalar loads) and
   // their union; sub-tiles outside the union are not computed
@@ -299,7 +300,7 @@ __device__ __forceinline__ void idx_segment(const IdxParams &p, unsigned char (&
         const int64_t sn = tk + sub * 32;
         // wave-uniform: the sub-tile exists and is not wholly above this wave's
         // diagonal (lower-triangle mode) or outside its windows (window mode)
-        const bool active = sn < k_end && !(p.causal == 2 && sn > wave_tok_last + p.coff) &&
+        const bool active = sn < k_end && !(p.split && ((it * C::SUBS + sub) & 3) != w) && !(p.causal == 2 && sn > wave_tok_last + p.coff) &&
                             !(win && (sn + 32 <= wmin || sn >= wmax));
         const int64_t s = sn + l32;
         float mv[C::TPW];  // window mode: the additive mask, loaded ahead of the MFMAs
@@ -375,7 +376,7 @@ __device__ __forceinline__ void fill_neg_inf_rows(float *out_b, int64_t Sk, int6
 // at most two segments (the end of the long row, the start of the short one).
 // Window mode pairs the blocks the same way over their window unions (for a
 // causal mask: the lower triangle's balance).  Modes 0 and 1 keep fixed chunks
-// of CHUNK keys (all rows as long as Sk).  WIN selects the window-mode
+// of p.chunk keys (all rows as long as Sk).  WIN selects the window-mode
 // instantiation (launched for causal == kCausalWindow only).
 template <int H, int D, bool FP8, bool RELU, bool WIN>
 __global__ void __launch_bounds__((IdxCfg<H, D, FP8>::NT))
@@ -469,10 +470,10 @@ indexer_score_kernel(const IdxParams p) {
     }
     return;
   } else {
-  const int64_t t0 = (int64_t)(gridDim.y - 1 - blockIdx.y) * C::TT;
-  const int64_t k0 = (int64_t)blockIdx.x * C::CHUNK;
+  const int64_t t0 = (int64_t)(gridDim.y - 1 - blockIdx.y) * (p.split ? C::TPW : C::TT);
+  const int64_t k0 = (int64_t)blockIdx.x * p.chunk;
   const int64_t t_last = (t0 + C::TT < p.Sq ? t0 + C::TT : p.Sq) - 1;
-  const int64_t chunk_end = k0 + C::CHUNK < p.Sk ? k0 + C::CHUNK : p.Sk;
+  const int64_t chunk_end = k0 + p.chunk < p.Sk ? k0 + p.chunk : p.Sk;
   const bool outside = p.causal == 1 && k0 > t_last + p.coff;
   if (outside) {
     // chunk wholly above the block's diagonal (mode 1): -inf only
@@ -522,7 +523,7 @@ static int pick_pieces(int64_t groups_per_piece, int64_t slots) {
 }
 
 template <int H, int D, bool FP8, bool RELU>
-static int launch_idx_act(const IdxParams &p, hipStream_t st) {
+static int launch_idx_act(IdxParams p, hipStream_t st) {
   using C = IdxCfg<H, D, FP8>;
   const int64_t ntb = (p.Sq + C::TT - 1) / C::TT;
   DSA_REQUIRE(ntb < 65536, "dsa_indexer_scores: %lld query tokens exceed the grid (%d per workgroup)",
@@ -535,7 +536,16 @@ static int launch_idx_act(const IdxParams &p, hipStream_t st) {
                                                    : resident_groups(indexer_score_kernel<H, D, FP8, RELU, false>, C::NT));
     grid = dim3((unsigned)pieces, (unsigned)npairs, (unsigned)p.B);
   } else {
-    grid = dim3((unsigned)((p.Sk + C::CHUNK - 1) / C::CHUNK), (unsigned)ntb, (unsigned)p.B);
+    // a workgroup takes 2048 keys, which costs the q operands' loads least;
+    // fewer when the grid would not fill the resident slots (a decode step:
+    // 16 tokens x 16384 keys of 64 e4m3 heads of 128 are 128 workgroups of
+    // 2048 keys, 29 us, or 512 of 512 keys, 11.5 us with the keys split among the waves)
+    const int64_t slots = resident_groups(indexer_score_kernel<H, D, FP8, RELU, false>, C::NT);
+    p.chunk = C::CHUNK;
+    // tokens for one wave: the other three would only load keys
+    p.split = p.Sq <= C::TPW;
+    while (p.chunk > C::KT && 2 * ((p.Sk + p.chunk - 1) / p.chunk) * ntb * p.B <= slots) p.chunk /= 2;
+    grid = dim3((unsigned)((p.Sk + p.chunk - 1) / p.chunk), (unsigned)ntb, (unsigned)p.B);
   }
   if (p.causal == kCausalWindow)
     hipLaunchKernelGGL((indexer_score_kernel<H, D, FP8, RELU, true>), grid, dim3(C::NT), 0, st, p);
@@ -585,6 +595,8 @@ static int indexer_scores_impl(const void *q, const void *w, const void *k, floa
   p.Sq = Sq;
   p.Sk = Sk;
   p.coff = coff;
+  p.split = 0;
+  p.chunk = 0;
   p.w_f32 = w_dtype == DSA_DTYPE_F32;
   p.causal = causal;
   p.relu = use_relu != 0;

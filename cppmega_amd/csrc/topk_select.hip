@@ -11,7 +11,8 @@
 // written in ascending order, padded with -1.
 //
 // Rows of up to 8192 columns run one wave per row (topk_wave_kernel), longer
-// rows one workgroup of NW waves per row (topk_block_kernel).  The row stays
+// ones, and few rows of over 2048, one workgroup of NW waves per row
+// (topk_block_kernel).  The row stays
 // in registers; a lower bound of the k-th largest score from per-lane subset
 // maxima keeps the lower scores out of the value-linear histogram, which
 // usually leaves a handful of members in the bucket holding the k-th largest;
@@ -148,6 +149,7 @@ template <int IPL>
 __device__ __forceinline__ void fence_values(float (&x)[IPL], int &ng) {
 #pragma unroll
   for (int i = 0; i < IPL; ++i) asm volatile("" : "+v"(x[i]));
+  if constexpr (IPL == kGroup) ng = __builtin_amdgcn_readfirstlane(ng);  // one group: ng may sit in a lane register
   asm volatile("" : "+s"(ng));
 }
 
@@ -155,36 +157,40 @@ __device__ __forceinline__ int lane_rank(uint64_t mask) {  // set lanes below th
   return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-// Suffix scan of a wave's 1024-bin histogram: the bin holding the r-th largest
-// element and the count above it.
+// The bin of a histogram (16-byte aligned) holding the r-th largest element and
+// the count above it.  Lane l sums the BPL bins from the l-th highest run down,
+// a scan over the lanes finds the run that the r-th falls into, and a second
+// one over that run's bins, one per lane, the bin.  A lane reads its run as
+// 16-byte words in an order rotated by its index: the words' runs lie BPL bins
+// apart, and in step the 64 lanes would all fall on 4 (BPL = 32) or 16 of the
+// 64 LDS banks (read so, bin by bin, the search had bounded the workgroup
+// kernel: top-256 of 16384 causal rows of 16384 columns took 285 us, now 151;
+// top-2048 of 2048 rows of 32768 181 us, now 80, at 3.4 TB/s of scores).
 template <int NBINS = kWaveBins>
 __device__ __forceinline__ void find_bucket(const int *hist, int r, int &bsel, int &above) {
   constexpr int BPL = NBINS / 64;
+  constexpr int W = BPL / 4;  // 16-byte words per lane
+  static_assert(W == 4 || W == 8, "the rotation covers the banks for 4 or 8 words per lane");
   const int lane = lane_id();
-  int cnt[BPL];
-  uint32_t local = 0u;
+  const i32x4 *run = reinterpret_cast<const i32x4 *>(hist + NBINS - (lane + 1) * BPL);
+  const int rot = lane / (16 / W);
+  int local = 0;
 #pragma unroll
-  for (int q = 0; q < BPL; ++q) {
-    cnt[q] = hist[NBINS - 1 - (lane * BPL + q)];
-    local += (uint32_t)cnt[q];
+  for (int q = 0; q < W; ++q) {
+    const i32x4 c = run[(q + rot) & (W - 1)];
+    local += (c[0] + c[1]) + (c[2] + c[3]);
   }
-  const int excl = (int)(wv::wave_incl_scan(local) - local);
-  const bool cross = excl < r && excl + (int)local >= r;
-  int bsel_l = 0, above_l = 0;
-  if (cross) {
-    int acc = excl;
-#pragma unroll
-    for (int q = 0; q < BPL; ++q) {
-      if (acc < r && acc + cnt[q] >= r) {
-        bsel_l = NBINS - 1 - (lane * BPL + q);
-        above_l = acc;
-      }
-      acc += cnt[q];
-    }
-  }
-  const int cl = __ffsll((unsigned long long)wv::ballot(cross)) - 1;  // exactly one lane crosses
-  bsel = (int)wv::readlane((uint32_t)bsel_l, cl < 0 ? 0 : cl);
-  above = (int)wv::readlane((uint32_t)above_l, cl < 0 ? 0 : cl);
+  const int excl = (int)wv::wave_incl_scan((uint32_t)local) - local;
+  const uint64_t cross = wv::ballot(excl < r && excl + local >= r);  // exactly one lane crosses
+  const int cl = cross ? __ffsll((unsigned long long)cross) - 1 : 0;
+  const int before = (int)wv::readlane((uint32_t)excl, cl);
+  const int top = NBINS - 1 - cl * BPL;  // the run's highest bin
+  const int cnt = lane < BPL ? hist[top - lane] : 0;
+  const int ex2 = before + (int)wv::wave_incl_scan((uint32_t)cnt) - cnt;
+  const uint64_t hit = wv::ballot(ex2 < r && ex2 + cnt >= r);
+  const int bl = hit ? __ffsll((unsigned long long)hit) - 1 : 0;
+  bsel = top - bl;
+  above = (int)wv::readlane((uint32_t)ex2, bl);
 }
 
 // Exact rank among <= 64 values held one per lane (lanes >= mm hold padding):
@@ -212,7 +218,7 @@ topk_wave_kernel(const TopkParams p) {
   static_assert(IPL % kGroup == 0, "items come in whole groups");
   constexpr int NG = IPL / kGroup;
   constexpr int BPL = kWaveBins / 64;
-  __shared__ int s_hist[4][kWaveBins + 64];
+  __shared__ __attribute__((aligned(16))) int s_hist[4][kWaveBins + 64];
   __shared__ float s_list[4][64];
   // the wave index is uniform: make the row and everything derived from it scalar
   const int w = __builtin_amdgcn_readfirstlane(wave_id()), lane = lane_id();
@@ -250,7 +256,7 @@ topk_wave_kernel(const TopkParams p) {
     }
   }
 #pragma unroll
-  for (int q = 0; q < BPL; ++q) hist[lane * BPL + q] = 0;
+  for (int q = 0; q < BPL / 4; ++q) reinterpret_cast<i32x4 *>(hist)[q * 64 + lane] = i32x4{0, 0, 0, 0};
   // only the last loaded group reaches past the window
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
@@ -340,7 +346,7 @@ topk_wave_kernel(const TopkParams p) {
       wave_lds_sync();
       int bsel, above;
       find_bucket(hist, r, bsel, above);
-      m = hist[bsel];
+      m = __builtin_amdgcn_readfirstlane(hist[bsel]);
       r -= above;
       const uint32_t bsel_bits = kBinBits + (uint32_t)bsel;
       wave_lds_sync();  // histogram reads finish before it is reused
@@ -408,7 +414,7 @@ topk_wave_kernel(const TopkParams p) {
     const int bl = 32 - __clz((int)(B - A));
     const int shift = bl > 10 ? bl - 10 : 0;
 #pragma unroll
-    for (int q = 0; q < BPL; ++q) hist[lane * BPL + q] = 0;
+    for (int q = 0; q < BPL / 4; ++q) reinterpret_cast<i32x4 *>(hist)[q * 64 + lane] = i32x4{0, 0, 0, 0};
     wave_lds_sync();
     fence_values(x, ng);
 #pragma unroll
@@ -422,7 +428,7 @@ topk_wave_kernel(const TopkParams p) {
     wave_lds_sync();
     int bsel, above;
     find_bucket(hist, r, bsel, above);
-    m = hist[bsel];
+    m = __builtin_amdgcn_readfirstlane(hist[bsel]);
     wave_lds_sync();
     r -= above;
     fence_values(x, ng);
@@ -523,7 +529,7 @@ constexpr int kBlockBins = 2048;
 
 template <int NW>
 struct BlockLds {
-  int hist[kBlockBins + 64];  // + one bin per lane for the scores below the bound
+  __attribute__((aligned(16))) int hist[kBlockBins + 64];  // + one bin per lane for the scores below the bound
   float list[NW][64];   // bucket members, one region per wave
   float redf[2 * NW];
   int redi[2 * NW];
@@ -572,7 +578,7 @@ __global__ void __launch_bounds__(64 * NW) topk_block_kernel(const TopkParams p)
   static_assert(IPL % kGroup == 0, "items come in whole groups");
   constexpr int NG = IPL / kGroup;
   constexpr int SEG = 64 * IPL;
-  constexpr int kSub = 8;
+  constexpr int kSub = 32 / NW;  // 2048 subsets in the workgroup: a bound for every top-k up to 2048
   static_assert(kGroup % kSub == 0, "every group feeds every subset");
   __shared__ BlockLds<NW> sm;
   int *hist = sm.hist;
@@ -693,7 +699,7 @@ __global__ void __launch_bounds__(64 * NW) topk_block_kernel(const TopkParams p)
       __syncthreads();
       int bsel, above;
       find_bucket<kBlockBins>(hist, r, bsel, above);
-      m = hist[bsel];
+      m = __builtin_amdgcn_readfirstlane(hist[bsel]);
       r -= above;
       const uint32_t bsel_bits = kBinBits + (uint32_t)bsel;
       fence_values(x, ng);
@@ -769,7 +775,7 @@ __global__ void __launch_bounds__(64 * NW) topk_block_kernel(const TopkParams p)
     __syncthreads();
     int bsel, above;
     find_bucket<kBlockBins>(hist, r, bsel, above);
-    m = hist[bsel];
+    m = __builtin_amdgcn_readfirstlane(hist[bsel]);
     r -= above;
     fence_values(x, ng);
     float mlo = INFINITY, mhi = -INFINITY;
@@ -909,6 +915,18 @@ constexpr int64_t kTopkOnePass = 32768;  // the longest row (or segment) one ker
 // One launch over rows (segment mode: segments) of up to kTopkOnePass columns.
 static int topk_run(const TopkParams &p, hipStream_t st) {
   const int64_t len = p.nseg > 1 ? p.seg_len : p.row_len;
+  // Few rows leave compute units idle at one wave (or 4 or 8 waves) per row, and
+  // a row's time is one wave's passes over its 64 to 128 items per lane: spread
+  // such rows over more waves.  16 rows, top-2048: 4096 columns 10.8 -> 6.2 us,
+  // 8192 18.3 -> 7.6, 16384 12.7 -> 10.5, 32768 15.9 -> 14.3.  The lines lie where
+  // the rows fill the chip either way: 1024 rows of 8192 still 20.5 -> 15.4, 2048
+  // rows of 4096 16.2 -> 15.5; 512 rows of 16384 15.2 -> 15.9.
+  if (len > 2048 && p.rows <= (len <= 8192 ? 1024 : 256)) {
+    if (len <= 4096) return launch_topk_block<4, 16>(p, st);
+    if (len <= 8192) return launch_topk_block<8, 16>(p, st);
+    if (len <= 16384) return launch_topk_block<16, 16>(p, st);
+    if (len <= kTopkOnePass) return launch_topk_block<16, 32>(p, st);
+  }
   // causal rows longer than 8192 columns: the rows whose window still fits
   // 8192 columns (t < 8192 - causal_offset in each batch) take one wave per
   // row instead of a workgroup whose later waves would hold no column
