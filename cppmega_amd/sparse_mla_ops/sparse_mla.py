@@ -23,7 +23,7 @@ import logging
 import torch
 
 from ._common import unwrap_quantized
-from .sparse_mla_bwd import build_inverse_index, side_stream, sparse_mla_bwd
+from .sparse_mla_bwd import sparse_mla_bwd
 from .sparse_mla_bwd_fp8 import sparse_mla_bwd_fp8
 from .sparse_mla_fwd import sparse_mla_fwd_interface
 from .sparse_mla_fwd_fp8 import _enforce_te_tensorwise_quant_backend, per_token_cast_to_fp8, \
@@ -66,16 +66,7 @@ class SparseMLA(torch.autograd.Function):
         ctx.scaling = scaling
         if d_v is None:
             d_v = q.shape[-1]
-        # the backward's inverse index depends on the indices alone: build it on a
-        # second stream while the forward kernel runs (the forward is queued
-        # first; the build waits only for the work before it)
-        need_index = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
-        ready = torch.cuda.Event() if need_index else None
-        if ready is not None:
-            ready.record()
         out, lse = sparse_mla_fwd_interface(q, kv, indices, sm_scale=scaling, d_v=d_v)
-        ctx.inverse_index = (build_inverse_index(q, kv, indices, d_v, stream=side_stream(q.device), after=ready)
-                             if need_index else None)
         ctx.d_v = d_v
         ctx.save_for_backward(q, kv, indices, out, lse)
         return out, lse
@@ -83,9 +74,12 @@ class SparseMLA(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output, grad_lse):
         q, kv, indices, out, lse = ctx.saved_tensors
-        dq, dkv = sparse_mla_bwd(q, kv, out, grad_output.contiguous(), indices, lse, sm_scale=ctx.scaling,
-                                 inverse_index=ctx.inverse_index)
-        ctx.inverse_index = None
+        # The backward builds its inverse index in the same call.  Built during the forward on
+        # a second stream it bought nothing (B 2, S 4096, 32 heads, top-256: 343 us a step either
+        # way, the build and the forward slowing each other), held 21 MB per layer until the
+        # backward, and cost the host more than the kernels of a small call (B 1, S 512, 16
+        # heads, top-64: 154 us a step, now 105).
+        dq, dkv = sparse_mla_bwd(q, kv, out, grad_output.contiguous(), indices, lse, sm_scale=ctx.scaling)
         return dq, dkv, None, None, None
 
 
@@ -135,14 +129,8 @@ class SparseMLA_FP8(torch.autograd.Function):
             k8 = k8_flat.reshape(kv.shape)
             kv_scale = ks_flat.reshape(kv.shape[:-2])
 
-        need_index = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
-        ready = torch.cuda.Event() if need_index else None
-        if ready is not None:
-            ready.record()
         out, lse = sparse_mla_fwd_fp8_interface(q8, k8, indices, q_scale=q_scale, kv_scale=kv_scale,
                                                 sm_scale=scaling, d_v=d_v)
-        ctx.inverse_index = (build_inverse_index(q8, k8, indices, d_v, stream=side_stream(q8.device), after=ready)
-                             if need_index else None)
         ctx.d_v = d_v
         ctx.save_for_backward(q8, k8, q_scale, kv_scale, indices, out, lse)
         return out, lse
@@ -151,8 +139,7 @@ class SparseMLA_FP8(torch.autograd.Function):
     def backward(ctx, grad_output, grad_lse):
         q8, k8, q_scale, kv_scale, indices, out, lse = ctx.saved_tensors
         dq, dkv = sparse_mla_bwd_fp8(q8, k8, q_scale, kv_scale, out, grad_output.contiguous(), indices, lse,
-                                     sm_scale=ctx.scaling, inverse_index=ctx.inverse_index)
-        ctx.inverse_index = None
+                                     sm_scale=ctx.scaling)
         return dq, dkv, None, None, None
 
 
