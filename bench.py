@@ -11,8 +11,8 @@ HBM before timing.  Prints one JSON line (see the fields below).
 
 The backward is three stages (inverse index, main kernel, dKV reduction).  The
 inverse index depends on the indices alone, so the step builds it before the
-forward (build_inverse_index; in training SparseMLA.apply builds it on a second
-stream instead, overlapping the layers that follow) and the backward call runs
+forward (build_inverse_index; in training the autograd function's backward builds
+it in its own call) and the backward call runs
 the main kernel and the reduction; their durations come from HIP events the
 library records on its stream during the timed steps (dsa_stage_timing), the
 inverse index's from events around its build.  The roofline object is
@@ -579,12 +579,10 @@ def main():
         sel = topk_indices(scores, TOPK, causal=True)
         if record:
             marks[2].record()
-        # the backward's inverse index depends on the indices alone.  In a training
-        # step SparseMLA.apply builds it on a second stream, overlapping the layers
-        # that follow the forward; in this isolated layer step nothing follows, and
-        # run beside the forward it stretches the forward by more than it takes
-        # alone (measured: 344-352 us with the overlap, 339 us in order, for
-        # build + forward + backward), so it is built first, in order (marks 5, 6)
+        # the backward's inverse index depends on the indices alone: it is built first,
+        # in order (marks 5, 6).  Run beside the forward it stretches the forward by
+        # more than it takes alone (measured: 344-352 us with the overlap, 339 us in
+        # order, for build + forward + backward)
         if record:
             marks[5].record()
         inv = build_inverse_index(q, kv, idx, D_V)
