@@ -96,19 +96,23 @@ def build_inverse_index(q, kv, indices, d_v, *, fp32_partials=None, stream=None,
         return None
     cur = torch.cuda.current_stream(q.device)
     side = stream if stream is not None else cur
-    buf = torch.empty(n, dtype=torch.uint8, device=q.device)
     if side != cur:
         if after is not None:
             side.wait_event(after)
         else:
             side.wait_stream(cur)
+    # Allocated on the stream that writes it: the current stream's pool may hand out a block
+    # that work queued there since ``after`` (a forward's workspace, freed when the call
+    # returned) still uses, and the build does not wait for that work.
+    with torch.cuda.stream(side):
+        buf = torch.empty(n, dtype=torch.uint8, device=q.device)
     rc = L.dsa_sparse_mla_bwd_build_index(indices.data_ptr(), B, S, S_kv, H, G, D, int(d_v), topk, flags, cap,
                                           buf.data_ptr(), n, side.cuda_stream)
     _lib.check(rc, "dsa_sparse_mla_bwd_build_index")
     event = None
     if side != cur:
         if not torch.cuda.is_current_stream_capturing():  # a capture keeps its pool alive itself
-            buf.record_stream(side)
+            buf.record_stream(cur)
             indices.record_stream(side)
         event = torch.cuda.Event()
         event.record(side)
