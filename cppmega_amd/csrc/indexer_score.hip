@@ -141,7 +141,8 @@ __device__ __forceinline__ void idx_segment(const IdxParams &p, unsigned char (&
   // holding channels [16 g32, +16) and [32 + 16 g32, +16) of each 64-channel chunk
   typedef typename std::conditional<FP8, i32x8, bf16x8>::type aop_t;
   aop_t A[C::MT][C::KSTEPS];
-  const int64_t wave_tok0 = t0 + (p.split ? 0 : w * C::TPW);
+  const bool split = !WIN && p.split != 0;  // (window mode never splits)
+  const int64_t wave_tok0 = t0 + (split ? 0 : w * C::TPW);
 #pragma unroll
   for (int m = 0; m < C::MT; ++m) {
     const int r = m * 32 + l32;
@@ -230,7 +231,7 @@ __device__ __forceinline__ void idx_segment(const IdxParams &p, unsigned char (&
     const int tl = C::TPW >= 2 ? 2 * j + g32 : 0;
     soff_lane[j] = (uint32_t)(((wave_tok0 + tl - t0) * p.Sk + k0 + l32) * 4);
   }
-  const bool wave_in_sq = wave_tok0 + C::TPW - 1 < p.Sq && !p.split;  // split: sub-tiles are picked below
+  const bool wave_in_sq = wave_tok0 + C::TPW - 1 < p.Sq && !split;  // split: sub-tiles are picked below
 
   // window mode: this wave's token windows (wave-uniform scalar loads) and
   // their union; sub-tiles outside the union are not computed
@@ -300,7 +301,7 @@ __device__ __forceinline__ void idx_segment(const IdxParams &p, unsigned char (&
         const int64_t sn = tk + sub * 32;
         // wave-uniform: the sub-tile exists and is not wholly above this wave's
         // diagonal (lower-triangle mode) or outside its windows (window mode)
-        const bool active = sn < k_end && !(p.split && ((it * C::SUBS + sub) & 3) != w) && !(p.causal == 2 && sn > wave_tok_last + p.coff) &&
+        const bool active = sn < k_end && !(split && ((it * C::SUBS + sub) & 3) != w) && !(p.causal == 2 && sn > wave_tok_last + p.coff) &&
                             !(win && (sn + 32 <= wmin || sn >= wmax));
         const int64_t s = sn + l32;
         float mv[C::TPW];  // window mode: the additive mask, loaded ahead of the MFMAs
