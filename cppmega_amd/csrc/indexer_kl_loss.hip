@@ -490,8 +490,11 @@ struct PassCfg {
 };
 
 // LOSS: the KL partial sums; GRAD: P (p.grad, or the sparse state's p.pc) and the
-// R partial sums.
-template <int D, int NW, bool LOSS, bool GRAD>
+// R partial sums.  FAR: a wave's 32 query rows, B * H * D * 2 bytes apart, span more
+// than the 4 GiB that the DMA's 32-bit offsets reach (a batch of several thousand
+// short sequences): each lane reads its row as operands by 64-bit addresses, one
+// sub-tile's products after the other.
+template <int D, int NW, bool LOSS, bool GRAD, bool FAR>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4))) kl_pass_kernel(Params p) {
   using C = Cfg<D, NW>;
   using PC = PassCfg<D, NW>;
@@ -547,7 +550,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
 #pragma unroll
   for (int i = 0; i < PC::QP; ++i) {
     const int u = 64 * i + lane, r = u / C::CPR;
-    qo[i] = (uint32_t)r * qpitch + (uint32_t)(((u - r * C::CPR) ^ PC::swz(r)) * 16);
+    qo[i] = (uint32_t)r * qpitch + (uint32_t)(((u - r * C::CPR) ^ PC::swz(r)) * 16);  // (not FAR: below 4 GiB)
   }
 #pragma unroll
   for (int i = 0; i < PC::KP; ++i) {
@@ -573,8 +576,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
   };
   auto key_rs = [&](int h) { return make_buffer_words(kbase + h / hpg * C::ROWB, kbytes); };
   auto query_rs = [&](int h) { return make_buffer_words(qb + h * C::ROWB, qbytes); };
-  constexpr int NF = PC::KP + PC::QP;  // loads per head
-  bool all_on = true, any_on = false;  // wave-uniform
+  constexpr int NF = PC::KP + (FAR ? 0 : PC::QP);  // loads per head
+  bool all_on = !FAR, any_on = false;  // wave-uniform
 #pragma unroll
   for (int sub = 0; sub < C::SUBS; ++sub) {
     all_on = all_on && sub_on[sub];
@@ -601,7 +604,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
     const unsigned char *ks = smem + (h & 1) * C::KC * C::ROWB;
     bf16x8 Q[C::KSTEPS];
 #pragma unroll
-    for (int k = 0; k < C::KSTEPS; ++k) Q[k] = operand(smem + PC::OFF_Q + w * 32 * C::ROWB, 0, k);
+    for (int k = 0; k < C::KSTEPS; ++k)
+      if constexpr (!FAR) Q[k] = operand(smem + PC::OFF_Q + w * 32 * C::ROWB, 0, k);
+    if constexpr (FAR) load_q_operand<D>(p, b, h, t, Q);
     const float bh = bn;
     const int hn = h + 1 < H ? h + 1 : h;  // (past the last head: its own again, unused)
     bn = beta_bt[(int64_t)hn * p.Sq];
@@ -992,6 +997,16 @@ static Layout layout(int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t D, in
   return L;
 }
 
+template <int D, int NW, bool LOSS, bool GRAD, bool FAR>
+static int launch_pass(const Params &p, int64_t items, hipStream_t st) {
+  const auto pass = kl_pass_kernel<D, NW, LOSS, GRAD, FAR>;
+  constexpr int lds = PassCfg<D, NW>::BYTES;
+  const hipError_t e = hipFuncSetAttribute((const void *)pass, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return set_error(DSA_ERR_HIP, "kl_pass_kernel: LDS attribute: %s", hipGetErrorString(e));
+  hipLaunchKernelGGL(pass, dim3((unsigned)items), dim3(64 * NW), lds, st, p);
+  return check_launch("kl_pass_kernel");
+}
+
 template <int D, int NWS, int NWP, bool LOSS, bool GRAD>
 static int launch_mfma(const Params &p, hipStream_t st) {
   using CS = Cfg<D, NWS>;
@@ -1008,12 +1023,9 @@ static int launch_mfma(const Params &p, hipStream_t st) {
     q.NI += (lt < p.Sk - 1 ? lt : p.Sk - 1) / CP::KC + 1;
   }
   const int64_t items = (p.B * q.NI + 7) / 8 * 8;
-  const auto pass = kl_pass_kernel<D, NWP, LOSS, GRAD>;
-  constexpr int lds = PassCfg<D, NWP>::BYTES;
-  const hipError_t e = hipFuncSetAttribute((const void *)pass, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if (e != hipSuccess) return set_error(DSA_ERR_HIP, "kl_pass_kernel: LDS attribute: %s", hipGetErrorString(e));
-  hipLaunchKernelGGL(pass, dim3((unsigned)items), dim3(CP::NT), lds, st, q);
-  rc = check_launch("kl_pass_kernel");
+  const int64_t rows = p.Sq < 32 ? p.Sq : 32;  // of a wave
+  const bool far = (rows - 1) * p.B * p.H * CP::ROWB + CP::ROWB > (int64_t)0xffffffff;
+  rc = far ? launch_pass<D, NWP, LOSS, GRAD, true>(q, items, st) : launch_pass<D, NWP, LOSS, GRAD, false>(q, items, st);
   if (rc) return rc;
   if (p.pc != nullptr) {
     hipLaunchKernelGGL(kl_rows_state_kernel<D>, dim3((unsigned)((p.B * p.Sq + 3) / 4)), dim3(kNT), 0, st, p);
