@@ -880,7 +880,8 @@ __global__ void __launch_bounds__(kNT) kl_rows_state_kernel(Params p) {
   }
   if (lane == 0) {
     p.rows[row] = nan_row ? __builtin_nanf("") : kl * kLn2;
-    p.flag[row] = nan_row ? __builtin_nanf("") : 0.0f;
+    // (a NaN P, from any head, makes kl and R NaN, and with R every column's gradient)
+    p.flag[row] = nan_row || kl != kl ? __builtin_nanf("") : 0.0f;
   }
   for (int e = lane; e < n; e += 64) {
     const float q = exp2_fast(fmaf(x[e], kLog2e, -gam));
