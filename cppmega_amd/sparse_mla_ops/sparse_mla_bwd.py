@@ -111,9 +111,10 @@ def build_inverse_index(q, kv, indices, d_v, *, fp32_partials=None, stream=None,
     _lib.check(rc, "dsa_sparse_mla_bwd_build_index")
     event = None
     if side != cur:
-        if not torch.cuda.is_current_stream_capturing():  # a capture keeps its pool alive itself
-            buf.record_stream(cur)
-            indices.record_stream(side)
+        # also in a capture, whose pool would hand a freed block to the next build while an
+        # earlier backward still reads it on replay (recorded blocks stay out until its end)
+        buf.record_stream(cur)
+        indices.record_stream(side)
         event = torch.cuda.Event()
         event.record(side)
     return InverseIndex(buf, event, (B, S, S_kv, H, G, D, int(d_v), topk, flags, cap, indices.data_ptr()))
@@ -137,7 +138,9 @@ def _launch_bwd(q, kv, o, do, indices, lse, delta, sm_scale, dtype_code, q_scale
             raise ValueError(f"inverse_index was built for another call: built for {inverse_index.key}, "
                              f"called with {key} (B, S, S_kv, H, G, D, d_v, topk, flags, pass_bytes, indices)")
         if inverse_index.event is not None:
-            torch.cuda.current_stream(q.device).wait_event(inverse_index.event)
+            cur = torch.cuda.current_stream(q.device)
+            cur.wait_event(inverse_index.event)
+            inverse_index.buf.record_stream(cur)
         ws_bytes = int(L.dsa_sparse_mla_bwd_indexed_workspace_size(B, S, S_kv, H, G, D, d_v, topk, flags, cap))
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device)
         ix = inverse_index.buf
