@@ -38,6 +38,7 @@ EXPORTED_SYMBOLS = (
     "dsa_sparse_mla_fwd_workspace_size",
     "dsa_sparse_mla_fwd_call_workspace_size",
     "dsa_sparse_mla_fwd_ws",
+    "dsa_sparse_mla_fwd_call",
     "dsa_sparse_mla_bwd_workspace_size",
     "dsa_sparse_mla_bwd_index_size",
     "dsa_sparse_mla_bwd_indexed_workspace_size",
@@ -93,6 +94,9 @@ _SIGNATURES = {
     "dsa_sparse_mla_fwd_ws": (_i32, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                      _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                      _f32, _i32, _c_void_p, _c_void_p, _c_void_p, _size_t, _c_void_p]),
+    "dsa_sparse_mla_fwd_call": (_i32, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+                                       _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+                                       _f32, _i32, _c_void_p, _c_void_p, _c_void_p, _size_t, _c_void_p]),
     "dsa_sparse_mla_bwd_workspace_size": (_size_t, [_i64] * 8 + [_i32, _u64]),
     "dsa_sparse_mla_bwd_index_size": (_size_t, [_i64] * 8 + [_i32, _u64]),
     "dsa_sparse_mla_bwd_indexed_workspace_size": (_size_t, [_i64] * 8 + [_i32, _u64]),

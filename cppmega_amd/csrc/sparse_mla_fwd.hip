@@ -597,5 +597,17 @@ extern "C" int dsa_sparse_mla_fwd_ws(const void *q, const void *kv, const int32_
   const size_t need = dsa_sparse_mla_fwd_workspace_size(B, S_kv, G, D_qk, D_v, dtype);
   DSA_REQUIRE(need == 0 || workspace, "dsa_sparse_mla_fwd_ws: null workspace (%zu bytes required)", need);
   return sparse_mla_fwd_impl(q, kv, indices, out, lse2, B, S, S_kv, H, G, D_qk, D_v, topk, sm_scale, dtype, q_scale,
-                             kv_scale, need || dtype == DSA_DTYPE_BF16 ? workspace : nullptr, workspace_bytes, stream);
+                             kv_scale, need ? workspace : nullptr, workspace_bytes, stream);
+}
+
+extern "C" int dsa_sparse_mla_fwd_call(const void *q, const void *kv, const int32_t *indices, void *out, float *lse2,
+                                       int64_t B, int64_t S, int64_t S_kv, int64_t H, int64_t G, int64_t D_qk,
+                                       int64_t D_v, int64_t topk, float sm_scale, int dtype, const float *q_scale,
+                                       const float *kv_scale, void *workspace, size_t workspace_bytes, void *stream) {
+  if (dtype != DSA_DTYPE_BF16)
+    return dsa_sparse_mla_fwd_ws(q, kv, indices, out, lse2, B, S, S_kv, H, G, D_qk, D_v, topk, sm_scale, dtype, q_scale,
+                                 kv_scale, workspace, workspace_bytes, stream);
+  DSA_REQUIRE(((uintptr_t)workspace & 15) == 0, "dsa_sparse_mla_fwd_call: workspace not 16-byte aligned");
+  return sparse_mla_fwd_impl(q, kv, indices, out, lse2, B, S, S_kv, H, G, D_qk, D_v, topk, sm_scale, dtype, q_scale,
+                             kv_scale, workspace, workspace_bytes, stream);
 }

@@ -29,11 +29,11 @@ def _launch_fwd(q, kv, indices, sm_scale, d_v, dtype_code, q_scale=None, kv_scal
     # e4m3: the V rows dequantised to bf16 once per call; bf16, few tokens: the results of splits of the slots
     ws_bytes = int(L.dsa_sparse_mla_fwd_call_workspace_size(B, S, S_kv, H, G, D, d_v, topk, dtype_code))
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device) if ws_bytes else None
-    rc = L.dsa_sparse_mla_fwd_ws(
+    rc = L.dsa_sparse_mla_fwd_call(
         q.data_ptr(), kv.data_ptr(), indices.data_ptr(), out.data_ptr(), lse.data_ptr(),
         B, S, S_kv, H, G, D, d_v, topk, float(sm_scale), dtype_code,
         _lib.ptr(q_scale), _lib.ptr(kv_scale), _lib.ptr(ws), ws_bytes, stream)
-    _lib.check(rc, "dsa_sparse_mla_fwd_ws")
+    _lib.check(rc, "dsa_sparse_mla_fwd_call")
     return out, lse
 
 

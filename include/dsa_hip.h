@@ -101,12 +101,16 @@ int dsa_sparse_mla_fwd(const void *q, const void *kv, const int32_t *indices,
  * B * S_kv * G * D_v bf16, 0 for the d_qk = 576 kernels, which keep converting
  * V in LDS; MXFP8: B * S_kv * G * D_qk bf16 plus 256; bf16 input: 0, and then
  * `workspace` may be NULL).  Replaces the same reference interfaces as
- * dsa_sparse_mla_fwd.
- * dsa_sparse_mla_fwd_call_workspace_size returns the bytes the whole call can
- * use: the same for e4m3 and MXFP8; for bf16 input with too few tokens to fill
- * the GPU, room for the results of several workgroups per (token, head) that
- * share its slots.  Given a smaller workspace (or none), a bf16 call runs
- * unsplit.
+ * dsa_sparse_mla_fwd.  A bf16 call neither reads nor writes `workspace`.
+ *
+ * dsa_sparse_mla_fwd_call is the same call for a caller that gives bf16 input a
+ * workspace too.  dsa_sparse_mla_fwd_call_workspace_size returns the bytes it can
+ * use: those of dsa_sparse_mla_fwd_workspace_size for e4m3 and MXFP8; for bf16
+ * input with too few tokens to fill the GPU, room for the results of several
+ * workgroups per (token, head) that share its slots.  Given a smaller workspace
+ * (or NULL), a bf16 call runs unsplit.  The contents belong to one call from its
+ * launch to its end: two calls that may run at the same time (on two streams)
+ * need a workspace each.  It is 16-byte aligned for bf16 input.
  */
 size_t dsa_sparse_mla_fwd_workspace_size(int64_t B, int64_t S_kv, int64_t G,
                                          int64_t D_qk, int64_t D_v, int dtype);
@@ -119,6 +123,12 @@ int dsa_sparse_mla_fwd_ws(const void *q, const void *kv, const int32_t *indices,
                           int64_t D_v, int64_t topk, float sm_scale, int dtype,
                           const float *q_scale, const float *kv_scale,
                           void *workspace, size_t workspace_bytes, void *stream);
+int dsa_sparse_mla_fwd_call(const void *q, const void *kv, const int32_t *indices,
+                            void *out, float *lse2, int64_t B, int64_t S,
+                            int64_t S_kv, int64_t H, int64_t G, int64_t D_qk,
+                            int64_t D_v, int64_t topk, float sm_scale, int dtype,
+                            const float *q_scale, const float *kv_scale,
+                            void *workspace, size_t workspace_bytes, void *stream);
 
 /* dsa_sparse_mla_bwd flags */
 enum dsa_bwd_flags {

@@ -109,3 +109,37 @@ def test_wide_forward_split_matches_unsplit(dev):
                                     torch.cuda.current_stream().cuda_stream), "dsa_sparse_mla_fwd")
     torch.testing.assert_close(out.float(), out1.float(), rtol=2 ** -7, atol=2 ** -7)
     torch.testing.assert_close(lse, lse1, rtol=1e-5, atol=1e-4)
+
+
+def test_bf16_workspace_is_used_only_where_offered_for_splits(dev):
+    """dsa_sparse_mla_fwd_ws neither reads nor writes a bf16 caller's workspace (one buffer
+    may serve several streams); dsa_sparse_mla_fwd_call splits with a large enough one only,
+    and refuses a misaligned one."""
+    from cppmega_amd import _lib
+    B, S, S_kv, H, topk, DV = 4, 1, 700, 128, 512, 512
+    g = torch.Generator().manual_seed(4)
+    q = (torch.randn((B, S, H, D), generator=g) * 0.5).to(torch.bfloat16).to(dev)
+    kv = (torch.randn((B, S_kv, 1, D), generator=g) * 0.5).to(torch.bfloat16).to(dev)
+    idx = torch.rand((B, S, 1, S_kv), generator=g).argsort(dim=-1)[..., :topk].to(torch.int32).contiguous().to(dev)
+    L, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    n = int(L.dsa_sparse_mla_fwd_call_workspace_size(B, S, S_kv, H, 1, D, DV, topk, _lib.DTYPE_BF16))
+    assert n > 0
+
+    def call(fn, ws, nbytes):
+        out = torch.empty((B, S, H, DV), dtype=torch.bfloat16, device=dev)
+        lse = torch.empty((B, S, H), device=dev)
+        rc = fn(q.data_ptr(), kv.data_ptr(), idx.data_ptr(), out.data_ptr(), lse.data_ptr(), B, S, S_kv, H, 1, D, DV, topk,
+                D ** -0.5, _lib.DTYPE_BF16, None, None, ws, nbytes, st)
+        return rc, out, lse
+
+    ws = torch.full((n + 16,), 0x5a, dtype=torch.uint8, device=dev)
+    rc, out, lse = call(L.dsa_sparse_mla_fwd_ws, ws.data_ptr(), n)
+    assert rc == _lib.DSA_OK and bool((ws == 0x5a).all())
+    for p, nbytes in ((ws.data_ptr(), n - 1), (None, 0)):           # too small, none: unsplit
+        rc, o, l = call(L.dsa_sparse_mla_fwd_call, p, nbytes)
+        assert rc == _lib.DSA_OK and torch.equal(o, out) and torch.equal(l, lse)
+    assert bool((ws == 0x5a).all())
+    assert call(L.dsa_sparse_mla_fwd_call, ws.data_ptr() + 4, n)[0] == _lib.DSA_ERR_INVALID_ARG
+    rc, o, l = call(L.dsa_sparse_mla_fwd_call, ws.data_ptr(), n)
+    assert rc == _lib.DSA_OK and not bool((ws[:n] == 0x5a).all()) and bool((ws[n:] == 0x5a).all())
+    torch.testing.assert_close(o.float(), out.float(), rtol=2 ** -7, atol=2 ** -7)
