@@ -101,7 +101,7 @@ struct Params {
   int32_t *cpre;                  // [B, Sq, NC + 2] set columns before each key chunk, all, and those at or below the diagonal
   float *pc;                      // [B, Sq, K]   P, then v
   float *xc;                      // [B, Sq, K]   index score
-  float *flag;                    // [B, Sq]      NaN for a row whose loss is NaN, else 0
+  float *flag;                    // [B, Sq]      NaN for a row whose loss is not finite, else 0
   int64_t B, Sq, Sk, H, G, K, W, NC;
   int KC;                         // keys per chunk
   int64_t NI;                     // KL work items per batch (block, chunk pairs)
@@ -880,8 +880,9 @@ __global__ void __launch_bounds__(kNT) kl_rows_state_kernel(Params p) {
   }
   if (lane == 0) {
     p.rows[row] = nan_row ? __builtin_nanf("") : kl * kLn2;
-    // (a NaN P, from any head, makes kl and R NaN, and with R every column's gradient)
-    p.flag[row] = nan_row || kl != kl ? __builtin_nanf("") : 0.0f;
+    // a NaN or infinite P, from any head, makes R so, and 0 * R (Q is 0 outside the
+    // set) every other column's gradient NaN
+    p.flag[row] = nan_row || !(fabsf(R) < INFINITY) ? __builtin_nanf("") : 0.0f;
   }
   for (int e = lane; e < n; e += 64) {
     const float q = exp2_fast(fmaf(x[e], kLog2e, -gam));

@@ -57,11 +57,12 @@ def test_state_gradient_matches_direct(dev, b, sq, sk, np_, hn, topk, sparse):
         assert float((got - direct).abs().max()) <= 2 * bound * float(direct.abs().max())
 
 
+@pytest.mark.parametrize("value", ["nan", "inf"])
 @pytest.mark.parametrize("where", ["query", "key"])
-def test_nan_in_one_head_makes_the_row_nan(dev, where):
-    """A row whose loss is NaN has a NaN gradient over all its columns, those outside its
-    top-k set too, whichever head the NaN comes from (query: row 40; key: the rows that
-    pick key 30)."""
+def test_nan_or_inf_in_one_head_makes_the_row_nan(dev, where, value):
+    """A row whose loss is not finite has a NaN gradient over all its columns, those outside
+    its top-k set too, whichever head the NaN or infinity comes from (query: row 40; key:
+    the rows that pick key 30, of an infinite key those it scores +inf: -inf is no weight)."""
     b, s, np_, hn, topk = 2, 70, 3, 64, 12
     g = torch.Generator().manual_seed(9)
     z = torch.randn((b, s, s), generator=g).masked_fill_(torch.ones(s, s, dtype=torch.bool).triu(1), -torch.inf).to(dev)
@@ -69,20 +70,22 @@ def test_nan_in_one_head_makes_the_row_nan(dev, where):
     query = torch.randn((s, b, np_, hn), generator=g).to(torch.bfloat16).to(dev)
     key = torch.randn((s, b, np_, hn), generator=g).to(torch.bfloat16).to(dev)
     if where == "query":
-        query[40, 1, 2, 5] = torch.nan
+        query[40, 1, 2, 5] = float(value)
         bad = torch.zeros((b, s), dtype=torch.bool, device=dev)
         bad[1, 40] = True
     else:
-        key[30, 1, 1, 7] = torch.nan
+        key[30, 1, 1, 7] = float(value)
         bad = ((idx == 30).any(-1)) & (torch.arange(s, device=dev) >= 30)
         bad[0] = False
+        if value == "inf":
+            bad[1] &= query[:, 1, 1, 7] > 0
         assert 0 < int(bad.sum()) < s - 30
     with torch.no_grad():
         _, rows = indexer_kl_loss(z, idx, query, key, hn ** -0.5, 1.0, True, return_rows=True)
-    assert torch.equal(rows.isnan(), bad)
+    assert torch.equal(~rows.isfinite(), bad)
     zr = z.clone().requires_grad_()
     loss = indexer_kl_loss(zr, idx, query, key, hn ** -0.5, 1.0, True)
-    assert bool(loss.isnan())
+    assert not bool(loss.isfinite())
     grad, = torch.autograd.grad(loss, zr)
     assert torch.equal(grad.isnan(), bad[..., None].expand_as(grad))
     assert torch.equal(indexer_kl_loss_backward(1.0, z, idx, query, key, hn ** -0.5, 1.0, True).isnan(), grad.isnan())
