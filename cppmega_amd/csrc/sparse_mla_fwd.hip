@@ -503,8 +503,8 @@ static int sparse_mla_fwd_impl(const void *q, const void *kv, const int32_t *ind
     pe.gate_run = 0;
     if (wide_shape(D_qk, D_v)) {
       const WideFwdPlan pl = wide_fwd_plan(B * S * G, p.hpg, D_v, topk, false);
-      rc = pl.nt > 0 ? launch_fwd_wide_bf16(pe, D_qk, D_v, pl.nt, true, st)
-                     : launch_fwd_wide(pe, D_qk, D_v, false, st, false, true);
+      rc = pl.piped ? launch_fwd_wide_bf16(pe, D_qk, D_v, pl.nt, true, st)
+                    : launch_fwd_wide(pe, D_qk, D_v, pl.nt, false, st, false, true);
     }
     else if (D_qk == 128 && D_v == 64) rc = launch_fwd_t<128, 64, false, false, false, true>(pe, st);
     else if (D_qk == 128) rc = launch_fwd_t<128, 128, false, false, false, true>(pe, st);
@@ -538,7 +538,7 @@ static int sparse_mla_fwd_impl(const void *q, const void *kv, const int32_t *ind
     if (D_qk == 128 && D_v == 64) return launch_fwd<128, 64, true, true>(p, st);
     if (D_qk == 128 && D_v == 128) return launch_fwd<128, 128, true, true>(p, st);
     if (D_qk == 192 && D_v == 128) return launch_fwd<192, 128, true, true>(p, st);
-    if (wide_shape(D_qk, D_v)) return launch_fwd_wide(p, D_qk, D_v, true, st, true);
+    if (wide_shape(D_qk, D_v)) return launch_fwd_wide(p, D_qk, D_v, 1, true, st, true);
     return set_error(DSA_ERR_UNSUPPORTED, "dsa_sparse_mla_fwd: no MXFP8 kernel for d_qk=%lld d_v=%lld",
                      (long long)D_qk, (long long)D_v);
   }
@@ -552,8 +552,8 @@ static int sparse_mla_fwd_impl(const void *q, const void *kv, const int32_t *ind
     } else if (need != 0) {
       pl = wide_fwd_plan(B * S * G, p.hpg, D_v, topk, false);
     }
-    return f8 || pl.nt == 0 ? launch_fwd_wide(p, D_qk, D_v, f8, st)
-                            : launch_fwd_wide_bf16(p, D_qk, D_v, pl.nt, false, st);
+    return f8 || !pl.piped ? launch_fwd_wide(p, D_qk, D_v, pl.nt, f8, st)
+                           : launch_fwd_wide_bf16(p, D_qk, D_v, pl.nt, false, st);
   }
   if (D_qk == 128 && D_v == 64) return f8 ? launch_fwd<128, 64, true>(p, st) : launch_fwd<128, 64, false>(p, st);
   if (D_qk == 128 && D_v == 128) return f8 ? launch_fwd<128, 128, true>(p, st) : launch_fwd<128, 128, false>(p, st);

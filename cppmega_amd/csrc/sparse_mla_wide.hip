@@ -345,29 +345,28 @@ static int launch_fwd_wide_nt(const FwdParams &p, hipStream_t st) {
 }
 
 // e4m3: two head tiles per workgroup when a kv group has at least 64 heads (the
-// gather and dequantisation of a block serve both), else one.  bf16: one (the
-// host sends larger groups to launch_fwd_wide_bf16).
+// gather and dequantisation of a block serve both), else one.  bf16: nt.
 template <int D_QK, int D_V, bool FP8, bool MX = false, bool QMX = false>
-static int launch_fwd_wide_t(const FwdParams &p, hipStream_t st) {
-  if constexpr (FP8) {
-    if (p.ntiles >= 2) return launch_fwd_wide_nt<D_QK, D_V, FP8, MX, 2, QMX>(p, st);
-  }
-  return launch_fwd_wide_nt<D_QK, D_V, FP8, MX, 1, QMX>(p, st);
+static int launch_fwd_wide_t(const FwdParams &p, int nt, hipStream_t st) {
+  return (FP8 ? p.ntiles : nt) >= 2 ? launch_fwd_wide_nt<D_QK, D_V, FP8, MX, 2, QMX>(p, st)
+                                    : launch_fwd_wide_nt<D_QK, D_V, FP8, MX, 1, QMX>(p, st);
 }
 
-int launch_fwd_wide(const FwdParams &p, int64_t d_qk, int64_t d_v, bool fp8, hipStream_t st, bool mx, bool qmx) {
+int launch_fwd_wide(const FwdParams &p, int64_t d_qk, int64_t d_v, int nt, bool fp8, hipStream_t st, bool mx, bool qmx) {
   if (qmx) {
-    if (d_qk == 576 && d_v == 512) return launch_fwd_wide_t<576, 512, false, false, true>(p, st);
+    if (d_qk == 576 && d_v == 512) return launch_fwd_wide_t<576, 512, false, false, true>(p, nt, st);
     return set_error(DSA_ERR_UNSUPPORTED, "sparse_mla_fwd(wide): no converted-Q kernel for d_qk=%lld d_v=%lld",
                      (long long)d_qk, (long long)d_v);
   }
   if (mx) {
-    if (d_qk == 576 && d_v == 512) return launch_fwd_wide_t<576, 512, true, true>(p, st);
+    if (d_qk == 576 && d_v == 512) return launch_fwd_wide_t<576, 512, true, true>(p, nt, st);
     return set_error(DSA_ERR_UNSUPPORTED, "sparse_mla_fwd(wide): no MXFP8 kernel for d_qk=%lld d_v=%lld",
                      (long long)d_qk, (long long)d_v);
   }
-  if (d_qk == 576 && d_v == 512) return fp8 ? launch_fwd_wide_t<576, 512, true>(p, st) : launch_fwd_wide_t<576, 512, false>(p, st);
-  if (d_qk == 576 && d_v == 576) return fp8 ? launch_fwd_wide_t<576, 576, true>(p, st) : launch_fwd_wide_t<576, 576, false>(p, st);
+  if (d_qk == 576 && d_v == 512)
+    return fp8 ? launch_fwd_wide_t<576, 512, true>(p, nt, st) : launch_fwd_wide_t<576, 512, false>(p, nt, st);
+  if (d_qk == 576 && d_v == 576)
+    return fp8 ? launch_fwd_wide_t<576, 576, true>(p, nt, st) : launch_fwd_wide_t<576, 576, false>(p, nt, st);
   return set_error(DSA_ERR_UNSUPPORTED, "sparse_mla_fwd(wide): no kernel for d_qk=%lld d_v=%lld", (long long)d_qk,
                    (long long)d_v);
 }

@@ -16,19 +16,20 @@ inline bool wide_shape(int64_t d_qk, int64_t d_v) { return d_qk == 576 && (d_v =
 // passes depend on it).
 inline bool wide_row(int64_t d_qk) { return d_qk == 576; }
 
-// Forward of bf16 rows, pipelined: head tiles per workgroup (0: the kernel of
-// launch_fwd_wide instead) and splits of the slots, and the launch (p.nsplit > 1:
-// p.part_o / p.part_ml hold the splits' results); qmx: Q converted from e4m3
-// codes and 32-channel block scales as it is loaded.
+// How a forward of bf16 rows runs: head tiles per workgroup, splits of the slots and
+// the kernel, launch_fwd_wide_bf16's (pipelined; nsplit > 1: p.part_o / p.part_ml hold
+// the splits' results) or launch_fwd_wide's.
 struct WideFwdPlan {
   int nt, nsplit;
+  bool piped;
 };
 WideFwdPlan wide_fwd_plan(int64_t tgs, int64_t hpg, int64_t d_v, int64_t topk, bool may_split);
+// qmx (here and below): Q converted from e4m3 codes and 32-channel block scales as it is loaded.
 int launch_fwd_wide_bf16(const FwdParams &p, int64_t d_qk, int64_t d_v, int nt, bool qmx, hipStream_t st);
 
-// Forward over all (token, kv group, 32-head tile) items: e4m3 rows (mx: with one
-// scale per 32 channels), or bf16 rows (qmx: as above).
-int launch_fwd_wide(const FwdParams &p, int64_t d_qk, int64_t d_v, bool fp8, hipStream_t st, bool mx = false,
+// Forward over all (token, kv group, nt 32-head tiles) items: e4m3 rows (mx: with one
+// scale per 32 channels; nt is chosen here), or bf16 rows.
+int launch_fwd_wide(const FwdParams &p, int64_t d_qk, int64_t d_v, int nt, bool fp8, hipStream_t st, bool mx = false,
                     bool qmx = false);
 // Backward main pass (P, dS and dQ, then the partial dKV rows at CSR positions); bf16 or e4m3.
 int launch_bwd_main_wide(const BwdParams &p, int64_t d_qk, int64_t d_v, bool fp8, bool f32p, hipStream_t st);

@@ -337,27 +337,72 @@ static int launch_wide_bf16(const FwdParams &p, hipStream_t st) {
   return check_launch("sparse_mla_fwd(wide combine)");
 }
 
-// tgs (token, kv group) pairs of hpg heads.  Head tiles per workgroup: as many as
-// the group has (d_v = 576: two, O's registers), since they share a block's rows
-// (s = 2048, h = 128, top-k 2048: 1358 us with four tiles, 1957 with two; h = 96:
-// 814 against 1165); a group of one tile takes launch_fwd_wide's kernel.
-// Too few workgroups for 256 compute units: the slots are split, at least four
-// blocks each; every split writes and the combination reads 2 KiB of fp32 O per
-// head, so past 8 splits the workgroups come from narrower head tiles instead
-// (16 tokens, h = 128, top-k 2048: 130 us before, 47 us as 4 tiles x 16 splits,
-// 39 us as 2 x 8; 1 token: 127 us before, 28 us as 1 x 16).
-WideFwdPlan wide_fwd_plan(int64_t tgs, int64_t hpg, int64_t d_v, int64_t topk, bool may_split) {
-  const int64_t ntiles = (hpg + 31) / 32, most = (topk + 31) / 32 / 4;
-  WideFwdPlan pl;
-  pl.nt = ntiles >= 3 && d_v == 512 ? 4 : (ntiles >= 2 ? 2 : 1);
-  pl.nsplit = 1;
-  const auto wanted = [&] { return 256 / (tgs * ((ntiles + pl.nt - 1) / pl.nt)); };
-  if (may_split && most > 1 && wanted() > 1) {
-    while (pl.nt > 1 && wanted() > 8) pl.nt /= 2;
-    pl.nsplit = (int)(wanted() < most ? wanted() : most);
+// Microseconds of one launch over tgs (token, kv group) pairs of hpg heads and nblk
+// blocks of 32 slots: a workgroup's prologue and epilogue and its time a block, each
+// with what 256 workgroups at once add to it, by the rounds that the grid takes on
+// 256 compute units.  Fitted to graph-replayed launches of 1 to 2048 tokens, 16 to
+// 256 heads, top-32 to top-2048 (the plan that it picks took 0.9% longer than the
+// best of the kernels over those, and at most 11% longer).
+//   kernel of launch_fwd_wide, one tile: the shortest prologue, and two workgroups
+//     share a compute unit (1 token, 128 heads, top-64: 8.8 us; pipelined, four
+//     tiles: 19.3); two tiles: half the gathers (100 tokens, 96 heads, top-64:
+//     13.7 us; one tile 14.7);
+//   pipelined, two or four tiles: a block's rows serve all of them (2048 tokens, 128
+//     heads, top-256: 304 us with four tiles, 371 with one, 394 with two; s = 2048,
+//     top-k 2048: 1358 us with four, 1957 with two);
+//   pipelined with split slots: the combination's launch and, per 2 KiB fp32 row
+//     that it reads, its traffic (16 tokens, 128 heads, top-2048: 40 us as two tiles
+//     x 8 splits, 49 as four x 16, 130 unsplit; 1 token: 28 us as one x 16, 127
+//     unsplit; but 64 tokens, 128 heads, top-256: 37 us as four x 2, 22 as one tile
+//     of the other kernel).
+static double wide_fwd_us(bool piped, int nt, int64_t nsplit, int64_t tgs, int64_t hpg, int64_t nblk) {
+  const int64_t tiles = (hpg + 31) / 32, wg = tgs * ((tiles + nt - 1) / nt) * nsplit;
+  const double per = (double)((nblk + nsplit - 1) / nsplit), x = (double)wg / 256;
+  if (nsplit > 1) {
+    const double rows = (double)(tgs * hpg * nsplit) / 4096;
+    if (nt == 1) return 11.0 + 1.46 * per + 1.9 * x + 3.8 * rows;
+    return nt == 2 ? 15.6 + 1.65 * per + 2.9 * x + 2.5 * rows : 19.0 + 2.1 * per + 3.0 * x + 2.5 * rows;
   }
-  if (pl.nt == 1 && pl.nsplit <= 1) pl.nt = 0;
-  return pl;
+  const int64_t full = wg / 256;
+  if (!piped && nt == 1) {
+    const auto round = [&](double y) {  // y * 256 workgroups, two of them on a compute unit past one each
+      if (y <= 0) return 0.0;
+      return y <= 1 ? 5.6 + 1.5 * y + (1.7 + 0.1 * y) * per : 8.0 + 2.3 * y + 2.36 * per;
+    };
+    if (x <= 2) return round(x);
+    // more rounds: they run into each other where a workgroup has few blocks
+    const int64_t two = full / 2;
+    const double flow = round(2) + (x / 2 - 1) * (9.2 + 1.86 * per), apart = (double)two * round(2) + round(x - 2 * (double)two);
+    return flow + (apart > flow ? apart - flow : 0.0) * (per < 32 ? per / 32 : 1.0);
+  }
+  const double f = piped ? (nt == 2 ? 10.0 : 4.7 + 2.6 * (double)(tiles < 4 ? tiles : 4)) : 8.3;
+  const double fx = nt == 2 ? 3.3 : 4.0, b = piped ? (nt == 2 ? 1.68 : 2.1) : 1.88, bx = piped ? 0.18 : 0.29;
+  const double rest = x - (double)full;
+  return (double)full * (f + fx + (b + bx) * per) + (rest > 0 ? f + fx * rest + (b + bx * rest) * per : 0.0);
+}
+
+// The kernel, head tiles per workgroup (at most two at d_v = 576: O's registers) and
+// splits of the slots, at least four blocks each and within one round, that take
+// the least time.
+WideFwdPlan wide_fwd_plan(int64_t tgs, int64_t hpg, int64_t d_v, int64_t topk, bool may_split) {
+  const int64_t ntiles = (hpg + 31) / 32, nblk = (topk + 31) / 32;
+  WideFwdPlan best{1, 1, false};
+  double us = wide_fwd_us(false, 1, 1, tgs, hpg, nblk);
+  const auto offer = [&](bool piped, int nt, int64_t nsplit) {
+    const double t = wide_fwd_us(piped, nt, nsplit, tgs, hpg, nblk);
+    if (t < us) {
+      us = t;
+      best = WideFwdPlan{nt, (int)nsplit, piped};
+    }
+  };
+  if (ntiles >= 2) offer(false, 2, 1);
+  for (int nt = 1; nt <= 4; nt *= 2) {
+    if (nt > 1 && (ntiles <= nt / 2 || (nt == 4 && d_v != 512))) break;
+    if (nt > 1) offer(true, nt, 1);
+    const int64_t wg = tgs * ((ntiles + nt - 1) / nt);
+    for (int64_t ns = 2; may_split && ns <= nblk / 4 && ns * wg <= 256; ++ns) offer(true, nt, ns);
+  }
+  return best;
 }
 
 int launch_fwd_wide_bf16(const FwdParams &p, int64_t d_qk, int64_t d_v, int nt, bool qmx, hipStream_t st) {

@@ -132,6 +132,20 @@ def test_bwd_workspace_bounded_by_pass_cap(lib):
     assert int(lib.dsa_sparse_mla_bwd_indexed_workspace_size(2, 4096, 4096, 32, 1, 128, 64, 256, 0, 0)) < one
 
 
+def test_wide_forward_splits_only_where_it_pays(lib):
+    """The wide bf16 forward splits a token's slots over workgroups (and asks for a
+    workspace of one fp32 row, m and l per head and split) where the tokens leave the
+    GPU idle and each split still has enough blocks: not for short rows, where the
+    combination costs more than the split saves."""
+    size = lambda B, S, H, topk, dv=512: int(lib.dsa_sparse_mla_fwd_call_workspace_size(
+        B, S, 8192, H, 1, 576, dv, topk, _lib.DTYPE_BF16))
+    assert size(16, 1, 128, 2048) == 16 * 128 * 8 * (512 + 2) * 4
+    assert size(1, 1, 128, 2048) == 128 * 16 * (512 + 2) * 4
+    assert size(1, 1, 16, 256) > 0
+    for B, S, H, topk in ((32, 1, 128, 256), (1, 64, 64, 256), (1, 100, 128, 256), (64, 1, 128, 512), (1, 300, 128, 2048)):
+        assert size(B, S, H, topk) == 0, (B, S, H, topk)
+
+
 def test_fused_indexer_topk_limits(lib):
     """The fused indexer + top-k's top-k bound per shape, and its refusals
     (unsupported shape, top-k past the bound, bad flags, null pointers)

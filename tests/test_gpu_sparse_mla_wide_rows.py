@@ -64,13 +64,18 @@ def test_wide_rows_e4m3_two_rows_per_entry(dev):
 
 
 @pytest.mark.parametrize("B,S,S_kv,H,G,DV,topk", [
-    (2, 1, 3000, 128, 1, 512, 2048),     # 16 splits of one head tile each
-    (20, 1, 600, 128, 1, 512, 513),      # two head tiles, splits of uneven blocks
-    (3, 7, 500, 96, 1, 512, 300),        # two head tiles of three (the last workgroup's second is empty)
-    (1, 40, 700, 128, 1, 512, 600),      # four head tiles
-    (1, 2, 600, 64, 2, 576, 290),        # kv groups, V the whole row
-    (1, 70, 300, 128, 1, 512, 200),      # four head tiles, no split
-    (1, 40, 300, 100, 1, 576, 100),      # two head tiles of four, no split
+    # the kernel, head tiles per workgroup x splits that the plan picks
+    (2, 1, 3000, 128, 1, 512, 2048),     # pipelined, 1 x 16
+    (20, 1, 600, 128, 1, 512, 513),      # pipelined, 1 x 3 of uneven blocks
+    (3, 7, 500, 96, 1, 512, 300),        # unpipelined, one tile of three
+    (1, 40, 700, 128, 1, 512, 600),      # pipelined, 2 x 3
+    (1, 2, 600, 64, 2, 576, 290),        # kv groups, V the whole row: pipelined, 1 x 2
+    (1, 70, 300, 128, 1, 512, 200),      # pipelined, two tiles, no split
+    (1, 40, 300, 100, 1, 576, 100),      # unpipelined, one tile of four, the last ragged
+    (1, 100, 300, 96, 1, 512, 70),       # unpipelined, two tiles of three (the last workgroup's second is empty)
+    (1, 50, 300, 200, 2, 576, 70),       # the same with kv groups, V the whole row
+    (1, 200, 300, 128, 1, 512, 40),      # pipelined, four tiles, no split
+    (4, 15, 2100, 100, 1, 512, 2048),    # pipelined, 4 x 4, the last tile ragged
 ])
 def test_wide_forward_splits(dev, B, S, S_kv, H, G, DV, topk):
     """Few tokens against a long kv: the slots of a token split over workgroups.
