@@ -101,10 +101,12 @@ def build_inverse_index(q, kv, indices, d_v, *, fp32_partials=None, stream=None,
             side.wait_event(after)
         else:
             side.wait_stream(cur)
-    # Allocated on the stream that writes it: the current stream's pool may hand out a block
-    # that work queued there since ``after`` (a forward's workspace, freed when the call
-    # returned) still uses, and the build does not wait for that work.
-    with torch.cuda.stream(side):
+        # Allocated on the stream that writes it: the current stream's pool may hand out a block
+        # that work queued there since ``after`` (a forward's workspace, freed when the call
+        # returned) still uses, and the build does not wait for that work.
+        with torch.cuda.stream(side):
+            buf = torch.empty(n, dtype=torch.uint8, device=q.device)
+    else:
         buf = torch.empty(n, dtype=torch.uint8, device=q.device)
     rc = L.dsa_sparse_mla_bwd_build_index(indices.data_ptr(), B, S, S_kv, H, G, D, int(d_v), topk, flags, cap,
                                           buf.data_ptr(), n, side.cuda_stream)
