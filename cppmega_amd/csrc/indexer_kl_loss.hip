@@ -375,7 +375,11 @@ __global__ void __launch_bounds__(kNT) kl_mask_tiles_kernel(Params p) {
 // ---------------------------------------------------------------------------
 // 2. attention normalisers beta_h[t] (log2 units of c * q.k)
 // ---------------------------------------------------------------------------
-template <int D, int NW>
+// The admissible set: every column up to the diagonal, or the top-k set by the rows'
+// bitmask or by lane masks.
+enum StatsSet { kAllColumns, kRowBits, kLaneMasks };
+
+template <int D, int NW, StatsSet SET>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 4 : 2)))
 kl_attn_stats_kernel(Params p) {
   using C = Cfg<D, NW>;
@@ -403,12 +407,23 @@ kl_attn_stats_kernel(Params p) {
     ld.load(p, b, grp, 0, kr);
     ChunkLoader<D, NW>::store(KS[0], kr);
     __syncthreads();
-    // sparse: the wave's lane masks (scalar loads; the tile of 32 keys is 16 words)
+    // lane masks: scalar loads, the tile of 32 keys is 16 words
     typedef const __attribute__((address_space(4))) uint64_t *scalar_u64;
-    const scalar_u64 tiles =
-        p.sparse && wt0 < p.Sq ? (scalar_u64)(uintptr_t)(p.tiles + (b * ((p.Sq + 31) / 32) + wt0 / 32) * p.W * 16) : nullptr;
+    scalar_u64 tiles = nullptr;
+    if constexpr (SET == kLaneMasks)
+      if (wt0 < p.Sq) tiles = (scalar_u64)(uintptr_t)(p.tiles + (b * ((p.Sq + 31) / 32) + wt0 / 32) * p.W * 16);
+    // row bits: the chunk's words are loaded one chunk ahead
+    uint32_t mw[C::SUBS];
+#pragma unroll
+    for (int sub = 0; sub < C::SUBS; ++sub) mw[sub] = SET == kRowBits ? mask_word(p, b, t, 32 * sub) : 0xffffffffu;
     for (int ci = 0; ci < nch; ++ci) {
       if (ci + 1 < nch) ld.load(p, b, grp, (int64_t)(ci + 1) * C::KC, kr);
+      uint32_t mwn[C::SUBS];
+      if constexpr (SET == kRowBits) {
+#pragma unroll
+        for (int sub = 0; sub < C::SUBS; ++sub)
+          mwn[sub] = ci + 1 < nch ? mask_word(p, b, t, (int64_t)(ci + 1) * C::KC + 32 * sub) : 0u;
+      }
       const unsigned char *ks = KS[ci & 1];
 #pragma unroll
       for (int sub = 0; sub < C::SUBS; ++sub) {
@@ -417,25 +432,25 @@ kl_attn_stats_kernel(Params p) {
         const f32x16 acc = qk_subtile<D>(ks, sub, Q);
         // c > 0: max(c * acc) = c * max(acc), and exp2(c * acc - nm) is one fma
         float x[16], lm;
-        if (p.sparse) {
+        if constexpr (SET == kLaneMasks) {
 #pragma unroll
           for (int a = 0; a < 16; ++a) {
-            const uint64_t m = tiles[(key0 >> 5) * 16 + a];
-            x[a] = __builtin_amdgcn_inverse_ballot_w64(m) ? acc[a] : -INFINITY;
+            const uint64_t on = tiles[(key0 >> 5) * 16 + a];
+            x[a] = __builtin_amdgcn_inverse_ballot_w64(on) ? acc[a] : -INFINITY;
           }
           lm = x[0];
 #pragma unroll
           for (int a = 1; a < 15; a += 2) lm = max3(lm, x[a], x[a + 1]);
           lm = max3(lm, x[15], x[15]);
-        } else if (key0 + 31 > wt0 || key0 + 31 >= p.Sk || wt_last >= p.Sq) {
-          const uint32_t vb = valid_bits(p, 0xffffffffu, t, key0);
-#pragma unroll
-          for (int a = 0; a < 16; ++a) x[a] = keep_or_neginf(acc[a], vb, a);
         } else {
+          if (SET == kRowBits || key0 + 31 > wt0 || key0 + 31 >= p.Sk || wt_last >= p.Sq) {
+            const uint32_t vb = valid_bits(p, mw[sub], t, key0);
 #pragma unroll
-          for (int a = 0; a < 16; ++a) x[a] = acc[a];
-        }
-        if (!p.sparse) {
+            for (int a = 0; a < 16; ++a) x[a] = keep_or_neginf(acc[a], vb, a);
+          } else {
+#pragma unroll
+            for (int a = 0; a < 16; ++a) x[a] = acc[a];
+          }
           lm = x[0];
 #pragma unroll
           for (int a = 1; a < 16; ++a) lm = fmaxf(lm, x[a]);
@@ -446,6 +461,10 @@ kl_attn_stats_kernel(Params p) {
         for (int a = 0; a < 16; ++a) s += exp2_fast(fmaf(x[a], p.c, -nm));
         d = d * exp2_fast(m - nm) + s;
         m = nm;
+      }
+      if constexpr (SET == kRowBits) {
+#pragma unroll
+        for (int sub = 0; sub < C::SUBS; ++sub) mw[sub] = mwn[sub];
       }
       if (ci + 1 < nch) {
         ChunkLoader<D, NW>::store(KS[(ci + 1) & 1], kr);
@@ -1014,7 +1033,10 @@ static int launch_mfma(const Params &p, hipStream_t st) {
   using CS = Cfg<D, NWS>;
   using CP = Cfg<D, NWP>;
   const int64_t NBS = (p.Sq + CS::TB - 1) / CS::TB, NP = (NBS + 1) / 2;
-  hipLaunchKernelGGL((kl_attn_stats_kernel<D, NWS>), dim3((unsigned)(p.B * p.H * NP)), dim3(CS::NT), 0, st, p);
+  const dim3 gs((unsigned)(p.B * p.H * NP));
+  if (!p.sparse) hipLaunchKernelGGL((kl_attn_stats_kernel<D, NWS, kAllColumns>), gs, dim3(CS::NT), 0, st, p);
+  else if (p.tiles == nullptr) hipLaunchKernelGGL((kl_attn_stats_kernel<D, NWS, kRowBits>), gs, dim3(CS::NT), 0, st, p);
+  else hipLaunchKernelGGL((kl_attn_stats_kernel<D, NWS, kLaneMasks>), gs, dim3(CS::NT), 0, st, p);
   int rc = check_launch("kl_attn_stats_kernel");
   if (rc) return rc;
   const int64_t NBP = (p.Sq + CP::TB - 1) / CP::TB;
@@ -1093,12 +1115,21 @@ static int kl_setup(const char *fn, const float *index_scores, const void *topk_
   return DSA_OK;
 }
 
+// Whether the lane masks' launch (3 to 7 us) pays: against the row bitmask they take
+// off the statistics 3 us at 134 M scores (b = 2, s = 2048, 16 heads) of 64 or 128
+// dims and 9 at 537 M, but -2 to 1 up to 72 M; of 192 or 256 dims, whose registers the
+// bitmask's words overfill, 3 to 5 us at 17 M and -3 to 2 up to 8 M.
+static bool use_lane_masks(const Params &p, int64_t D) {
+  return (double)(p.B * p.H) * (double)p.Sq * (double)p.Sk >= (D <= 128 ? 1e8 : 1.2e7);
+}
+
 template <bool LOSS, bool GRAD>
-static int kl_launch(const Params &p, int64_t D, hipStream_t st) {
+static int kl_launch(Params p, int64_t D, hipStream_t st) {
   hipLaunchKernelGGL(kl_index_stats_kernel, dim3((unsigned)((p.B * p.Sq + 3) / 4)), dim3(kNT), 0, st, p);
   int rc = check_launch("kl_index_stats_kernel");
   if (rc) return rc;
-  if (p.sparse) {
+  if (!use_lane_masks(p, D)) p.tiles = nullptr;
+  if (p.sparse && p.tiles != nullptr) {
     hipLaunchKernelGGL(kl_mask_tiles_kernel, dim3((unsigned)(p.B * ((p.Sq + 31) / 32)), (unsigned)(p.W < 64 ? (p.W + 7) / 8 : 8)),
                        dim3(kNT), 0, st, p);
     rc = check_launch("kl_mask_tiles_kernel");
