@@ -25,7 +25,7 @@
 //     holds 16 keys of one token and row reductions stay in-lane); key chunks
 //     are double-buffered in LDS and shared by the 8 waves; a long and a short
 //     token block share one workgroup so every workgroup does equal work;
-//  3. kl_pass_kernel         per (b, 256-token block, key chunk): for every head
+//  3. kl_pass_kernel         per (b, 256- or 128-token block, key chunk): for every head
 //     recompute c * q.k, accumulate exp2(c * q.k - beta_h) in registers (the
 //     head sum of P), then form the KL terms of the chunk against
 //     Q = exp2(index * log2(e) - gamma) and write one partial sum per token;
@@ -584,18 +584,17 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
   const unsigned char *kbase = p.key + ((k0 * p.B + b) * p.G) * (int64_t)C::ROWB;
   const uint32_t lds = lds_address(smem);
   const uint32_t q_lds = lds + (uint32_t)(PC::OFF_Q + w * 32 * C::ROWB);
-  // piece i of this wave's loads for a head: its share of the key chunk (into
-  // buffer kbuf; a head of the same key group fetches it again), then its q slice
+  // this wave's loads: its share of the key chunk of a group of heads, into buffer
+  // kbuf, and its q slice of a head
   const int hpg = (int)(p.H / p.G), H = (int)p.H;
-  auto fetch = [&](i32x4 krs, i32x4 qrs, int kbuf, int i) {
-    if (i < PC::KP)
-      lds_dma_16(lds + (uint32_t)(kbuf * C::KC * C::ROWB + (w * PC::KP + i) * 1024), ko[i < PC::KP ? i : 0], krs, 0u);
-    else
-      lds_dma_16(q_lds + (uint32_t)((i - PC::KP) * 1024), qo[i < PC::KP ? 0 : i - PC::KP], qrs, 0u);
+  auto fetch_keys = [&](i32x4 krs, int kbuf) {
+#pragma unroll
+    for (int i = 0; i < PC::KP; ++i) lds_dma_16(lds + (uint32_t)(kbuf * C::KC * C::ROWB + (w * PC::KP + i) * 1024), ko[i], krs, 0u);
   };
-  auto key_rs = [&](int h) { return make_buffer_words(kbase + h / hpg * C::ROWB, kbytes); };
+  auto fetch_q = [&](i32x4 qrs, int i) { lds_dma_16(q_lds + (uint32_t)(i * 1024), qo[i], qrs, 0u); };
+  auto key_rs = [&](int grp) { return make_buffer_words(kbase + grp * C::ROWB, kbytes); };
   auto query_rs = [&](int h) { return make_buffer_words(qb + h * C::ROWB, qbytes); };
-  constexpr int NF = PC::KP + (FAR ? 0 : PC::QP);  // loads per head
+  constexpr int NF = FAR ? 0 : PC::QP;  // q loads per head
   bool all_on = !FAR, any_on = false;  // wave-uniform
 #pragma unroll
   for (int sub = 0; sub < C::SUBS; ++sub) {
@@ -608,19 +607,21 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
     return as_bf16x8(*reinterpret_cast<const i32x4 *>(tile + (r0 + l32) * C::ROWB + (((2 * k + g) ^ PC::swz(l32)) * 16)));
   };
   const float *beta_bt = p.beta + b * p.H * p.Sq + (t < p.Sq ? t : 0);
-  i32x4 krs = key_rs(0), qrs = query_rs(0);
+  i32x4 qrs = query_rs(0);
+  fetch_keys(key_rs(0), 0);
 #pragma unroll
-  for (int i = 0; i < NF; ++i) fetch(krs, qrs, 0, i);
+  for (int i = 0; i < NF; ++i) fetch_q(qrs, i);
   // The previous head's last sub-tile and its normaliser: its exp2 work runs
   // under the next head's first products (before head 0: exp2(-inf) = 0).
   f32x16 cur;
 #pragma unroll
   for (int a = 0; a < 16; ++a) cur[a] = 0.0f;
   float bprev = INFINITY, bn = beta_bt[0];
+  int grp = 0, left = hpg;  // the head's key group, and its heads still to come
   for (int h = 0; h < H; ++h) {
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this head's q and k, fetched a head ago
-    __syncthreads();                     // every wave's share of k; the other k buffer is consumed
-    const unsigned char *ks = smem + (h & 1) * C::KC * C::ROWB;
+    if (left == hpg) __syncthreads();    // every wave's share of the group's k; the other k buffer is consumed
+    const unsigned char *ks = smem + (grp & 1) * C::KC * C::ROWB;
     bf16x8 Q[C::KSTEPS];
 #pragma unroll
     for (int k = 0; k < C::KSTEPS; ++k)
@@ -629,9 +630,12 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
     const float bh = bn;
     const int hn = h + 1 < H ? h + 1 : h;  // (past the last head: its own again, unused)
     bn = beta_bt[(int64_t)hn * p.Sq];
-    krs = key_rs(hn);
     qrs = query_rs(hn);
-    const int kb = (h + 1) & 1;
+    if (--left == 0) {  // the last head of its group: the next group's keys
+      left = hpg;
+      ++grp;
+      fetch_keys(key_rs(grp < (int)p.G ? grp : grp - 1), grp & 1);
+    }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the q slice is in registers, its LDS free
     if (all_on) {
       // key operands are read two products ahead
@@ -657,12 +661,12 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
 #pragma unroll
           for (int e = 0; e < kE; ++e)
             if (k * kE + e < 16) P[ps][k * kE + e] += exp2_fast(fmaf(cur[k * kE + e], p.c, -pb));
-          // the next head's loads, spread over the first sub-tiles
-          constexpr int kPer = (NF + C::KSTEPS * (C::SUBS - 1) - 1) / (C::KSTEPS * (C::SUBS - 1));
+          // the next head's q loads, spread over the first sub-tile
+          constexpr int kPer = (NF + C::KSTEPS - 1) / C::KSTEPS;
 #pragma unroll
           for (int u = 0; u < kPer; ++u) {
             const int f = i * kPer + u;
-            if (f < NF) fetch(krs, qrs, kb, f);
+            if (f < NF) fetch_q(qrs, f);
           }
           __builtin_amdgcn_sched_barrier(0);  // keep this order
         }
@@ -671,7 +675,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
       bprev = bh;
     } else {
 #pragma unroll
-      for (int i = 0; i < NF; ++i) fetch(krs, qrs, kb, i);
+      for (int i = 0; i < NF; ++i) fetch_q(qrs, i);
       if (any_on) {
 #pragma unroll
         for (int sub = 0; sub < C::SUBS; ++sub) {
@@ -1018,6 +1022,16 @@ static Layout layout(int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t D, in
   return L;
 }
 
+// (token block, key chunk) pairs of one batch at or below the diagonal.
+static int64_t pass_items(const Params &p, int64_t TB, int64_t KC) {
+  int64_t n = 0;
+  for (int64_t t = 0; t < p.Sq; t += TB) {
+    const int64_t lt = (t + TB < p.Sq ? t + TB : p.Sq) - 1;
+    n += (lt < p.Sk - 1 ? lt : p.Sk - 1) / KC + 1;
+  }
+  return n;
+}
+
 template <int D, int NW, bool LOSS, bool GRAD, bool FAR>
 static int launch_pass(const Params &p, int64_t items, hipStream_t st) {
   const auto pass = kl_pass_kernel<D, NW, LOSS, GRAD, FAR>;
@@ -1039,13 +1053,8 @@ static int launch_mfma(const Params &p, hipStream_t st) {
   else hipLaunchKernelGGL((kl_attn_stats_kernel<D, NWS, kLaneMasks>), gs, dim3(CS::NT), 0, st, p);
   int rc = check_launch("kl_attn_stats_kernel");
   if (rc) return rc;
-  const int64_t NBP = (p.Sq + CP::TB - 1) / CP::TB;
   Params q = p;
-  q.NI = 0;
-  for (int64_t j = 0; j < NBP; ++j) {
-    const int64_t lt = (CP::TB * (j + 1) < p.Sq ? CP::TB * (j + 1) : p.Sq) - 1;
-    q.NI += (lt < p.Sk - 1 ? lt : p.Sk - 1) / CP::KC + 1;
-  }
+  q.NI = pass_items(p, CP::TB, CP::KC);
   const int64_t items = (p.B * q.NI + 7) / 8 * 8;
   const int64_t rows = p.Sq < 32 ? p.Sq : 32;  // of a wave
   const bool far = (rows - 1) * p.B * p.H * CP::ROWB + CP::ROWB > (int64_t)0xffffffff;
@@ -1123,6 +1132,17 @@ static bool use_lane_masks(const Params &p, int64_t D) {
   return (double)(p.B * p.H) * (double)p.Sq * (double)p.Sk >= (D <= 128 ? 1e8 : 1.2e7);
 }
 
+// The pass with 8 waves a workgroup (256 tokens) or 4 (128).  Four: twice the
+// workgroups, which at 64 dims also run two to a compute unit (b = 1, s = 4096, 32
+// heads, loss: 191 us, 215 with eight); from 128 dims on the LDS holds one, so half of
+// a compute unit's wave slots would stay empty, and they pay only while they all run
+// at once (32 heads of 128: s = 2048 125 us, 141 with eight; b = 2 181 and 155).
+template <int D, bool LOSS, bool GRAD>
+static int launch_by_size(const Params &p, hipStream_t st) {
+  if (D == 64 || p.B * pass_items(p, 128, Cfg<D, 4>::KC) <= 256) return launch_mfma<D, 8, 4, LOSS, GRAD>(p, st);
+  return launch_mfma<D, 8, D == 64 ? 4 : 8, LOSS, GRAD>(p, st);
+}
+
 template <bool LOSS, bool GRAD>
 static int kl_launch(Params p, int64_t D, hipStream_t st) {
   hipLaunchKernelGGL(kl_index_stats_kernel, dim3((unsigned)((p.B * p.Sq + 3) / 4)), dim3(kNT), 0, st, p);
@@ -1136,9 +1156,9 @@ static int kl_launch(Params p, int64_t D, hipStream_t st) {
     if (rc) return rc;
   }
   switch (D) {
-    case 64: return launch_mfma<64, 8, 8, LOSS, GRAD>(p, st);
-    case 128: return launch_mfma<128, 8, 8, LOSS, GRAD>(p, st);
-    case 192: return launch_mfma<192, 8, 8, LOSS, GRAD>(p, st);
+    case 64: return launch_by_size<64, LOSS, GRAD>(p, st);
+    case 128: return launch_by_size<128, LOSS, GRAD>(p, st);
+    case 192: return launch_by_size<192, LOSS, GRAD>(p, st);
     default:  // (eight q slices and two key chunks would pass 160 KiB)
       return launch_mfma<256, 8, 4, LOSS, GRAD>(p, st);
   }
