@@ -69,6 +69,7 @@ EXPORTED_SYMBOLS = (
     "dsa_indexer_kl_loss_state_size",
     "dsa_indexer_kl_loss_with_grad_workspace_size",
     "dsa_indexer_kl_loss_with_grad",
+    "dsa_indexer_kl_loss_grad_state",
     "dsa_indexer_kl_loss_grad_apply",
     "dsa_topk_index_mask",
     "dsa_stage_timing",
@@ -149,6 +150,8 @@ _SIGNATURES = {
     "dsa_indexer_kl_loss_with_grad": (_i32, [_c_void_p, _c_void_p, _i32, _i64, _c_void_p, _c_void_p, _c_void_p,
                                              _c_void_p, _c_void_p, _size_t, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _i32,
                                              _c_void_p, _size_t, _c_void_p]),
+    "dsa_indexer_kl_loss_grad_state": (_i32, [_c_void_p, _c_void_p, _i32, _i64, _c_void_p, _c_void_p, _c_void_p, _size_t]
+                                       + [_i64] * 6 + [_f32, _f32, _i32, _c_void_p, _size_t, _c_void_p]),
     "dsa_indexer_kl_loss_grad_apply": (_i32, [_c_void_p, _size_t, _c_void_p, _c_void_p] + [_i64] * 5
                                        + [_f32, _i32, _c_void_p]),
     "dsa_topk_index_mask": (_i32, [_c_void_p, _i32, _i64, _c_void_p, _i64, _i64, _i64, _i64, _i64,

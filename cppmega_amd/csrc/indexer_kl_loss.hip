@@ -59,6 +59,7 @@
 // sparse, the columns of the row's top-k set only, in column order (v is 0
 // elsewhere), with the set's bitmask: 12 MB instead of 128 MiB at top-256.
 #include "dsa_common.hpp"
+#include "wave_ops.hpp"
 
 namespace dsa {
 namespace kl {
@@ -150,15 +151,9 @@ __global__ void __launch_bounds__(kNT) kl_index_stats_kernel(Params p) {
       if (in) p.mask[row * p.W + i] = word;
       int at = 0;
       if (pre != nullptr) {  // rank of the word's first column, by a prefix sum over the lanes
-        const int n = __popc(word);
-        int x = n;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-          const int y = __shfl_up(x, off, 64);
-          if (lane >= off) x += y;
-        }
+        const int n = __popc(word), x = (int)wv::wave_incl_scan((uint32_t)n);
         at = before + x - n;
-        before += __shfl(x, 63, 64);
+        before += (int)wv::readlane((uint32_t)x, 63);
         if (in && i % wpc == 0) pre[i / wpc] = at;
         const int64_t lb = last_k - (int64_t)i * 32;  // last admissible bit of the word
         adm += __popc(lb >= 31 ? word : (lb < 0 ? 0u : word & ((2u << lb) - 1u)));
@@ -192,8 +187,7 @@ __global__ void __launch_bounds__(kNT) kl_index_stats_kernel(Params p) {
       }
     }
     if (pre != nullptr) {
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) adm += __shfl_xor(adm, off, 64);
+      adm = (int)wv::wave_reduce((uint32_t)adm, wv::AddU());
       if (lane == 0) {
         pre[p.NC] = before;
         pre[p.NC + 1] = adm;
@@ -1233,31 +1227,53 @@ static void kl_bind_state(dsa::kl::Params &p, void *state, const dsa::kl::State 
   p.flag = reinterpret_cast<float *>(s + S.flag);
 }
 
-extern "C" int dsa_indexer_kl_loss_with_grad(const float *index_scores, const void *topk_indices, int topk_dtype,
-                                             int64_t topk, const void *query, const void *key, float *loss,
-                                             float *row_loss, void *state, size_t state_bytes, int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t G,
-                                             int64_t D, float softmax_scale, float loss_coeff, int sparse,
-                                             void *workspace, size_t workspace_bytes, void *stream) {
+// loss null: the state alone (the rows' losses are in the workspace then).
+static int kl_with_grad(const char *fn, const float *index_scores, const void *topk_indices, int topk_dtype, int64_t topk,
+                        const void *query, const void *key, float *loss, float *row_loss, void *state,
+                        size_t state_bytes, int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t G, int64_t D,
+                        float softmax_scale, float loss_coeff, int sparse, void *workspace, size_t workspace_bytes,
+                        void *stream) {
   using namespace dsa;
   using namespace dsa::kl;
-  DSA_REQUIRE(loss, "dsa_indexer_kl_loss_with_grad: null loss pointer");
   Params p;
-  int rc = kl_setup("dsa_indexer_kl_loss_with_grad", index_scores, topk_indices, topk_dtype, topk, query, key, B, Sq, Sk,
-                    H, G, D, softmax_scale, loss_coeff, sparse, workspace, workspace_bytes, p, true);
+  int rc = kl_setup(fn, index_scores, topk_indices, topk_dtype, topk, query, key, B, Sq, Sk, H, G, D, softmax_scale,
+                    loss_coeff, sparse, workspace, workspace_bytes, p, true);
   if (rc) return rc;
   const State S = state_layout(B, Sq, Sk, D, topk, sparse);
   if (!state || state_bytes < S.total)
-    return set_error(DSA_ERR_WORKSPACE, "dsa_indexer_kl_loss_with_grad: state %zu bytes < %zu required",
-                     state ? state_bytes : (size_t)0, S.total);
+    return set_error(DSA_ERR_WORKSPACE, "%s: state %zu bytes < %zu required", fn, state ? state_bytes : (size_t)0, S.total);
   kl_bind_state(p, state, S);
   if (!p.sparse) p.grad = static_cast<float *>(state);
   if (row_loss) p.rows = row_loss;
   p.loss = loss;
   hipStream_t st = static_cast<hipStream_t>(stream);
   rc = kl_launch<true, true>(p, D, st);
-  if (rc) return rc;
+  if (rc || !loss) return rc;
   hipLaunchKernelGGL(kl_mean_kernel, dim3(1), dim3(1024), 0, st, p);
   return check_launch("kl_mean_kernel");
+}
+
+extern "C" int dsa_indexer_kl_loss_with_grad(const float *index_scores, const void *topk_indices, int topk_dtype,
+                                             int64_t topk, const void *query, const void *key, float *loss,
+                                             float *row_loss, void *state, size_t state_bytes, int64_t B, int64_t Sq,
+                                             int64_t Sk, int64_t H, int64_t G, int64_t D, float softmax_scale,
+                                             float loss_coeff, int sparse, void *workspace, size_t workspace_bytes,
+                                             void *stream) {
+  using namespace dsa;
+  DSA_REQUIRE(loss, "dsa_indexer_kl_loss_with_grad: null loss pointer");
+  return kl_with_grad("dsa_indexer_kl_loss_with_grad", index_scores, topk_indices, topk_dtype, topk, query, key, loss,
+                      row_loss, state, state_bytes, B, Sq, Sk, H, G, D, softmax_scale, loss_coeff, sparse, workspace,
+                      workspace_bytes, stream);
+}
+
+extern "C" int dsa_indexer_kl_loss_grad_state(const float *index_scores, const void *topk_indices, int topk_dtype,
+                                              int64_t topk, const void *query, const void *key, void *state,
+                                              size_t state_bytes, int64_t B, int64_t Sq, int64_t Sk, int64_t H,
+                                              int64_t G, int64_t D, float softmax_scale, float loss_coeff, int sparse,
+                                              void *workspace, size_t workspace_bytes, void *stream) {
+  return kl_with_grad("dsa_indexer_kl_loss_grad_state", index_scores, topk_indices, topk_dtype, topk, query, key, nullptr,
+                      nullptr, state, state_bytes, B, Sq, Sk, H, G, D, softmax_scale, loss_coeff, sparse, workspace,
+                      workspace_bytes, stream);
 }
 
 extern "C" int dsa_indexer_kl_loss_grad_apply(const void *state, size_t state_bytes, const float *grad_loss,

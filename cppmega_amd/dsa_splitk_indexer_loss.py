@@ -91,9 +91,10 @@ def _forward(index_scores, topk_indices, query, key, softmax_scale, loss_coeff, 
     return loss, rows
 
 
-def _forward_state(index_scores, topk_indices, query, key, softmax_scale, loss_coeff, sparse_loss, return_rows=False):
-    """(loss, state, args of _apply_state, per-row losses or None): the loss and its gradient up to the upstream
-    factor."""
+def _forward_state(index_scores, topk_indices, query, key, softmax_scale, loss_coeff, sparse_loss, return_rows=False,
+                   want_loss=True):
+    """(loss or None, state, args of _apply_state, per-row losses or None): the loss and its gradient up to the
+    upstream factor."""
     index_scores, topk_indices, tdt, topk, query, key, sparse, (b, sq, sk, np_, g, hn) = _prepare(
         index_scores, topk_indices, query, key, sparse_loss)
     dev = _lib.ensure_device(query)
@@ -103,13 +104,16 @@ def _forward_state(index_scores, topk_indices, query, key, softmax_scale, loss_c
                      dtype=torch.uint8, device=query.device)
     state = torch.empty(max(int(lib.dsa_indexer_kl_loss_state_size(b, sq, sk, hn, topk, sp)), 1),
                         dtype=torch.uint8, device=query.device)
-    loss = torch.empty((), dtype=torch.float32, device=query.device)
+    inputs = (index_scores.data_ptr(), _lib.ptr(topk_indices), tdt, topk, query.data_ptr(), key.data_ptr())
+    rest = (state.data_ptr(), state.numel(), b, sq, sk, np_, g, hn, float(softmax_scale), float(loss_coeff), sp,
+            ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
+    loss = torch.empty((), dtype=torch.float32, device=query.device) if want_loss else None
     rows = torch.empty((b, sq), dtype=torch.float32, device=query.device) if return_rows else None
-    rc = lib.dsa_indexer_kl_loss_with_grad(
-        index_scores.data_ptr(), _lib.ptr(topk_indices), tdt, topk, query.data_ptr(), key.data_ptr(), loss.data_ptr(),
-        _lib.ptr(rows), state.data_ptr(), state.numel(), b, sq, sk, np_, g, hn, float(softmax_scale), float(loss_coeff), sp,
-        ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
-    _lib.check(rc, "dsa_indexer_kl_loss_with_grad")
+    if want_loss:
+        rc = lib.dsa_indexer_kl_loss_with_grad(*inputs, loss.data_ptr(), _lib.ptr(rows), *rest)
+    else:
+        rc = lib.dsa_indexer_kl_loss_grad_state(*inputs, *rest)
+    _lib.check(rc, "dsa_indexer_kl_loss_with_grad" if want_loss else "dsa_indexer_kl_loss_grad_state")
     return loss, state, (b, sq, sk, hn, topk, float(loss_coeff), sp), rows
 
 
@@ -132,7 +136,8 @@ def indexer_kl_loss_backward(grad_loss, index_scores, topk_indices, query, key, 
     recomputed on the GPU.  NaN over a row whose loss is NaN."""
     gl = torch.as_tensor(grad_loss, dtype=torch.float32, device=query.device).reshape(1).contiguous()
     if sparse_loss:  # the top-k columns' state, expanded
-        _, state, args, _ = _forward_state(index_scores, topk_indices, query, key, softmax_scale, loss_coeff, True)
+        _, state, args, _ = _forward_state(index_scores, topk_indices, query, key, softmax_scale, loss_coeff, True,
+                                           want_loss=False)
         return _apply_state(state, gl, args)
     index_scores, topk_indices, tdt, topk, query, key, sparse, (b, sq, sk, np_, g, hn) = _prepare(
         index_scores, topk_indices, query, key, sparse_loss)

@@ -550,6 +550,7 @@ int dsa_indexer_kl_loss_backward(const float *index_scores,
  * the scores, or (sparse) 4 bytes per top-k entry and about Sk / 8 + Sk / 32
  * bytes per row.  loss_coeff is read by the second call.  The workspace
  * (dsa_indexer_kl_loss_with_grad_workspace_size) is needed by the first only.
+ * dsa_indexer_kl_loss_grad_state leaves the same state and no loss.
  */
 size_t dsa_indexer_kl_loss_state_size(int64_t B, int64_t Sq, int64_t Sk, int64_t D,
                                       int64_t topk, int sparse);
@@ -564,6 +565,13 @@ int dsa_indexer_kl_loss_with_grad(const float *index_scores, const void *topk_in
                                   float softmax_scale, float loss_coeff, int sparse,
                                   void *workspace, size_t workspace_bytes,
                                   void *stream);
+int dsa_indexer_kl_loss_grad_state(const float *index_scores, const void *topk_indices,
+                                   int topk_dtype, int64_t topk, const void *query,
+                                   const void *key, void *state, size_t state_bytes,
+                                   int64_t B, int64_t Sq, int64_t Sk, int64_t H, int64_t G,
+                                   int64_t D, float softmax_scale, float loss_coeff,
+                                   int sparse, void *workspace, size_t workspace_bytes,
+                                   void *stream);
 int dsa_indexer_kl_loss_grad_apply(const void *state, size_t state_bytes,
                                    const float *grad_loss, float *grad_index_scores,
                                    int64_t B, int64_t Sq, int64_t Sk, int64_t D,
