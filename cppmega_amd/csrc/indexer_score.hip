@@ -545,7 +545,17 @@ static int launch_idx_act(IdxParams p, hipStream_t st) {
     p.chunk = C::CHUNK;
     // tokens for one wave: the other three would only load keys
     p.split = p.Sq <= C::TPW;
-    while (p.chunk > C::KT && 2 * ((p.Sk + p.chunk - 1) / p.chunk) * ntb * p.B <= slots) p.chunk /= 2;
+    for (; p.chunk > C::KT; p.chunk /= 2) {
+      const int64_t wgs = 2 * ((p.Sk + p.chunk - 1) / p.chunk) * ntb * p.B;
+      if (wgs > slots) break;
+      // Past one workgroup on each of 256 compute units, 64 KiB of q operands (rows of
+      // 256 bytes) must be worth their second load: chunks of 512 keys, or of 256 where
+      // the token block's q is read by several workgroups already (64 bf16 heads of 128:
+      // 64 tokens x 512 keys x batch 16 15.1 us whole, 16.2 in halves; 16 tokens x 256 keys
+      // x batch 32 7.4 us in 128 keys, 10.3 in 64; 8 tokens x 16384 keys x batch 4 15.0 us
+      // in 512 keys, 14.1 in 256)
+      if (C::ROWB >= 256 && wgs > 256 && p.chunk < 1024 && (p.chunk < 512 || p.Sk <= p.chunk)) break;
+    }
     grid = dim3((unsigned)((p.Sk + p.chunk - 1) / p.chunk), (unsigned)ntb, (unsigned)p.B);
   }
   if (p.causal == kCausalWindow)

@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from cppmega_amd import index_scores, topk_indices
+from oracle import fp8 as ofp8
 from oracle import indexer as oix
 from oracle import topk as otk
 
@@ -68,6 +69,41 @@ def test_scores_of_few_tokens(dev, Sq, Sk, B, H, D, causal):
     if causal:
         ref = ref.masked_fill(torch.ones(Sq, Sk, dtype=torch.bool).triu(1), float("-inf"))
     assert torch.equal(torch.isneginf(got), torch.isneginf(ref))
+    fin = torch.isfinite(ref)
+    # fp32 sums in another order: the bar of the dense score tests
+    assert (got[fin] - ref[fin]).abs().max() <= 1e-3 * ref[fin].abs().max().clamp_min(1e-6)
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("Sq,Sk,B,H,D,fp8", [
+    # e4m3: one wave's tokens, whose keys the four waves share by 32-key sub-tiles (tiles of 128 keys at D 128, 256 at 64)
+    (1, 127, 2, 64, 128, True), (1, 129, 2, 64, 128, True), (1, 511, 1, 64, 128, True), (1, 2049, 3, 64, 128, True),
+    (1, 257, 2, 64, 64, True), (2, 255, 1, 32, 64, True), (4, 2047, 2, 16, 64, True), (2, 513, 3, 32, 128, True),
+    (1, 5000, 16, 64, 128, True),
+    # e4m3: more tokens, chunks of one tile and more
+    (5, 300, 2, 64, 128, True), (17, 600, 1, 16, 64, True),
+    # bf16 rows of 256 bytes: whole, 512-key and 256-key chunks at one workgroup a compute unit
+    (64, 512, 16, 64, 128, False), (16, 256, 32, 64, 128, False), (8, 8193, 4, 64, 128, False),
+])
+def test_scores_of_few_tokens_write_every_column(dev, Sq, Sk, B, H, D, fp8, causal):
+    """Every column is owned by exactly one wave: an output full of NaN is overwritten."""
+    g = torch.Generator().manual_seed(Sq * 17 + Sk)
+    q = torch.randn((Sq, B, H, D), generator=g).to(torch.bfloat16)
+    k = torch.randn((Sk, B, D), generator=g).to(torch.bfloat16)
+    w = torch.randn((Sq, B, H), generator=g) / H ** 0.5
+    kw = {}
+    if fp8:
+        q, qs = ofp8.tensorwise_quantize(q)
+        k, ks = ofp8.tensorwise_quantize(k)
+        kw = dict(q_scale=qs.to(dev), k_scale=ks.to(dev))
+        ref = oix.compute_index_scores(q.float(), w, k.float(), q_scale=qs, k_scale=ks)
+    else:
+        ref = oix.compute_index_scores(q, w, k)
+    out = torch.full((B, Sq, Sk), float("nan"), device=dev)
+    got = index_scores(q.to(dev), w.to(dev), k.to(dev), causal=causal, out=out, **kw).cpu()
+    if causal:
+        ref = ref.masked_fill(torch.ones(Sq, Sk, dtype=torch.bool).triu(1), float("-inf"))
+    assert torch.equal(torch.isneginf(got), torch.isneginf(ref)) and not bool(got.isnan().any())
     fin = torch.isfinite(ref)
     # fp32 sums in another order: the bar of the dense score tests
     assert (got[fin] - ref[fin]).abs().max() <= 1e-3 * ref[fin].abs().max().clamp_min(1e-6)
