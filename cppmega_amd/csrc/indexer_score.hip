@@ -21,6 +21,7 @@
 // tiles above its last token.  Late (longer) token blocks are scheduled first.
 // This file is compiled with IEEE mode off and NaN inputs left undefined, so
 // the ReLU is a single v_max_f32 per element.
+#include <mutex>
 #include <type_traits>
 
 #include "dsa_common.hpp"
@@ -488,13 +489,16 @@ indexer_score_kernel(const IdxParams p) {
 // Workgroups of `kernel` resident at once on the current device (cached per device).
 template <class K>
 static int64_t resident_groups(K kernel, int threads) {
-  // cached per (device, kernel): kernels of one signature share the type K
+  // cached per (device, kernel): kernels of one signature share the type K; calls
+  // come from several threads
   struct Entry { const void *k; int dev; int groups; };
   static Entry cache[256];
   static int used = 0;
+  static std::mutex lock;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 0;
   const void *kp = reinterpret_cast<const void *>(kernel);
+  const std::lock_guard<std::mutex> hold(lock);
   for (int i = 0; i < used; ++i)
     if (cache[i].k == kp && cache[i].dev == dev) return cache[i].groups;
   int cus = 0, per_cu = 0;
