@@ -3,14 +3,14 @@
 ``build_inverse_index`` builds the backward's kv-row -> entries index from the
 indices alone (on a second stream, overlapping whatever runs meanwhile) and
 ``sparse_mla_bwd(..., inverse_index=...)`` then runs only the main kernel and
-the dKV reduction.  The result must be the same bits as the one-call backward,
-through the autograd functions, and across replays of a captured HIP graph.
+the dKV reduction.  The result must be the same bits as the one-call backward
+(the autograd functions' too), and across replays of a captured HIP graph.
 """
 import pytest
 import torch
 
 from cppmega_amd import synthetic
-from cppmega_amd.sparse_mla_ops import (SparseMLA, SparseMLA_FP8, build_inverse_index, side_stream,
+from cppmega_amd.sparse_mla_ops import (SparseMLA, SparseMLA_FP8, build_inverse_index, per_token_cast_to_fp8, side_stream,
                                         sparse_mla_bwd, sparse_mla_bwd_fp8, sparse_mla_fwd_fp8_interface,
                                         sparse_mla_fwd_interface)
 
@@ -66,24 +66,43 @@ def test_prebuilt_index_fp8(dev):
     assert torch.equal(dq0, dq1) and torch.equal(dkv0, dkv1)
 
 
-def test_autograd_builds_the_index_during_the_forward(dev):
-    """SparseMLA.apply builds the index on the side stream in its forward; the
-    gradients equal the direct backward's bit for bit (bf16 and FP8 classes)."""
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+def test_autograd_matches_direct_and_prebuilt(dev, fp8):
+    """SparseMLA.apply / SparseMLA_FP8.apply hold their outputs and saved inputs until the
+    backward, no index; their gradients equal the direct backward's and that of one with an
+    index built ahead, bit for bit."""
     B, S, H, D, DV, topk = 1, 192, 32, 128, 64, 64
     q, kv, idx, do, scale = _case(dev, B, S, H, 1, D, DV, topk, seed=9)
     qd, kvd = q.clone().requires_grad_(), kv.clone().requires_grad_()
-    out, lse = SparseMLA.apply(qd, kvd, idx, scale, DV)
-    out.backward(do)
-    out2, lse2 = sparse_mla_fwd_interface(q, kv, idx, sm_scale=scale, d_v=DV)
-    dq, dkv = sparse_mla_bwd(q, kv, out2, do, idx, lse2, sm_scale=scale)
-    assert torch.equal(out, out2) and torch.equal(qd.grad, dq) and torch.equal(kvd.grad, dkv)
-    # no grad needed: no index is built
-    with torch.no_grad():
-        SparseMLA.apply(q, kv, idx, scale, DV)
-    qf, kvf = q.clone().requires_grad_(), kv.clone().requires_grad_()
-    of, _ = SparseMLA_FP8.apply(qf, kvf, idx, scale, DV)
-    of.backward(do)
-    assert torch.isfinite(qf.grad).all() and torch.isfinite(kvf.grad).all()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated(dev)
+    out, lse = (SparseMLA_FP8 if fp8 else SparseMLA).apply(qd, kvd, idx, scale, DV)
+    held = torch.cuda.memory_allocated(dev) - before
+    kept = [out, lse] + ([q.to(torch.float8_e4m3fn), kv.to(torch.float8_e4m3fn)] if fp8 else [])
+    # blocks are whole multiples of 512 bytes; e4m3 also keeps its scales, per tensor, token and row
+    limit = sum(-(-t.numel() * t.element_size() // 512) * 512 for t in kept) + (3 * 512 + 4 * B * S * 2 if fp8 else 0)
+    assert held <= limit < limit + int(_index_bytes(q, kv, idx, DV))
+    dq, dkv = torch.autograd.grad(out, (qd, kvd), do)
+    if fp8:
+        q8, qs = per_token_cast_to_fp8(q.reshape(-1, H * D))
+        k8, ks = per_token_cast_to_fp8(kv.reshape(-1, D))
+        q8, k8, qs, ks = q8.view(q.shape), k8.view(kv.shape), qs.reshape(B, S).contiguous(), ks.reshape(B, S).contiguous()
+        o2, l2 = sparse_mla_fwd_fp8_interface(q8, k8, idx, q_scale=qs, kv_scale=ks, sm_scale=scale, d_v=DV)
+        back = lambda **kw: sparse_mla_bwd_fp8(q8, k8, qs, ks, o2, do, idx, l2, sm_scale=scale, **kw)
+        ix = build_inverse_index(q8, k8, idx, DV, stream=side_stream(dev))
+    else:
+        o2, l2 = sparse_mla_fwd_interface(q, kv, idx, sm_scale=scale, d_v=DV)
+        back = lambda **kw: sparse_mla_bwd(q, kv, o2, do, idx, l2, sm_scale=scale, **kw)
+        ix = build_inverse_index(q, kv, idx, DV, stream=side_stream(dev))
+    assert torch.equal(out, o2) and torch.equal(lse, l2)
+    for ref in (back(), back(inverse_index=ix)):
+        assert torch.equal(dq, ref[0]) and torch.equal(dkv, ref[1])
+
+
+def _index_bytes(q, kv, idx, DV):
+    from cppmega_amd import _lib
+    B, S, H, D = q.shape
+    return _lib.load().dsa_sparse_mla_bwd_index_size(B, S, kv.shape[1], H, 1, D, DV, idx.shape[-1], 0, 0)
 
 
 def test_prebuilt_index_in_a_graph(dev):
