@@ -110,19 +110,23 @@ def test_fp8_quantize_validation(lib):
 
 def test_bwd_workspace_bounded_by_pass_cap(lib):
     """The backward runs in passes sized to a per-call cap on its partial dKV
-    rows (the pass_bytes argument, 0 = 4 GiB), so its workspace is bounded: at
-    cfg5 (s = 16384, h = 128, d_qk = 576, topk = 2048) one pass would hold
-    ~155 GB of fp16 rows; with the default cap the workspace stays under 5 GiB,
-    and a smaller cap shrinks it further (down to one 32-token chunk per pass,
-    ~302 MB of rows at cfg5).  The cap is an argument, not process state: two
-    queries with different caps do not affect each other."""
+    rows and, at d_qk = 576, its P and dS tiles (the pass_bytes argument, 0 =
+    4 GiB), so its workspace is bounded: at cfg5 (s = 16384, h = 128, d_qk = 576,
+    topk = 2048) a token takes 2048 rows of 1153 bytes and 1 MiB of tiles, one
+    pass would hold 56 GB; with the default cap the workspace stays under 5 GiB,
+    and a smaller cap shrinks it further, down to one 32-token chunk per pass
+    (109 MB).  The cap is an argument, not process state: two queries with
+    different caps do not affect each other."""
     wsz = lib.dsa_sparse_mla_bwd_workspace_size
-    ws = int(wsz(1, 16384, 16384, 128, 1, 576, 512, 2048, 0, 0))
+    cfg5 = lambda cap: int(wsz(1, 16384, 16384, 128, 1, 576, 512, 2048, 0, cap))
+    ws = cfg5(0)
     assert 0 < ws < 5 * (1 << 30), ws
-    assert int(wsz(1, 16384, 16384, 128, 1, 576, 512, 2048, 0, 4 << 30)) == ws
-    ws_small = int(wsz(1, 16384, 16384, 128, 1, 576, 512, 2048, 0, 256 << 20))
-    assert ws_small < ws and ws_small < 512 << 20, ws_small
-    assert int(wsz(1, 16384, 16384, 128, 1, 576, 512, 2048, 0, 0)) == ws      # no state left behind
+    assert cfg5(4 << 30) == ws
+    token = 2048 * 1153 + 64 * 4 * 4096
+    chunk, two, floor = cfg5(32 * token), cfg5(64 * token), cfg5(32 * token - 1)
+    assert 32 * token < two - chunk < 33 * token and chunk < two < ws      # a chunk more of rows, tiles and index
+    assert floor == cfg5(1) == chunk and 32 * token < chunk < 256 << 20    # never less than a chunk
+    assert cfg5(0) == ws                                                   # no state left behind
     # cfg2 fits one pass: its size does not depend on the cap while the cap covers it
     one = int(wsz(2, 4096, 4096, 32, 1, 128, 64, 256, 0, 0))
     assert one > 2 * 4096 * 256 * 257
