@@ -502,13 +502,21 @@ struct PassCfg {
   static_assert(C::CPR % 8 == 0, "swizzle within the row");
 };
 
+// kOwnKeys: every head has its key head, whose chunk's loads are spread over the
+// products as q's are.  kSharedKeys: a group of heads shares one; the next group's
+// chunk is fetched at once, by the group's last head, and one barrier serves the
+// group (spread conditionally, or at once for every head, the loads cost the former
+// case 3 to 7%).  kFarRows: as shared, and a wave's 32 query rows, B * H * D * 2 bytes
+// apart, span more than the 4 GiB that the DMA's 32-bit offsets reach (a batch of
+// several thousand short sequences): each lane reads its row as operands by 64-bit
+// addresses, one sub-tile's products after the other.
+enum PassForm { kOwnKeys, kSharedKeys, kFarRows };
+
 // LOSS: the KL partial sums; GRAD: P (p.grad, or the sparse state's p.pc) and the
-// R partial sums.  FAR: a wave's 32 query rows, B * H * D * 2 bytes apart, span more
-// than the 4 GiB that the DMA's 32-bit offsets reach (a batch of several thousand
-// short sequences): each lane reads its row as operands by 64-bit addresses, one
-// sub-tile's products after the other.
-template <int D, int NW, bool LOSS, bool GRAD, bool FAR>
+// R partial sums.
+template <int D, int NW, bool LOSS, bool GRAD, PassForm FORM>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4))) kl_pass_kernel(Params p) {
+  constexpr bool OWN = FORM == kOwnKeys, FAR = FORM == kFarRows;
   using C = Cfg<D, NW>;
   using PC = PassCfg<D, NW>;
   constexpr int kTB = C::TB;
@@ -578,17 +586,19 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
   const unsigned char *kbase = p.key + ((k0 * p.B + b) * p.G) * (int64_t)C::ROWB;
   const uint32_t lds = lds_address(smem);
   const uint32_t q_lds = lds + (uint32_t)(PC::OFF_Q + w * 32 * C::ROWB);
-  // this wave's loads: its share of the key chunk of a group of heads, into buffer
-  // kbuf, and its q slice of a head
-  const int hpg = (int)(p.H / p.G), H = (int)p.H;
-  auto fetch_keys = [&](i32x4 krs, int kbuf) {
-#pragma unroll
-    for (int i = 0; i < PC::KP; ++i) lds_dma_16(lds + (uint32_t)(kbuf * C::KC * C::ROWB + (w * PC::KP + i) * 1024), ko[i], krs, 0u);
+  // this wave's loads: its share of a key head's chunk, into buffer kbuf, and its q slice of a head
+  const int hpg = OWN ? 1 : (int)(p.H / p.G), H = (int)p.H;
+  auto fetch_k = [&](i32x4 krs, int kbuf, int i) {
+    lds_dma_16(lds + (uint32_t)(kbuf * C::KC * C::ROWB + (w * PC::KP + i) * 1024), ko[i], krs, 0u);
   };
   auto fetch_q = [&](i32x4 qrs, int i) { lds_dma_16(q_lds + (uint32_t)(i * 1024), qo[i], qrs, 0u); };
   auto key_rs = [&](int grp) { return make_buffer_words(kbase + grp * C::ROWB, kbytes); };
   auto query_rs = [&](int h) { return make_buffer_words(qb + h * C::ROWB, qbytes); };
-  constexpr int NF = FAR ? 0 : PC::QP;  // q loads per head
+  constexpr int NK = OWN ? PC::KP : 0, NF = NK + (FAR ? 0 : PC::QP);  // loads spread over a head's products: k's, then q's
+  auto fetch = [&](i32x4 krs, i32x4 qrs, int kbuf, int i) {
+    if (i < NK) fetch_k(krs, kbuf, i < PC::KP ? i : 0);
+    else fetch_q(qrs, i - NK < PC::QP ? i - NK : 0);
+  };
   bool all_on = !FAR, any_on = false;  // wave-uniform
 #pragma unroll
   for (int sub = 0; sub < C::SUBS; ++sub) {
@@ -601,10 +611,11 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
     return as_bf16x8(*reinterpret_cast<const i32x4 *>(tile + (r0 + l32) * C::ROWB + (((2 * k + g) ^ PC::swz(l32)) * 16)));
   };
   const float *beta_bt = p.beta + b * p.H * p.Sq + (t < p.Sq ? t : 0);
-  i32x4 qrs = query_rs(0);
-  fetch_keys(key_rs(0), 0);
+  i32x4 krs = key_rs(0), qrs = query_rs(0);
 #pragma unroll
-  for (int i = 0; i < NF; ++i) fetch_q(qrs, i);
+  for (int i = NK; i < PC::KP; ++i) fetch_k(krs, 0, i);
+#pragma unroll
+  for (int i = 0; i < NF; ++i) fetch(krs, qrs, 0, i);
   // The previous head's last sub-tile and its normaliser: its exp2 work runs
   // under the next head's first products (before head 0: exp2(-inf) = 0).
   f32x16 cur;
@@ -614,7 +625,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
   int grp = 0, left = hpg;  // the head's key group, and its heads still to come
   for (int h = 0; h < H; ++h) {
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this head's q and k, fetched a head ago
-    if (left == hpg) __syncthreads();    // every wave's share of the group's k; the other k buffer is consumed
+    if (OWN || left == hpg) __syncthreads();  // every wave's share of the group's k; the other k buffer is consumed
     const unsigned char *ks = smem + (grp & 1) * C::KC * C::ROWB;
     bf16x8 Q[C::KSTEPS];
 #pragma unroll
@@ -625,11 +636,14 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
     const int hn = h + 1 < H ? h + 1 : h;  // (past the last head: its own again, unused)
     bn = beta_bt[(int64_t)hn * p.Sq];
     qrs = query_rs(hn);
-    if (--left == 0) {  // the last head of its group: the next group's keys
+    if (OWN || --left == 0) {  // the last head of its group: the next group's keys
       left = hpg;
       ++grp;
-      fetch_keys(key_rs(grp < (int)p.G ? grp : grp - 1), grp & 1);
+      krs = key_rs(grp < (int)p.G ? grp : grp - 1);
+#pragma unroll
+      for (int i = NK; i < PC::KP; ++i) fetch_k(krs, grp & 1, i);
     }
+    const int kb = grp & 1;
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the q slice is in registers, its LDS free
     if (all_on) {
       // key operands are read two products ahead
@@ -655,12 +669,12 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
 #pragma unroll
           for (int e = 0; e < kE; ++e)
             if (k * kE + e < 16) P[ps][k * kE + e] += exp2_fast(fmaf(cur[k * kE + e], p.c, -pb));
-          // the next head's q loads, spread over the first sub-tile
-          constexpr int kPer = (NF + C::KSTEPS - 1) / C::KSTEPS;
+          // the next head's loads, spread over the first sub-tiles
+          constexpr int kPer = (NF + C::KSTEPS * (C::SUBS - 1) - 1) / (C::KSTEPS * (C::SUBS - 1));
 #pragma unroll
           for (int u = 0; u < kPer; ++u) {
             const int f = i * kPer + u;
-            if (f < NF) fetch_q(qrs, f);
+            if (f < NF) fetch(krs, qrs, kb, f);
           }
           __builtin_amdgcn_sched_barrier(0);  // keep this order
         }
@@ -669,7 +683,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
       bprev = bh;
     } else {
 #pragma unroll
-      for (int i = 0; i < NF; ++i) fetch_q(qrs, i);
+      for (int i = 0; i < NF; ++i) fetch(krs, qrs, kb, i);
       if (any_on) {
 #pragma unroll
         for (int sub = 0; sub < C::SUBS; ++sub) {
@@ -1026,9 +1040,9 @@ static int64_t pass_items(const Params &p, int64_t TB, int64_t KC) {
   return n;
 }
 
-template <int D, int NW, bool LOSS, bool GRAD, bool FAR>
+template <int D, int NW, bool LOSS, bool GRAD, PassForm FORM>
 static int launch_pass(const Params &p, int64_t items, hipStream_t st) {
-  const auto pass = kl_pass_kernel<D, NW, LOSS, GRAD, FAR>;
+  const auto pass = kl_pass_kernel<D, NW, LOSS, GRAD, FORM>;
   constexpr int lds = PassCfg<D, NW>::BYTES;
   const hipError_t e = hipFuncSetAttribute((const void *)pass, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return set_error(DSA_ERR_HIP, "kl_pass_kernel: LDS attribute: %s", hipGetErrorString(e));
@@ -1052,7 +1066,9 @@ static int launch_mfma(const Params &p, hipStream_t st) {
   const int64_t items = (p.B * q.NI + 7) / 8 * 8;
   const int64_t rows = p.Sq < 32 ? p.Sq : 32;  // of a wave
   const bool far = (rows - 1) * p.B * p.H * CP::ROWB + CP::ROWB > (int64_t)0xffffffff;
-  rc = far ? launch_pass<D, NWP, LOSS, GRAD, true>(q, items, st) : launch_pass<D, NWP, LOSS, GRAD, false>(q, items, st);
+  if (far) rc = launch_pass<D, NWP, LOSS, GRAD, kFarRows>(q, items, st);
+  else if (p.G < p.H) rc = launch_pass<D, NWP, LOSS, GRAD, kSharedKeys>(q, items, st);
+  else rc = launch_pass<D, NWP, LOSS, GRAD, kOwnKeys>(q, items, st);
   if (rc) return rc;
   if (p.pc != nullptr) {
     hipLaunchKernelGGL(kl_rows_state_kernel<D>, dim3((unsigned)((p.B * p.Sq + 3) / 4)), dim3(kNT), 0, st, p);
