@@ -14,11 +14,14 @@
 //   Q[t, s]   = softmax_s (index_scores[t, :] + sparse top-k mask) over all s
 //   loss      = coeff * mean_t sum_s P (ln(P + 1e-10) - ln(Q + 1e-10))
 //
-// Five stream-ordered kernels, all deterministic (no atomics outside LDS):
+// Stream-ordered kernels, all deterministic (no atomics outside LDS).  The loss alone
+// (dsa_indexer_kl_loss) is 1 to 5; the other entry points are listed below it.
 //  1. kl_index_stats_kernel  one wave per (b, t): the log2 normaliser
 //     gamma = max + log2(sum exp2(x - max)) of x = index_scores * log2(e) over
 //     the row (sparse: over the row's top-k set, built as a bitmask in LDS and
-//     written out for the other kernels);
+//     written out for the other kernels; with a sparse state also the set's ranks
+//     and scores in column order);
+//  1a. kl_mask_tiles_kernel  sparse, large calls: the bitmask as lane masks for 2;
 //  2. kl_attn_stats_kernel   per (b, head, pair of 256-token blocks): the log2
 //     normaliser beta_h[t] of c * q.k (c = scale * log2(e)) over s <= t, on
 //     MFMA 32x32x16 bf16 with S^T = K . Q^T (keys on M, tokens on N, so a lane
@@ -49,15 +52,21 @@
 //     whole row of the gradient in place over P (16-byte loads and stores).
 //
 // Loss and gradient together (dsa_indexer_kl_loss_with_grad, what autograd
-// takes): the gradient is linear in g, so one run of kernels 1-3 leaves the
-// loss and a state from which dsa_indexer_kl_loss_grad_apply forms the gradient
-// for any g.  Recomputing in the backward ran both q.k kernels twice (index
-// stats, statistics and pass again: 565 of the 1510 us of a sparse training step
-// at b = 2, s = 4096, 32 heads of 128).  The state holds
+// takes; dsa_indexer_kl_loss_grad_state leaves the loss out): the gradient is
+// linear in g, so one run of the two q.k kernels leaves the loss and a state from
+// which dsa_indexer_kl_loss_grad_apply forms the gradient for any g (a backward that
+// recomputed would run them again: 565 us at b = 2, s = 4096, 32 heads of 128).
+// The state holds
 //   v_s = Q_s * R - P_s * Q_s / (Q_s + 1e-10):
-// dense, every column (the size of the scores, which then need not be kept);
+// dense, every column (the size of the scores, which then need not be kept):
+// kernels 1 to 6, then
+//  7. kl_scale_kernel        the gradient, g * coeff / (B * Sq) * v;
 // sparse, the columns of the row's top-k set only, in column order (v is 0
-// elsewhere), with the set's bitmask: 12 MB instead of 128 MiB at top-256.
+// elsewhere), with the set's bitmask: 12 MB instead of 128 MiB at top-256.  Kernels
+// 1 to 3, where 3 leaves the set's P at its ranks, then
+//  4s. kl_rows_state_kernel  one wave per row: the row's loss and R over the set, v;
+//  5, and
+//  7s. kl_expand_kernel      the gradient's rows from the bitmask, the ranks and v.
 #include "dsa_common.hpp"
 #include "wave_ops.hpp"
 
@@ -342,8 +351,8 @@ __device__ __forceinline__ int64_t block_chunks(const Params &p, int64_t blk, in
 // token's top-k set at or below its diagonal: the select operand, straight from
 // scalar registers, of accumulator register a in kl_attn_stats_kernel.  One
 // transposition serves every head; forming the selects per head from the row
-// bitmask took two VALU operations an element there (with it 229 -> 192 us at
-// b = 2, s = 4096, 32 heads of 128).  A workgroup takes a (b, 32-token block) and
+// bitmask takes two VALU operations an element there (174 us with lane masks at
+// b = 2, s = 4096, 32 heads of 128; use_lane_masks).  A workgroup takes a (b, 32-token block) and
 // every gridDim.y-th group of four words at or below the diagonal.
 __global__ void __launch_bounds__(kNT) kl_mask_tiles_kernel(Params p) {
   const int lane = lane_id(), g = lane >> 5, l32 = lane & 31;
@@ -483,9 +492,10 @@ kl_attn_stats_kernel(Params p) {
 // global, q's 32 rows of 16 bytes per instruction cost more address cycles than
 // the arithmetic), each wave owns its 32 tokens' q slice, and a wave whose four
 // key sub-tiles all count runs the next sub-tile's products under the current
-// one's exp2.  256 tokens share a key chunk.  At b = 2, s = 4096, 32 heads of 128:
-// 315 us before, 239 us now, of which the VALU's share is about 150 us (544
-// workgroups are a little over two rounds of 256 compute units).
+// one's exp2.  256 tokens share a key chunk, or 128 (launch_by_size).  At b = 2, s = 4096,
+// 32 heads of 128: 230 us, 315 with the operands read straight from global; the VALU's
+// share is about 150 us (544 workgroups are a little over two rounds of 256 compute
+// units).
 template <int D, int NW>
 struct PassCfg {
   using C = Cfg<D, NW>;

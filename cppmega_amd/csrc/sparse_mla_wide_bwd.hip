@@ -10,13 +10,17 @@
 //      heads (128 at a time) with Q and dO resident in registers as MFMA
 //      operands, written as one fp16 row (scaled by a power of two) or fp32
 //      row per (token, slot) at its CSR position.
-// One kernel for both holds Q and dO of at most 32 heads, so each (token, slot)
-// left four partial rows at 128 heads: 29 GB written and read again at
-// s = 4096, h = 128, top-k 2048 (18.0 ms for that kernel, 5.4 ms for the
+// One kernel for both would hold Q and dO of at most 32 heads, so each (token,
+// slot) would leave four partial rows at 128 heads: 29 GB written and read again
+// at s = 4096, h = 128, top-k 2048 (18.0 ms for such a kernel, 5.4 ms for the
 // reduction).  P and dS of all heads are 512 bytes per (token, slot), less than
 // one partial row's 1152, and buy the sum over heads before the row is stored:
-// scores 4.0 ms (2.6 TFLOP of the three products), rows 2.8 ms (11.5 GB of HBM
-// traffic), reduction 1.1 ms.
+// scores 4.1 ms (2.6 TFLOP of the three products), rows 2.8 ms (11.5 GB of HBM
+// traffic), reduction 1.1 ms.  Up to 32 heads there is one row either way; the two
+// kernels are no slower there (s = 2048, one kernel and two: 32 heads, top-64 296
+// and 279 us, top-512 1093 and 882, top-2048 3765 and 2959; e4m3, top-512 1159 and
+// 1122; s = 300, top-64 75 and 75), as each holds fewer operands and the scores run
+// in the two-barrier pipeline.
 #include <type_traits>
 
 #include "dsa_common.hpp"

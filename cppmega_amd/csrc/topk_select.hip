@@ -917,10 +917,10 @@ static int topk_run(const TopkParams &p, hipStream_t st) {
   const int64_t len = p.nseg > 1 ? p.seg_len : p.row_len;
   // Few rows leave compute units idle at one wave (or 4 or 8 waves) per row, and
   // a row's time is one wave's passes over its 64 to 128 items per lane: spread
-  // such rows over more waves.  16 rows, top-2048: 4096 columns 10.8 -> 6.2 us,
-  // 8192 18.3 -> 7.6, 16384 12.7 -> 10.5, 32768 15.9 -> 14.3.  The lines lie where
-  // the rows fill the chip either way: 1024 rows of 8192 still 20.5 -> 15.4, 2048
-  // rows of 4096 16.2 -> 15.5; 512 rows of 16384 15.2 -> 15.9.
+  // such rows over more waves.  16 rows, top-2048, spread and as for many rows: 4096
+  // columns 6.2 and 10.8 us, 8192 7.6 and 18.3, 16384 10.5 and 12.7, 32768 14.3 and
+  // 15.9.  The lines lie where the rows fill the chip either way: 1024 rows of 8192
+  // 15.4 and 20.5 us, 2048 rows of 4096 15.5 and 16.2, 512 rows of 16384 15.9 and 15.2.
   if (len > 2048 && p.rows <= (len <= 8192 ? 1024 : 256)) {
     if (len <= 4096) return launch_topk_block<4, 16>(p, st);
     if (len <= 8192) return launch_topk_block<8, 16>(p, st);

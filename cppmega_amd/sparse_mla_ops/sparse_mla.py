@@ -74,11 +74,11 @@ class SparseMLA(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output, grad_lse):
         q, kv, indices, out, lse = ctx.saved_tensors
-        # The backward builds its inverse index in the same call.  Built during the forward on
-        # a second stream it bought nothing (B 2, S 4096, 32 heads, top-256: 343 us a step either
-        # way, the build and the forward slowing each other), held 21 MB per layer until the
-        # backward, and cost the host more than the kernels of a small call (B 1, S 512, 16
-        # heads, top-64: 154 us a step, now 105).
+        # The backward builds its inverse index in the same call.  Beside the forward, on a second
+        # stream, the two slow each other by what it saves (B 2, S 4096, 32 heads, top-256: 343 us
+        # a step either way); it would hold 21 MB per layer until the backward, and its events
+        # and stream switch cost a small call more than its kernels (B 1, S 512, 16 heads, top-64,
+        # bound by the host: 198 us a step, 140 as here).
         dq, dkv = sparse_mla_bwd(q, kv, out, grad_output.contiguous(), indices, lse, sm_scale=ctx.scaling)
         return dq, dkv, None, None, None
 
