@@ -55,6 +55,13 @@ def _inputs(B, S, H, D, G, K, seed, spread=True, pow2=True):
     (2, 40, 16, 576, 512, 1, 40, False),
     (1, 36, 64, 576, 512, 2, 48, False),
     (1, 24, 96, 576, 512, 1, 40, False),   # two head tiles per workgroup, one empty
+    # exact dequantisation, where the bf16 kernels run: one head tile of three, two of three,
+    # pipelined two and four; kv groups of two tiles
+    (1, 24, 96, 576, 512, 1, 40, True),
+    (1, 100, 96, 576, 512, 1, 70, True),
+    (1, 90, 128, 576, 512, 1, 200, True),
+    (1, 200, 128, 576, 512, 1, 40, True),
+    (1, 90, 128, 576, 512, 2, 40, True),
 ])
 def test_mxfp8_fwd_matches_oracle(dev, B, S, H, D, DV, G, K, pow2):
     q8, qs, kv8, ks, idx = _inputs(B, S, H, D, G, K, seed=S + D, pow2=pow2)
